@@ -432,6 +432,27 @@ int keep_vq_grouped_gemm_q8(const void* x, int x_dtype, int64_t x_rows, const in
                             int64_t routes, int64_t num_experts, int64_t N, int64_t K, int64_t group_size,
                             void* workspace, int64_t workspace_bytes, void* out, int out_dtype, void* stream);
 
+/* The same sorted-route GEMM on 8-bit E8 codes (uint8 [E, N, K/8], `table` the
+ * packed 8-bit E8 table, uint32[256]), storing its rows as
+ * keep_vq_grouped_gemm_q8 does for E8P. x is fp16 or bf16 and enters the matrix
+ * cores as it is, the weights x 4 exact in either type: no workspace. Replaces
+ * gather_vqmm_sorted_routes on 8-bit codes (vq_switch.py:620-913). */
+int keep_vq_grouped_gemm_e8(const void* x, int x_dtype, int64_t x_rows, const int32_t* lhs,
+                            const int32_t* out_index, const uint8_t* codes, const void* scales, int scale_dtype,
+                            const uint32_t* table, const int32_t* tile_expert, const int32_t* tile_offset,
+                            const int32_t* tile_count, int64_t n_tiles, int64_t routes, int64_t num_experts,
+                            int64_t N, int64_t K, int64_t group_size, void* out, int out_dtype, void* stream);
+
+/* One matrix against many rows on the matrix cores: out[m, :] = W . x[m, :]
+ * for x fp16 or bf16 [rows, K], codes [N, K/8] (code_bits 16: E8P, `tables` =
+ * keep_e8p_prepare's buffer; 8: E8, `tables` = the packed 8-bit E8 table),
+ * scales [N, K/group_size]. Arithmetic as keep_vq_grouped_gemm_q8 (E8P; bf16
+ * rows need its workspace for `rows` rows) or keep_vq_grouped_gemm_e8 (no
+ * workspace). Replaces vq_qmm (src/ramp/kernels/vq_qmm.py:93-152) on many rows. */
+int keep_vq_gemm(const void* x, int x_dtype, int64_t rows, const void* codes, int code_bits, const void* scales,
+                 int scale_dtype, const void* tables, int64_t N, int64_t K, int64_t group_size, void* workspace,
+                 int64_t workspace_bytes, void* out, int out_dtype, void* stream);
+
 /* The gate and up projections of the same tiles in one pass, with SwiGLU
  * (silu(min(g, L)) * clip(u, -L, L), plain for L <= 0) in fp32 and h stored
  * in bf16 at the route's sorted position: h_out[p, :] for p < routes, I

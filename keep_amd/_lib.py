@@ -53,6 +53,10 @@ _SIGS = {
                             c_int64, _P, c_int, _P],
     "keep_vq_grouped_gemm_q8": [_P, c_int, c_int64, _P, _P, _P, c_int, _P, c_int, _P, _P, _P, _P, c_int64, c_int64,
                                 c_int64, c_int64, c_int64, c_int64, _P, c_int64, _P, c_int, _P],
+    "keep_vq_grouped_gemm_e8": [_P, c_int, c_int64, _P, _P, _P, _P, c_int, _P, _P, _P, _P, c_int64, c_int64, c_int64,
+                                c_int64, c_int64, c_int64, _P, c_int, _P],
+    "keep_vq_gemm": [_P, c_int, c_int64, _P, c_int, _P, c_int, _P, c_int64, c_int64, c_int64, _P, c_int64, _P, c_int,
+                     _P],
     "keep_vq_grouped_swiglu_q8": [_P, c_int, c_int64, _P, _P, _P, _P, _P, c_int, _P, _P, _P, _P, c_int64, c_int64,
                                   c_int64, c_int64, c_int64, c_int64, c_float, _P, c_int64, _P, _P],
     "keep_vq_grouped_swiglu_nested_q8": [_P, c_int, c_int64, _P, _P, _P, _P, _P, c_int, _P, _P, _P, _P, _P, c_int,

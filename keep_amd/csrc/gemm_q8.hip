@@ -62,8 +62,14 @@ typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h2v __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-__device__ __forceinline__ f32x16 mfma32_f16(h8 a, h8 b, f32x16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+// One 32x32x16 MFMA of 16-bit operands (BF: the bits are bf16's, else fp16's).
+template <bool BF>
+__device__ __forceinline__ f32x16 mfma32(h8 a, h8 b, f32x16 c) {
+  typedef __bf16 b8 __attribute__((ext_vector_type(8)));
+  if constexpr (BF)
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(b8, a), __builtin_bit_cast(b8, b), c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
 }
 
 // Bytes q + 128 (mod 256) of eight integer weights q -> the fp16 values q.
@@ -142,14 +148,15 @@ struct GQArgs {
   const uint16_t *c0, *c1;  // codes [E][N][K / 8] (gate/up: gate, up)
   const void *s0, *s1;      // scales [E][N][G]
   int sdt;
-  const void* tq;           // E8P: T and M (keep_e8p_prepare); residual: the packed 8-bit E8 table
+  const void* tq;           // E8P: T and M (keep_e8p_prepare); E8: the packed 8-bit E8 table
   const uint32_t* tq_bad;
-  const int32_t *te, *to, *tc;
+  const int32_t *te, *to, *tc;  // null: one matrix, tile i = rows 64 i ..
   int64_t n_tiles, routes;
   int64_t E, N, K, G, kpg;  // kpg: K blocks per scale group
   float limit;
   void* out;
   int odt;
+  int add;                      // E8: add to the fp32 output instead of storing
   int64_t ncb, total, per_xcd;  // column blocks, work items, items per XCD
   // the fused residual (HOT)
   const uint8_t *rc0, *rc1;  // residual codes [hot_rows][N][K / 8] (gate/up: gate, up)
@@ -160,9 +167,16 @@ struct GQArgs {
   const uint32_t* t8;        // the packed 8-bit E8 table (uint32[256])
 };
 
-// RES: the nested tier's 8-bit E8 residual instead of E8P base codes (one code
-// byte per codeword, one 8-byte lookup); the result is added to the fp32
-// output (the base projection's). HOT: E8P base codes and, on the tiles of an
+// E8: 8-bit E8 codes instead of E8P (one code byte per codeword). The LDS image
+// holds an entry's eight weights x 4 ready in the A rows' 16-bit type (sixteen
+// copies of 16 bytes, 64 KiB), so a codeword is one byte permute and one
+// 16-byte lookup with no conversion: 1 VALU instead of the 10 of the byte image
+// this replaced. bf16 rows stay bf16 (the weights are exact in it), without a
+// row factor. LDS-bound: per k-step a wave reads 1 KiB per m-tile and 1 KiB of
+// lookups per n-tile. 2048 bf16 rows against 4096 x 4096, groups of 512: 77 us
+// (896 TFLOP/s; a mat-vec per row took 3,900 us). The result is stored, or added
+// to the fp32 output (a.add: the nested tier's residual onto the base
+// projection's). HOT: E8P base codes and, on the tiles of an
 // expert with a residual row (hot[e] in [0, hot_rows)), that row's 8-bit E8
 // residual codes, decoded from a second LDS image and multiplied by the same A
 // operands into a second accumulator; base and residual are scaled and summed
@@ -172,12 +186,13 @@ struct GQArgs {
 // range other than -1 makes the tile's rows NaN. XT: the A rows' element type.
 // NTW: 32-column n-tiles per wave (2: items of 512 columns; 1: of 256, for
 // problems with too few items to spread over the CUs).
-template <bool GATEUP, bool GROUPED, typename XT, bool RES = false, int NTW = 2, bool HOT = false>
+template <bool GATEUP, bool GROUPED, typename XT, bool E8 = false, int NTW = 2, bool HOT = false>
 __global__ __launch_bounds__(GQ_THREADS) void k_gemm_e8(GQArgs a) {
-  static_assert(!(HOT && (RES || GROUPED)), "the fused residual takes E8P base codes and per-row scales");
+  static_assert(!(HOT && (E8 || GROUPED)), "the fused residual takes E8P base codes and per-row scales");
   constexpr int D = 2;                         // K blocks in flight
   constexpr int NCOL = GQ_WAVES * 32 * NTW;    // output columns per work item
   constexpr int XV = sizeof(XT) == 4 ? 4 : 2;           // 16-byte A loads per thread and K block
+  constexpr bool BF = E8 && std::is_same<XT, bf16s>::value;  // bf16 operands
   __shared__ uint4 tqs[TQR_BYTES / 16];
   __shared__ uint2 t8s[HOT ? T8R_BYTES / 8 : 1];  // HOT: the residual image
   __shared__ __attribute__((aligned(16))) uint8_t ash[2][GQ_M * GQ_ROW];
@@ -201,8 +216,19 @@ __global__ __launch_bounds__(GQ_THREADS) void k_gemm_e8(GQArgs a) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) row[i] = make_uint2(b[0], b[1]);
     };
-    if constexpr (RES) {
-      e8_row(((const uint32_t*)a.tq)[e], (char*)tqs);
+    if constexpr (E8) {  // entry e: copies of the eight weights 2 (nibble d - 8) as 16-bit floats
+      const uint32_t p = ((const uint32_t*)a.tq)[e];
+      uint32_t b[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {  // encode_half_units(v) is the 16-bit pattern of v / 2
+        constexpr int PK = BF ? PAIR_BF16 : PAIR_F16;
+        const int lo = 4 * ((int)((p >> (8 * i)) & 15u) - 8), hi = 4 * ((int)((p >> (8 * i + 4)) & 15u) - 8);
+        b[i] = encode_half_units<PK>(lo) | (encode_half_units<PK>(hi) << 16);
+      }
+      const uint4 v = make_uint4(b[0], b[1], b[2], b[3]);
+      uint4* row = tqs + e * 16 + (tid & 1) * 8;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) row[i] = v;
     } else {  // row e: sixteen copies of (T'[e], M[e]), T' = T ^ 0x80 per byte, natural dim order
       const uint2 t = gq_natural(((const uint2*)a.tq)[e]), m = gq_natural(((const uint2*)a.tq)[256 + e]);
       const uint4 v = make_uint4(t.x ^ 0x80808080u, t.y ^ 0x80808080u, m.x, m.y);
@@ -227,11 +253,10 @@ __global__ __launch_bounds__(GQ_THREADS) void k_gemm_e8(GQArgs a) {
   // block, in two halves: the LDS image lookups (look), then the bytes -> fp16
   // (cvt), so that a k-step's lookups are issued two k-steps before its MFMAs.
   auto look = [&](const uint4& q, int s) -> uint4 {
-    if constexpr (RES) {  // code bytes: codeword s is byte s of q.x / q.y
-      const uint32_t w = s < 4 ? q.x : q.y;
-      const uint32_t byte = (w >> (8 * (s & 3))) & 0xffu;
-      const uint2 x = *(const uint2*)(img + byte * 128u + (uint32_t)(lane & 15) * 8u);
-      return make_uint4(x.x, x.y, 0u, 0u);
+    if constexpr (E8) {  // code bytes: codeword s is byte s of q.x / q.y
+      const uint32_t ad = __builtin_amdgcn_perm(s < 4 ? q.x : q.y, (uint32_t)(lane & 15) << 4,
+                                                0x0c0c0400u + ((uint32_t)(s & 3) << 8));
+      return *(const uint4*)(img + ad);
     } else {
       const uint32_t w = s < 2 ? q.x : (s < 4 ? q.y : (s < 6 ? q.z : q.w));
       const bool hi = (s & 1) != 0;
@@ -241,7 +266,10 @@ __global__ __launch_bounds__(GQ_THREADS) void k_gemm_e8(GQArgs a) {
       return make_uint4(x1.x, x1.y, x2.x, x2.y);
     }
   };
-  auto cvt = [&](const uint4& r) -> h8 { return gq_f16_of_bytes(make_uint2(r.x ^ r.z, r.y ^ r.w)); };
+  auto cvt = [&](const uint4& r) -> h8 {
+    if constexpr (E8) return __builtin_bit_cast(h8, r);
+    else return gq_f16_of_bytes(make_uint2(r.x ^ r.z, r.y ^ r.w));
+  };
   // HOT: the residual codeword s of this lane's 8 code bytes -> its 8 bytes q + 128
   auto look_r = [&](const uint2& r, int s) -> uint2 {
     const uint32_t w = s < 4 ? r.x : r.y;
@@ -256,12 +284,12 @@ __global__ __launch_bounds__(GQ_THREADS) void k_gemm_e8(GQArgs a) {
     const int64_t w = xcd * a.per_xcd + j;
     if (w >= a.total) break;
     const int64_t cb = w / a.n_tiles, tile = w - cb * a.n_tiles;
-    const int cnt_raw = a.tc[tile];
-    const int64_t off = a.to[tile];
+    const int cnt_raw = a.te ? a.tc[tile] : (int)min((int64_t)GQ_M, a.routes - tile * GQ_M);
+    const int64_t off = a.te ? (int64_t)a.to[tile] : tile * GQ_M;
     const int cnt = min(cnt_raw, GQ_M);
     if (cnt_raw <= 0 || off < 0 || off + cnt > a.routes) continue;  // nothing can be written safely
-    const int64_t e = a.te[tile];
-    if (RES && e < 0) continue;  // routes off the residual tier (row -1): nothing to add
+    const int64_t e = a.te ? a.te[tile] : 0;
+    if (E8 && a.add && e < 0) continue;  // routes off the residual tier (row -1): nothing to add
     bool bad = e < 0 || e >= a.E || cnt_raw > GQ_M;  // rows written as NaN
     int64_t hr = -1;  // HOT: the tile's residual row
     if constexpr (HOT) {
@@ -300,8 +328,8 @@ __global__ __launch_bounds__(GQ_THREADS) void k_gemm_e8(GQArgs a) {
       }
       nv[jn] = n[jn] < a.N;
       crow[jn] = (bad || !nv[jn]) ? 0 : e * a.N + n[jn];
-      // E8P: 16 bytes per K block (codewords 8 h ..); residual: 8 bytes (one byte per codeword)
-      cp[jn] = RES ? (const uint8_t*)cbase + crow[jn] * C + 8 * h : (const uint8_t*)(cbase + crow[jn] * C + 8 * h);
+      // E8P: 16 bytes per K block (codewords 8 h ..); E8: 8 bytes (one byte per codeword)
+      cp[jn] = E8 ? (const uint8_t*)cbase + crow[jn] * C + 8 * h : (const uint8_t*)(cbase + crow[jn] * C + 8 * h);
       rrow[jn] = (hr < 0 || !nv[jn]) ? 0 : hr * a.N + n[jn];
       rp[jn] = HOT ? rbase + rrow[jn] * C + 8 * h : nullptr;
     }
@@ -331,7 +359,7 @@ __global__ __launch_bounds__(GQ_THREADS) void k_gemm_e8(GQArgs a) {
       const int kq = min(u, nkb - 1), ka = min(u + 1, nkb - 1);
 #pragma unroll
       for (int jn = 0; jn < NTW; ++jn) {
-        if constexpr (RES) {
+        if constexpr (E8) {
           const uint2 v = ldg8_q(cp[jn] + kq * 16);
           b.q[jn] = make_uint4(v.x, v.y, 0u, 0u);
         } else {
@@ -343,10 +371,10 @@ __global__ __launch_bounds__(GQ_THREADS) void k_gemm_e8(GQArgs a) {
       for (int i = 0; i < XV; ++i) b.ax[i] = ldg16_q(ap + ((int64_t)ka * GQ_KB + 64 * (i / (XV / 2))) * sizeof(XT) +
                                                      16 * (i % (XV / 2)));
     };
-    // 16 elements of the row (x r for bf16 / fp32) -> fp16 (round to nearest even), into the A buffer
+    // 16 elements of the row (x r for bf16 / fp32) -> fp16 (round to nearest even; E8: bf16 as it is), into the A buffer
     auto stage = [&](int buf, const uint4 (&ax)[XV]) {
       uint4 o[2];
-      if constexpr (sizeof(XT) == 2 && !std::is_same<XT, bf16s>::value) {
+      if constexpr (BF || std::is_same<XT, _Float16>::value) {
         o[0] = ax[0];
         o[1] = ax[1];
       } else {
@@ -458,8 +486,8 @@ __global__ __launch_bounds__(GQ_THREADS) void k_gemm_e8(GQArgs a) {
 #pragma unroll
             for (int jn = 0; jn < NTW; ++jn) {
 #pragma unroll
-              for (int mt = 0; mt < NT; ++mt) acc[mt][jn] = mfma32_f16(A[mt], Bc[jn], acc[mt][jn]);
-              if constexpr (HT) acc[1][jn] = mfma32_f16(A[0], Rc[jn], acc[1][jn]);
+              for (int mt = 0; mt < NT; ++mt) acc[mt][jn] = mfma32<BF>(A[mt], Bc[jn], acc[mt][jn]);
+              if constexpr (HT) acc[1][jn] = mfma32<BF>(A[0], Rc[jn], acc[1][jn]);
             }
 #pragma unroll
             for (int jn = 0; jn < NTW; ++jn) {
@@ -521,7 +549,7 @@ __global__ __launch_bounds__(GQ_THREADS) void k_gemm_e8(GQArgs a) {
             } else {
               if (m < cnt && nv[jn]) {
                 const int64_t o = (int64_t)s_orow[m] * a.N + n[jn];
-                if constexpr (RES) ((float*)a.out)[o] += val;
+                if (E8 && a.add) ((float*)a.out)[o] += val;
                 else if (a.odt == KEEP_F32) ((float*)a.out)[o] = val;
                 else if (a.odt == KEEP_BF16) ((uint16_t*)a.out)[o] = from_float<bf16s>(val).bits;
                 else ((_Float16*)a.out)[o] = (_Float16)val;
@@ -597,22 +625,22 @@ const float2* gq_rowscale(const void* x, int x_dtype, int64_t rows, int64_t K, v
   return rs;
 }
 
-template <bool GATEUP, bool RES, typename XT, int NTW, bool HOT>
+template <bool GATEUP, bool E8, typename XT, int NTW, bool HOT>
 void gq_launch_x(const GQArgs& a, dim3 grid, hipStream_t s) {
   if constexpr (HOT) hipLaunchKernelGGL((k_gemm_e8<GATEUP, false, XT, false, NTW, true>), grid, dim3(GQ_THREADS), 0, s, a);
-  else if (a.G > 1) hipLaunchKernelGGL((k_gemm_e8<GATEUP, true, XT, RES, NTW>), grid, dim3(GQ_THREADS), 0, s, a);
-  else hipLaunchKernelGGL((k_gemm_e8<GATEUP, false, XT, RES, NTW>), grid, dim3(GQ_THREADS), 0, s, a);
+  else if (a.G > 1) hipLaunchKernelGGL((k_gemm_e8<GATEUP, true, XT, E8, NTW>), grid, dim3(GQ_THREADS), 0, s, a);
+  else hipLaunchKernelGGL((k_gemm_e8<GATEUP, false, XT, E8, NTW>), grid, dim3(GQ_THREADS), 0, s, a);
 }
 
-template <bool GATEUP, bool RES, int NTW, bool HOT = false>
+template <bool GATEUP, bool E8, int NTW, bool HOT = false>
 void gq_launch_t(const GQArgs& a, dim3 grid, hipStream_t s) {
-  if (a.xdt == KEEP_F16) gq_launch_x<GATEUP, RES, _Float16, NTW, HOT>(a, grid, s);
-  else if (a.xdt == KEEP_BF16) gq_launch_x<GATEUP, RES, bf16s, NTW, HOT>(a, grid, s);
-  else gq_launch_x<GATEUP, RES, float, NTW, HOT>(a, grid, s);
+  if (a.xdt == KEEP_F16) gq_launch_x<GATEUP, E8, _Float16, NTW, HOT>(a, grid, s);
+  else if (a.xdt == KEEP_BF16) gq_launch_x<GATEUP, E8, bf16s, NTW, HOT>(a, grid, s);
+  else gq_launch_x<GATEUP, E8, float, NTW, HOT>(a, grid, s);
 }
 
 // hot: the fused residual (a.hot, a.rc0 / a.rc1, ... set; per-row scales)
-void gq_launch(GQArgs& a, bool gateup, hipStream_t s, bool res = false, bool hot = false) {
+void gq_launch(GQArgs& a, bool gateup, hipStream_t s, bool e8 = false, bool hot = false) {
   int dev = 0, cus = 256;
   if (hipGetDevice(&dev) == hipSuccess)
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
@@ -622,19 +650,24 @@ void gq_launch(GQArgs& a, bool gateup, hipStream_t s, bool res = false, bool hot
     a.total = a.ncb * a.n_tiles;
     a.per_xcd = (a.total + GQ_XCDS - 1) / GQ_XCDS;
   };
+  shape(256);
+  const int64_t narrow_rounds = (a.total + cus - 1) / cus;
   shape(512);
-  const bool wide = a.total >= 4 * (int64_t)cus;
+  // routed tiles: items of 512 columns once there are four per CU (uneven tiles need several to balance); one
+  // matrix: its items are alike, so whichever form takes fewer rounds of the chip (a wide item takes ~1.6 times a
+  // narrow one: its A reads feed twice the MFMAs)
+  const bool wide = a.te ? a.total >= 4 * (int64_t)cus : 8 * ((a.total + cus - 1) / cus) <= 5 * narrow_rounds;
   if (!wide) shape(256);
   const int64_t per = std::max<int64_t>(1, std::min<int64_t>(a.per_xcd, cus / GQ_XCDS));
   const dim3 grid((unsigned)(per * GQ_XCDS));
   if (wide) {
     if (hot) gateup ? gq_launch_t<true, false, 2, true>(a, grid, s) : gq_launch_t<false, false, 2, true>(a, grid, s);
-    else if (res) gq_launch_t<false, true, 2>(a, grid, s);
+    else if (e8) gq_launch_t<false, true, 2>(a, grid, s);
     else if (gateup) gq_launch_t<true, false, 2>(a, grid, s);
     else gq_launch_t<false, false, 2>(a, grid, s);
   } else {
     if (hot) gateup ? gq_launch_t<true, false, 1, true>(a, grid, s) : gq_launch_t<false, false, 1, true>(a, grid, s);
-    else if (res) gq_launch_t<false, true, 1>(a, grid, s);
+    else if (e8) gq_launch_t<false, true, 1>(a, grid, s);
     else if (gateup) gq_launch_t<true, false, 1>(a, grid, s);
     else gq_launch_t<false, false, 1>(a, grid, s);
   }
@@ -685,11 +718,12 @@ extern "C" int keep_vq_grouped_gemm_q8(const void* x, int x_dtype, int64_t x_row
   hipStream_t s = (hipStream_t)stream;
   GQArgs a{};
   a.x = x; a.xdt = x_dtype; a.x_rows = x_rows; a.lhs = lhs;
-  a.rs = gq_rowscale(x, x_dtype, x_rows, K, workspace, s);
+  a.rs = code_bits == 8 && x_dtype == KEEP_BF16 ? nullptr : gq_rowscale(x, x_dtype, x_rows, K, workspace, s);
   a.oidx = out_index; a.c0 = a.c1 = (const uint16_t*)codes; a.s0 = a.s1 = scales; a.sdt = scale_dtype;
   if (code_bits == 8) {  // `prepared` is the packed 8-bit E8 table, uint32[256]
     a.tq = prepared;
     a.tq_bad = nullptr;
+    a.add = 1;
   } else {
     a.tq = (const char*)prepared + TQ_OFFSET;
     a.tq_bad = (const uint32_t*)((const char*)prepared + TQ_FLAG_OFFSET);
@@ -699,6 +733,72 @@ extern "C" int keep_vq_grouped_gemm_q8(const void* x, int x_dtype, int64_t x_row
   a.out = out; a.odt = out_dtype;
   gq_launch(a, false, s, code_bits == 8);
   return launch_status("keep_vq_grouped_gemm_q8");
+}
+
+// Sizes, types and pointers that the two storing entry points below share.
+static int gq_store_check(const void* x, int x_dtype, const void* codes, int code_align, const void* scales,
+                          int scale_dtype, const void* tables, int64_t N, int64_t K, int64_t group_size,
+                          const void* out, int out_dtype) {
+  KEEP_REQUIRE(x_dtype == KEEP_F16 || x_dtype == KEEP_BF16, "the storing GEMMs need fp16 or bf16 activations");
+  KEEP_REQUIRE(dtype_ok(scale_dtype) && dtype_ok(out_dtype), "bad dtype enum");
+  KEEP_REQUIRE(gq_shape_ok(K, group_size),
+               "grouped GEMM needs K and the scale group multiples of %d, the group dividing K (K=%lld, "
+               "group_size=%lld)",
+               GQ_KB, (long long)K, (long long)group_size);
+  KEEP_REQUIRE(N > 0, "bad sizes");
+  KEEP_REQUIRE(x && codes && scales && tables && out, "null pointer argument");
+  KEEP_REQUIRE(aligned(x, 16) && aligned(codes, code_align) && aligned(scales, 4) && aligned(tables, 16),
+               "x and the table must be 16-byte aligned, codes %d bytes, scales 4 bytes", code_align);
+  return KEEP_OK;
+}
+
+extern "C" int keep_vq_grouped_gemm_e8(const void* x, int x_dtype, int64_t x_rows, const int32_t* lhs,
+                                       const int32_t* out_index, const uint8_t* codes, const void* scales,
+                                       int scale_dtype, const uint32_t* table, const int32_t* tile_expert,
+                                       const int32_t* tile_offset, const int32_t* tile_count, int64_t n_tiles,
+                                       int64_t routes, int64_t num_experts, int64_t N, int64_t K,
+                                       int64_t group_size, void* out, int out_dtype, void* stream) {
+  KEEP_REQUIRE_DIMS(x_rows, n_tiles, routes, num_experts, N, K, group_size);
+  if (n_tiles == 0 || routes == 0) return KEEP_OK;
+  const int rc = gq_store_check(x, x_dtype, codes, 8, scales, scale_dtype, table, N, K, group_size, out, out_dtype);
+  if (rc != KEEP_OK) return rc;
+  KEEP_REQUIRE(x_rows > 0 && num_experts > 0, "bad sizes");
+  KEEP_REQUIRE(tile_expert && tile_offset && tile_count, "null pointer argument");
+  GQArgs a{};
+  a.x = x; a.xdt = x_dtype; a.x_rows = x_rows; a.lhs = lhs; a.oidx = out_index;
+  a.c0 = a.c1 = (const uint16_t*)codes; a.s0 = a.s1 = scales; a.sdt = scale_dtype; a.tq = table;
+  a.te = tile_expert; a.to = tile_offset; a.tc = tile_count; a.n_tiles = n_tiles; a.routes = routes;
+  a.E = num_experts; a.N = N; a.K = K; a.G = K / group_size; a.kpg = group_size / GQ_KB;
+  a.out = out; a.odt = out_dtype;
+  gq_launch(a, false, (hipStream_t)stream, true);
+  return launch_status("keep_vq_grouped_gemm_e8");
+}
+
+extern "C" int keep_vq_gemm(const void* x, int x_dtype, int64_t rows, const void* codes, int code_bits,
+                            const void* scales, int scale_dtype, const void* tables, int64_t N, int64_t K,
+                            int64_t group_size, void* workspace, int64_t workspace_bytes, void* out, int out_dtype,
+                            void* stream) {
+  KEEP_REQUIRE_DIMS(rows, N, K, group_size);
+  KEEP_REQUIRE(code_bits == 16 || code_bits == 8, "code_bits must be 8 or 16, got %d", code_bits);
+  if (rows == 0) return KEEP_OK;
+  const int rc = gq_store_check(x, x_dtype, codes, code_bits, scales, scale_dtype, tables, N, K, group_size, out,
+                                out_dtype);
+  if (rc != KEEP_OK) return rc;
+  const bool factors = code_bits == 16 && x_dtype == KEEP_BF16;
+  KEEP_REQUIRE(!factors || (workspace && aligned(workspace, 16) && workspace_bytes >= gq_ws_bytes(rows)),
+               "bf16 rows against E8P codes need a 16-byte aligned workspace of %lld bytes, got %lld",
+               (long long)gq_ws_bytes(rows), (long long)workspace_bytes);
+  hipStream_t s = (hipStream_t)stream;
+  GQArgs a{};
+  a.x = x; a.xdt = x_dtype; a.x_rows = rows;
+  a.rs = factors ? gq_rowscale(x, x_dtype, rows, K, workspace, s) : nullptr;
+  a.c0 = a.c1 = (const uint16_t*)codes; a.s0 = a.s1 = scales; a.sdt = scale_dtype;
+  a.tq = code_bits == 16 ? (const char*)tables + TQ_OFFSET : (const char*)tables;
+  a.n_tiles = (rows + GQ_M - 1) / GQ_M; a.routes = rows;
+  a.E = 1; a.N = N; a.K = K; a.G = K / group_size; a.kpg = group_size / GQ_KB;
+  a.out = out; a.odt = out_dtype;
+  gq_launch(a, false, s, code_bits == 8);
+  return launch_status("keep_vq_gemm");
 }
 
 extern "C" int keep_vq_grouped_swiglu_q8(const void* x, int x_dtype, int64_t x_rows, const int32_t* lhs,

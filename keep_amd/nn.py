@@ -135,8 +135,7 @@ class QuantizedVQLinear:
             w = w @ torch.as_tensor(rotation_matrix).to(device=device, dtype=torch.float32)
         q = quantize_weight_rtn(w, group_size=group_size, code_bits=code_bits)
         out_dim, in_dim = w.shape
-        return cls(input_dims=in_dim, output_dims=out_dim, codes=q.codes, scales=q.scales,
-                   codebook=torch.from_numpy(q.codebook.view(np.int32)).to(device), bias=bias,
+        return cls(input_dims=in_dim, output_dims=out_dim, codes=q.codes, scales=q.scales, bias=bias,
                    group_size=q.group_size, code_bits=q.code_bits, rht_signs=rht_signs,
                    rotation_matrix=rotation_matrix)
 

@@ -38,6 +38,10 @@ NO_RESIDUAL = 0xFFFFFFFF
 # below it the wave-per-rows mat-vec serves every route directly.
 GEMM_ROUTE_THRESHOLD = 128
 GEMM_ROUTE_TILE = 64
+# rows x outputs from which one matrix goes to the MFMA GEMM. Both times grow with K (the mat-vec's also with rows
+# x outputs: 2.0 us per row of 4096 x 4096 in 8 bits, 2.9 in 16; the GEMM's floor there is 25 us in 8 bits, 34 / 42
+# in 16 for fp16 / bf16 rows), so they meet near 13 rows of 4096 outputs and near 100 of 520 at K = 1024.
+MATRIX_GEMM_CELLS = 1 << 16
 _VERIFY_DEFAULT_M_ROWS = 4
 VERIFY_MROWS_VALUES = (1, 2, 3, 4, 8)
 
@@ -112,8 +116,17 @@ def prepared_table(codebook: torch.Tensor) -> torch.Tensor:
     nbytes = _lib.load().keep_e8p_prepared_bytes()
     out = torch.empty(nbytes, dtype=torch.uint8, device=codebook.device)
     _lib.call("keep_e8p_prepare", codebook.data_ptr(), out.data_ptr(), _stream(codebook.device))
+    if not torch.cuda.is_current_stream_capturing():
+        torch.cuda.current_stream(codebook.device).synchronize()  # once: any stream may read it from here on
     _PREPARED[key] = (codebook, out)
     return out
+
+
+def _may_prepare(codebook: torch.Tensor) -> bool:
+    """Whether ``prepared_table`` can serve a call that needs not have it: a table first built under graph
+    capture would be filled by that graph's replays only."""
+
+    return (codebook.data_ptr(), str(codebook.device)) in _PREPARED or not torch.cuda.is_current_stream_capturing()
 
 
 def half2_pairs(grid: np.ndarray) -> np.ndarray:
@@ -348,6 +361,36 @@ def grouped_gemm(x: torch.Tensor, codes: torch.Tensor, scales: torch.Tensor, cod
     return out
 
 
+def grouped_gemm_e8(x: torch.Tensor, codes: torch.Tensor, scales: torch.Tensor, codebook: torch.Tensor,
+                    tile_descriptors, *, lhs: torch.Tensor | None, out_index: torch.Tensor | None, routes: int,
+                    input_dims: int, output_dims: int, group_size: int) -> torch.Tensor:
+    """``keep_vq_grouped_gemm_e8``: ``grouped_gemm`` on 8-bit E8 codes (fp16 or bf16 rows as they are)."""
+
+    device = x.device
+    out = torch.empty((routes, output_dims), dtype=x.dtype, device=device)
+    te, to, tc = tile_descriptors
+    _lib.call("keep_vq_grouped_gemm_e8", x.data_ptr(), _dtype_code(x, "x"), x.shape[0], _ptr(lhs), _ptr(out_index),
+              codes.data_ptr(), scales.data_ptr(), _dtype_code(scales, "scales"), codebook.data_ptr(), te.data_ptr(),
+              to.data_ptr(), tc.data_ptr(), te.numel(), routes, codes.shape[0], output_dims, input_dims, group_size,
+              out.data_ptr(), _DT[out.dtype], _stream(device))
+    return out
+
+
+def matrix_gemm(x: torch.Tensor, codes: torch.Tensor, scales: torch.Tensor, codebook: torch.Tensor, *,
+                input_dims: int, output_dims: int, group_size: int, code_bits: int) -> torch.Tensor:
+    """``keep_vq_gemm``: one matrix (``codes [N, K/8]``) against all rows of ``x`` on the matrix cores."""
+
+    device = x.device
+    M = x.shape[0]
+    out = torch.empty((M, output_dims), dtype=x.dtype, device=device)
+    ws = _q8_workspace(M, input_dims, device) if code_bits == 16 and x.dtype == torch.bfloat16 else None
+    table = prepared_table(codebook) if code_bits == 16 else codebook
+    _lib.call("keep_vq_gemm", x.data_ptr(), _DT[x.dtype], M, codes.data_ptr(), code_bits, scales.data_ptr(),
+              _dtype_code(scales, "scales"), table.data_ptr(), output_dims, input_dims, group_size, _ptr(ws),
+              0 if ws is None else ws.numel(), out.data_ptr(), _DT[out.dtype], _stream(device))
+    return out
+
+
 def grouped_residual_add(out: torch.Tensor, x: torch.Tensor, codes: torch.Tensor, scales: torch.Tensor,
                          tile_descriptors, *, lhs: torch.Tensor | None, out_index: torch.Tensor | None, routes: int,
                          input_dims: int, output_dims: int, group_size: int,
@@ -485,11 +528,18 @@ def route_combine(y: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype 
 
 
 def gemm_eligible(*, code_bits: int, x_dtype: torch.dtype, input_dims: int, group_size: int) -> bool:
-    """Whether the grouped GEMM (fp16 matrix cores) serves this call (E8P, fp16/bf16/fp32
-    activations, K and the scale group multiples of 128)."""
+    """Whether the grouped GEMM (16-bit matrix cores) serves this call: K and the scale group multiples of
+    128, E8P with fp16/bf16/fp32 activations or 8-bit E8 with fp16/bf16 ones (fp32 rows would lose bits)."""
 
-    return (code_bits == 16 and x_dtype in (torch.float16, torch.bfloat16, torch.float32) and input_dims % 128 == 0
-            and group_size % 128 == 0)
+    return ((x_dtype in (torch.float16, torch.bfloat16) or (code_bits == 16 and x_dtype == torch.float32))
+            and input_dims % 128 == 0 and group_size % 128 == 0)
+
+
+def _gemm_pointers_ok(codes: torch.Tensor, scales: torch.Tensor, codebook: torch.Tensor, code_bits: int) -> bool:
+    """The storing GEMMs' loads: one K block of codes per lane, scales in aligned words, the table in 16-byte
+    rows. (Views at odd offsets stay on the mat-vec, whose loads are narrower.)"""
+
+    return not (codes.data_ptr() % code_bits or scales.data_ptr() % 4 or codebook.data_ptr() % 16)
 
 
 # --------------------------------------------------------------------------- decode
@@ -581,6 +631,13 @@ def vq_qmm(x, codes, scales, codebook=None, *, in_dim: int, out_dim: int, group_
         raise ValueError(f"scales must have shape ({out_dim}, {in_dim // group_size}), found {tuple(s.shape)}")
     cb = _codebook_tensor(codebook, code_bits, device)
     M = xt.shape[0]
+    # E8P on the matrix cores takes the default table only: they decode it from odd half-units, the mat-vec any
+    if (M * out_dim >= MATRIX_GEMM_CELLS and xt.dtype in (torch.float16, torch.bfloat16)
+            and gemm_eligible(code_bits=code_bits, x_dtype=xt.dtype, input_dims=in_dim, group_size=group_size)
+            and (code_bits == 8 or (cb is _default_codebook(16, device) and _may_prepare(cb)))
+            and _gemm_pointers_ok(c, s, cb, code_bits)):
+        return matrix_gemm(xt, c, s, cb, input_dims=in_dim, output_dims=out_dim, group_size=group_size,
+                           code_bits=code_bits)
     return routed_matvec(xt, c.reshape(1, out_dim, -1), s.reshape(1, out_dim, -1), cb, None, input_dims=in_dim,
                          output_dims=out_dim, group_size=group_size, code_bits=code_bits, routes=M)
 
@@ -670,7 +727,8 @@ def gather_vqmm(x, codes, scales, codebook, rhs_indices, *, lhs_indices=None, in
     if R == 0:
         return torch.zeros(out_shape, dtype=od, device=device)
 
-    eligible = gemm_eligible(code_bits=code_bits, x_dtype=xt.dtype, input_dims=input_dims, group_size=group_size)
+    eligible = gemm_eligible(code_bits=code_bits, x_dtype=xt.dtype, input_dims=input_dims, group_size=group_size) \
+        and (code_bits == 16 or _gemm_pointers_ok(c, s, cb, 8))
     strategy = route_strategy
     if strategy == "auto":
         strategy = "sorted_tiled" if eligible and (sorted_indices or R >= GEMM_ROUTE_THRESHOLD) else "direct"
@@ -686,6 +744,10 @@ def gather_vqmm(x, codes, scales, codebook, rhs_indices, *, lhs_indices=None, in
     full_lhs = lhs if lhs is not None else torch.arange(R, dtype=torch.int32, device=device) // x_div
     order, inverse, _, _, te, to, tc, _ = route_plan(flat_rhs, E, GEMM_ROUTE_TILE)
     sorted_lhs = full_lhs[order.long()].contiguous()
+    if eligible and code_bits == 8:
+        y = grouped_gemm_e8(xt, c, s, cb, (te, to, tc), lhs=sorted_lhs, out_index=order, routes=R,
+                            input_dims=input_dims, output_dims=output_dims, group_size=group_size)
+        return y.reshape(out_shape)
     if eligible:  # rows land in route order directly
         y = grouped_gemm(xt, c, s, cb, (te, to, tc), lhs=sorted_lhs, routes=R, input_dims=input_dims,
                          output_dims=output_dims, group_size=group_size, out_index=order)
@@ -739,7 +801,14 @@ def gather_vqmm_sorted_routes(x, codes, scales, codebook, sorted_rhs, sorted_lhs
         xt = xt.to(torch.float16)  # the reference's native path runs fp16 activations (vq_switch.py:758-761)
     skip_gather = x_pre_sorted and xt.shape[0] == R
     use_lhs = None if skip_gather else lhs
-    if gemm_eligible(code_bits=code_bits, x_dtype=xt.dtype, input_dims=input_dims, group_size=group_size):
+    eligible = gemm_eligible(code_bits=code_bits, x_dtype=xt.dtype, input_dims=input_dims, group_size=group_size)
+    if eligible and code_bits == 8 and R >= GEMM_ROUTE_THRESHOLD and _gemm_pointers_ok(c, s, cb, 8):
+        # a plan of its own, rows back at their positions: 8-bit calls never had to be sorted, nor their tiles right
+        order, _, _, _, te, to, tc, _ = route_plan(rhs, E, GEMM_ROUTE_TILE)
+        return grouped_gemm_e8(xt, c, s, cb, (te, to, tc), lhs=order if use_lhs is None else use_lhs[order.long()],
+                               out_index=order, routes=R, input_dims=input_dims, output_dims=output_dims,
+                               group_size=group_size)
+    if eligible and code_bits == 16:
         if tile_descriptors is None:
             _, _, _, _, te, to, tc, _ = route_plan(rhs, E, GEMM_ROUTE_TILE)
         else:

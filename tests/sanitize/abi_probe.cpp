@@ -72,6 +72,8 @@ int main() {
   PROBE(keep_moe_tiles_layer);
   PROBE(keep_vq_grouped_gemm_q8_workspace_bytes);
   PROBE(keep_vq_grouped_gemm_q8);
+  PROBE(keep_vq_grouped_gemm_e8);
+  PROBE(keep_vq_gemm);
   PROBE(keep_vq_grouped_swiglu_q8);
   PROBE(keep_vq_grouped_swiglu_nested_q8);
   PROBE(keep_vq_grouped_gemm_nested_q8);

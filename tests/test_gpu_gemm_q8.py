@@ -236,3 +236,55 @@ def test_grouped_gemm_wide_items(dev, form, G):
             want = ops.round_bf16(ops.swiglu(oracle(*gate), oracle(*up), limit=7.0))
         got = h[inverse.long()].float().cpu().numpy()
         assert ops.elementwise_ok(got, want, rtol=TOL + 2.0 ** -7), "h beyond one bf16 ulp of the oracle's"
+
+
+@pytest.mark.parametrize("code_bits", [8, 16])
+@pytest.mark.parametrize("xdt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K,G", [(1024, 64, 128, 1), (129, 513, 640, 5), (2112, 1040, 256, 2), (65, 2056, 384, 1)])
+def test_one_matrix_gemm_vs_oracle(dev, code_bits, xdt, M, N, K, G):
+    """vq_qmm on the MFMA GEMM: partial row tiles (65 = one row past a tile),
+    partial column blocks, one K block, both item widths, per-row and grouped
+    scales. fp32 row dots against the fp64 oracle: within the rounding of the
+    16-bit output plus the path's bound."""
+    rng = np.random.default_rng(M + N)
+    codes = rng.integers(0, 1 << code_bits, (N, K // 8)).astype(np.uint8 if code_bits == 8 else np.uint16)
+    scales = np.exp(rng.normal(0, 0.3, (N, G))).astype(np.float16)
+    x = torch.from_numpy(rng.standard_normal((M, K)).astype(np.float32)).to(dev).to(xdt)
+    assert M * N >= kops.MATRIX_GEMM_CELLS
+    y = kops.vq_qmm(x, _t(codes, dev), _t(scales, dev), in_dim=K, out_dim=N, group_size=K // G, code_bits=code_bits)
+    assert y.dtype == xdt
+    dense = (e8p.decode_e8_1bit(codes) if code_bits == 8 else e8p.decode_e8p(codes)).astype(np.float64)
+    dense = dense.reshape(N, K) * np.repeat(scales.astype(np.float64), K // G, -1)
+    want = x.double().cpu().numpy() @ dense.T
+    ulp = 2.0 ** -9 if xdt == torch.float16 else 2.0 ** -8
+    _check(y, want, tol=TOL + ulp)
+
+
+@pytest.mark.parametrize("xdt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("E,T,k,N,K,G", [(7, 43, 3, 72, 128, 1), (3, 90, 2, 520, 512, 4), (200, 700, 4, 1032, 256, 2)])
+def test_routed_8bit_gemm_vs_oracle(dev, xdt, E, T, k, N, K, G):
+    """8-bit E8 routes on the sorted-route GEMM (tiles of one and two m-tiles,
+    partial column blocks, items of 256 and 512 columns), an out-of-range route
+    (NaN), and gather_vqmm_sorted_routes on unsorted routes: each row its own."""
+    rng = np.random.default_rng(E + T)
+    codes = rng.integers(0, 256, (E, N, K // 8), dtype=np.uint8)
+    scales = np.exp(rng.normal(0, 0.3, (E, N, G))).astype(np.float16)
+    rhs = rng.integers(0, E, (T, k)).astype(np.int32)
+    rhs[1, 0] = E
+    x = torch.from_numpy(rng.standard_normal((T, K)).astype(np.float32)).to(dev).to(xdt)
+    dense = e8p.decode_e8_1bit(codes).astype(np.float64).reshape(E, N, K) * np.repeat(
+        scales.astype(np.float64), K // G, -1)
+    flat = rhs.reshape(-1)
+    good = flat < E
+    xd = x.double().cpu().numpy()
+    want = np.stack([dense[min(e, E - 1)] @ xd[i // k] for i, e in enumerate(flat)])
+    ulp = 2.0 ** -9 if xdt == torch.float16 else 2.0 ** -8
+    kw = dict(input_dims=K, output_dims=N, group_size=K // G, code_bits=8)
+    with keep_amd.trace_gather_vqmm_calls() as tr:
+        y = kops.gather_vqmm(x, _t(codes, dev), _t(scales, dev), None, _t(rhs, dev), **kw).reshape(T * k, N)
+    assert tr[0]["implementation"] == "mfma_grouped_gemm"
+    lhs = torch.arange(T * k, device=dev, dtype=torch.int32) // k
+    z = kops.gather_vqmm_sorted_routes(x, _t(codes, dev), _t(scales, dev), None, _t(flat, dev), lhs, **kw)
+    for out in (y, z):
+        assert torch.isnan(out[torch.from_numpy(~good)]).all()
+        _check(out[torch.from_numpy(good)], want[good], tol=TOL + ulp)
