@@ -75,6 +75,12 @@ int keep_vq_encode(const float* vectors, int64_t n, int code_bits, const float* 
 int keep_group_absmax(const float* x, int64_t groups_total, int64_t group_size, float divisor, float* scales,
                       void* stream);
 
+/* keep_group_absmax's scales as the RTN quantiser takes them, in one pass:
+ * `safe` (fp32, groups_total) is what the vectors are divided by, 1 where the
+ * scale is not positive; `stored` (fp16, groups_total) the scale it keeps. */
+int keep_rtn_scales(const float* x, int64_t groups_total, int64_t group_size, float divisor, float* safe,
+                    void* stored, void* stream);
+
 /* Routed VQ mat-vec: out[r, :] = W[rhs[r]] . x[row(r), :] for r < routes,
  * row(r) = lhs ? lhs[r] : r / x_div. W[e] is [N, K] given by codes [E, N, K/8]
  * and scales [E, N, K/group_size]. fp32 accumulate. rhs may be NULL when

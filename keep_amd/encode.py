@@ -133,15 +133,17 @@ def quantize_weight_rtn(weight, *, group_size: int = 512, code_bits: int = 8, co
     groups = in_dim // group_size
     divisor = codebook_max_abs(code_bits)
     if scale_estimator == "max_abs":
-        scales = torch.empty((out_dim, groups), dtype=torch.float32, device=device)
-        _lib.call("keep_group_absmax", w.data_ptr(), out_dim * groups, group_size, divisor, scales.data_ptr(),
-                  ops._stream(device))
+        safe = torch.empty((out_dim, groups), dtype=torch.float32, device=device)
+        stored = torch.empty((out_dim, groups), dtype=torch.float16, device=device)
+        _lib.call("keep_rtn_scales", w.data_ptr(), out_dim * groups, group_size, divisor, safe.data_ptr(),
+                  stored.data_ptr(), ops._stream(device))
     else:
         q = torch.quantile(w.abs().reshape(out_dim, groups, group_size), 0.99, dim=-1)
         scales = (q.double() / divisor).float()
-    safe = torch.where(scales > 0, scales, torch.ones_like(scales)).contiguous()
+        safe = torch.where(scales > 0, scales, torch.ones_like(scales)).contiguous()
+        stored = scales.half()
     codes = _encode(w.reshape(-1, CODEWORD_DIM), code_bits, scales=safe, vps=group_size // CODEWORD_DIM)
     table = ops.e8_1bit_packed() if code_bits == 8 else ops.e8p_packed_abs_grid()
-    return QuantizedWeight(codes=codes.reshape(out_dim, in_dim // CODEWORD_DIM), scales=scales.half(),
+    return QuantizedWeight(codes=codes.reshape(out_dim, in_dim // CODEWORD_DIM), scales=stored,
                            codebook=table, group_size=group_size, code_bits=code_bits,
                            scale_estimator=scale_estimator)

@@ -48,6 +48,7 @@ int main() {
   PROBE(keep_e8_1bit_decode);
   PROBE(keep_vq_encode);
   PROBE(keep_group_absmax);
+  PROBE(keep_rtn_scales);
   PROBE(keep_vq_matvec);
   PROBE(keep_e8_1bit_matvec);
   PROBE(keep_vq_matvec_tiles);

@@ -162,3 +162,24 @@ def test_quantized_vq_switch_linear_from_weights(dev, code_bits, transform):
     assert np.abs(y - want).max() <= 2e-3 * np.abs(want).max()
     with pytest.raises(ValueError, match="3D"):
         keep_amd.QuantizedVQSwitchLinear.from_weights(torch.from_numpy(w[0]).to(dev), group_size=g)
+
+
+@pytest.mark.parametrize("code_bits", [8, 16])
+@pytest.mark.parametrize("n", [1, 31, 33, 128, 4097])
+def test_encode_bounds_edges_bit_exact(dev, code_bits, n):
+    """Groups of 32 vectors with a remainder; magnitudes from far below the
+    table's to past the +-64 the bounds serve, zero vectors, many equal
+    distances (small dyadic values), and non-finite vectors among them: every
+    finite vector's code is the exhaustive scan's."""
+    rng = np.random.default_rng(1000 * code_bits + n)
+    kind = rng.integers(0, 6, n)
+    v = rng.standard_normal((n, 8)) * np.array([0.6, 1e-5, 9.0, 0.0, 0.0, 300.0])[kind][:, None]
+    v[kind == 4] = rng.integers(-8, 9, ((kind == 4).sum(), 8)) / 4
+    v = v.astype(np.float32)
+    odd = np.zeros(n, bool)
+    if n > 40:
+        v[7, 3], v[39, 0], v[40] = np.nan, np.inf, -np.inf
+        odd[[7, 39, 40]] = True
+    enc = kenc.encode_e8p_rtn if code_bits == 16 else kenc.encode_e8_1bit_rtn
+    got = _u(enc(torch.from_numpy(v).to(dev)))
+    np.testing.assert_array_equal(got[~odd], oenc.nearest(v[~odd], code_bits))
