@@ -409,6 +409,27 @@ int keep_moe_tiles_layer(const float* logits, const float* bias_served, const fl
                          uint8_t* admit, void* h_work, void* workspace, int64_t workspace_bytes, void* out,
                          int out_dtype, void* stream);
 
+/* The same few-token layer for hidden sizes up to 8192 (H a multiple of 256;
+ * every other limit, the workspace and the arithmetic as keep_moe_tiles /
+ * keep_moe_tiles_layer): from 17 K slices on, each gate/up wave takes one or
+ * two projections of a second slice. */
+int keep_moe_wide_supported(int64_t T, int64_t num_experts, int64_t H, int64_t I, int64_t k, int64_t group_size_h,
+                            int64_t group_size_i);
+int keep_moe_wide(const void* x, int x_dtype, int64_t T, int64_t H, int64_t I, const int32_t* idx, const float* w,
+                  int64_t k, int64_t num_experts, const uint16_t* gate_codes, const void* gate_scales, const
+                  uint16_t* up_codes, const void* up_scales, const uint16_t* down_codes, const void* down_scales,
+                  int scale_dtype, int64_t group_size_h, int64_t group_size_i, const void* prepared, float
+                  swiglu_limit, void* h_work, void* workspace, int64_t workspace_bytes, void* out, int out_dtype,
+                  void* stream);
+int keep_moe_wide_layer(const float* logits, const float* bias_served, const float* bias_demand, int score_func, int
+                        renormalize, float route_scale, float tau, const int32_t* slot_map, int64_t num_slots,
+                        int64_t num_experts, int64_t k, const void* x, int x_dtype, int64_t T, int64_t H, int64_t I,
+                        const uint16_t* gate_codes, const void* gate_scales, const uint16_t* up_codes, const void*
+                        up_scales, const uint16_t* down_codes, const void* down_scales, int scale_dtype, int64_t
+                        group_size_h, int64_t group_size_i, const void* prepared, float swiglu_limit, int32_t* idx,
+                        float* w, int32_t* want, float* want_score, uint8_t* admit, void* h_work, void* workspace,
+                        int64_t workspace_bytes, void* out, int out_dtype, void* stream);
+
 /* Prefill grouped GEMM on the fp16 matrix cores over expert-sorted routes
  * (tiles of <= 64 routes of one expert from keep_route_plan): for every tile
  * t and route i < tile_count[t], with p = tile_offset[t] + i,

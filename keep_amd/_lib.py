@@ -41,8 +41,13 @@ _SIGS = {
                         c_int, c_int64, c_int64, _P, _P, c_float, _P, _P, c_int, _P],
     "keep_moe_tiles": [_P, c_int, c_int64, c_int64, c_int64, _P, _P, c_int64, c_int64, _P, _P, _P, _P, _P, _P, c_int,
                        c_int64, c_int64, _P, c_float, _P, _P, c_int64, _P, c_int, _P],
+    "keep_moe_wide": [_P, c_int, c_int64, c_int64, c_int64, _P, _P, c_int64, c_int64, _P, _P, _P, _P, _P, _P, c_int,
+                       c_int64, c_int64, _P, c_float, _P, _P, c_int64, _P, c_int, _P],
     "keep_moe_tiles_workspace_bytes": [c_int64, c_int64, c_int64, c_int64],
     "keep_moe_tiles_layer": [_P, _P, _P, c_int, c_int, c_float, c_float, _P, c_int64, c_int64, c_int64, _P, c_int,
+                             c_int64, c_int64, c_int64, _P, _P, _P, _P, _P, _P, c_int, c_int64, c_int64, _P, c_float,
+                             _P, _P, _P, _P, _P, _P, _P, c_int64, _P, c_int, _P],
+    "keep_moe_wide_layer": [_P, _P, _P, c_int, c_int, c_float, c_float, _P, c_int64, c_int64, c_int64, _P, c_int,
                              c_int64, c_int64, c_int64, _P, _P, _P, _P, _P, _P, c_int, c_int64, c_int64, _P, c_float,
                              _P, _P, _P, _P, _P, _P, _P, c_int64, _P, c_int, _P],
     "keep_vq_grouped_gemm_q8_workspace_bytes": [c_int64, c_int64],
@@ -67,6 +72,7 @@ _SIGS = {
                                        _P, _P, _P, c_int64, c_int64, c_int64, c_int64, c_int64, _P, c_int64, _P,
                                        c_int, _P],
     "keep_moe_tiles_supported": [c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64],
+    "keep_moe_wide_supported": [c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64],
     "keep_moe_gateup": [_P, c_int, c_int64, c_int64, c_int64, _P, _P, c_int64, c_int64, _P, _P, _P, _P, c_int,
                         c_int64, _P, _P, c_float, _P, _P],
     "keep_moe_layer_supported": [c_int64, c_int64, c_int64, c_int64, c_int64, c_int64],

@@ -83,10 +83,11 @@ __device__ __forceinline__ void mt_xterms(const void* x, int H, uint4* xt, float
   if (lane == 0) xinv[(size_t)t * S + s] = inv4s;
 }
 
-// Block t, wave s: token t's terms of slice s.
+// Block (t, b), wave w: token t's terms of slice 16 b + w.
 template <bool XBF>
 __global__ __launch_bounds__(1024) void k_q8_xterms(const void* x, int H, uint4* xt, float* xinv) {
-  mt_xterms<XBF>(x, H, xt, xinv, (int)blockIdx.x, (int)(threadIdx.x >> 6), (int)(threadIdx.x & 63));
+  const int s = (int)blockIdx.y * 16 + (int)(threadIdx.x >> 6);
+  if (s < (H >> 8)) mt_xterms<XBF>(x, H, xt, xinv, (int)blockIdx.x, s, (int)(threadIdx.x & 63));
 }
 
 // ------------------------------------------------------------------ fused prologue (few tokens)
@@ -125,7 +126,7 @@ __global__ __launch_bounds__(1024) void k_mt_prologue(MTPro p) {
   __shared__ int32_t s_r[MT_FUSED_MAX_T * 16];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   if ((int)blockIdx.x < p.T) {
-    if (wv < (p.H >> 8)) mt_xterms<XBF>(p.x, p.H, p.xt, p.xinv, (int)blockIdx.x, wv, lane);
+    for (int s = wv; s < (p.H >> 8); s += 16) mt_xterms<XBF>(p.x, p.H, p.xt, p.xinv, (int)blockIdx.x, s, lane);
     return;
   }
   for (int t = wv; t < p.T; t += 16) {
@@ -294,10 +295,18 @@ __device__ __forceinline__ int mt_route_of_lanes(int rr, uint32_t i) {
 // routes: A row 4i + t is term t of route i's token (t < 3; row 4i + 3 is
 // zero), so D rows 4i .. 4i + 2 of column j, in lane 16 i + j, are route i's
 // three partial dots with weight row j.
-template <bool XBF, int RPER>
+// WIDE: 17..32 K slices (H up to 8192). A wave owns slice wv and, of the second
+// set, slice 16 + wv, or where that set holds at most 8 slices one projection
+// of slice 16 + wv % 8, so that all 16 waves share it. A unit's two sets take
+// the place of two units in flight (the same bytes), and their dots are added
+// before the cross-wave sum. 4 bf16 tokens, top-8 of 128 experts of 7168 x
+// 2048, groups of 512: 85 us per layer against 286 on the packed-table
+// mat-vecs, which decode every route's codes on the VALU.
+template <bool XBF, int RPER, bool WIDE = false>
 __global__ __launch_bounds__(1024) void k_moeq_gateup_tiles(MTArgs a, MTRoute p) {
   constexpr int SEG = 128;  // units per segment (h staging capacity)
   constexpr bool ROUTE = RPER > 0;
+  static_assert(!(ROUTE && WIDE), "the routed kernel takes one slice per wave");
   __shared__ uint4 tqs[TQR_BYTES / 16];
   __shared__ float gred[2][16][2][MT_TILE][16];  // [parity][wave][gate, up][route][row]
   __shared__ uint16_t hst[MT_TILE][SEG * 16];    // the segment's h rows
@@ -394,12 +403,33 @@ __global__ __launch_bounds__(1024) void k_moeq_gateup_tiles(MTArgs a, MTRoute p)
   q8v4 A[4];
   float inv;
   uint4 araw[4];
-  auto issue_a = [&](int route_a, int route_d) {  // the routes of A row j and of this lane's D rows
+  auto issue_a = [&](int route_a, int route_d, int sl, float& inv) {  // the routes of A row j and of this lane's D rows
     const int tok_a = route_a / a.k, tok_d = route_d / a.k;
     const uint4* asrc = a.xt + ((size_t)tok_a * a.S + sl) * 48 + min(j & 3u, 2u) * 16 + g * 4;
 #pragma unroll
     for (int m = 0; m < 4; ++m) araw[m] = ldg16_q(asrc + m);
     inv = a.xinv[(size_t)tok_d * a.S + sl];
+  };
+  // WIDE: the second set's slice, and whether this wave takes one of its projections (hi: up) or both
+  const int n1 = WIDE ? a.S - 16 : 0;
+  const bool split = n1 <= 8, hi = split && wv >= 8;
+  const int w1 = split ? wv & 7 : wv;
+  const bool dec1 = WIDE && w1 < n1;
+  const int sl1 = 16 + (dec1 ? w1 : 0);
+  const uint32_t kc1 = (uint32_t)sl1 * 32 + g * 8;
+  const uint32_t grp1 = (uint32_t)(sl1 * 256) / (uint32_t)a.gsz_h;
+  q8v4 A1[WIDE ? 4 : 1];
+  float inv1 = 0.f;
+  auto load_set1 = [&](int u, Buf& b) {
+    if (!dec1) return;
+    const uint32_t row = unit_row(u) + j;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      if (t == 1 && split) break;
+      const bool up = t == 1 || hi;
+      b.q[t] = ldg16_q((up ? a.uc : a.gc) + (size_t)row * C + kc1);
+      if (!g1) b.s[t] = ldg4_q((const char*)(up ? a.us : a.gs) + ((row * (uint32_t)a.Gh + grp1) * sbytes & ~3u));
+    }
   };
   // routed: the wave forms the terms of its K slice itself, for the tile's four routes (routes past its
   // count repeat the last one), from its x chunks (issue_x), into its LDS rows; then A and 1 / (4 s)
@@ -438,7 +468,7 @@ __global__ __launch_bounds__(1024) void k_moeq_gateup_tiles(MTArgs a, MTRoute p)
       inv = RL.xinv[wv][g];
     }
   };
-  auto build_a = [&]() {
+  auto build_a = [&](q8v4 (&A)[4]) {
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
       const bool z = (j & 3u) == 3u;
@@ -469,18 +499,50 @@ __global__ __launch_bounds__(1024) void k_moeq_gateup_tiles(MTArgs a, MTRoute p)
             __builtin_amdgcn_readfirstlane(mt_route_of_lanes(rr, 2)), __builtin_amdgcn_readfirstlane(mt_route_of_lanes(rr, 3)));
     wait_vm_q<0>();
     build_x();
+    build_a(A);
+  } else if constexpr (WIDE) {
+    issue_a(mt_route_of_lanes(rr, j >> 2), mt_route_of_lanes(rr, g), sl1, inv1);
+    build_a(A1);
+    issue_a(mt_route_of_lanes(rr, j >> 2), mt_route_of_lanes(rr, g), sl, inv);
+    load_unit(u0, b0);
+    load_set1(u0, b1);
+    wait_vm_q<0>();
+    build_a(A);
   } else {
-    issue_a(mt_route_of_lanes(rr, j >> 2), mt_route_of_lanes(rr, g));
+    issue_a(mt_route_of_lanes(rr, j >> 2), mt_route_of_lanes(rr, g), sl, inv);
     load_unit(u0, b0);
     load_unit(u0 + 1, b1);
     wait_vm_q<4>();  // all but the second unit's four loads: the image, A and the first unit (loads retire in order)
+    build_a(A);
   }
-  build_a();
   rt_lds_barrier();  // the table image and the tile table
   if (ntb > 1) {
     nxt_row = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_td[1].row);
     nxt_nr = __builtin_amdgcn_readfirstlane(s_td[1].nr);
   }
+  // a unit's sums over the waves, SwiGLU (thread (route i, row jj)) and the staged h rows
+  auto finish = [&](int u, int par, const float (&scl)[2]) {
+    rt_lds_barrier();
+    if ((int)threadIdx.x < cur_nr * 16 && u < ue) {
+      // the LDS address is rebuilt here, not kept across the unit loop: held, it is spilled, and a
+      // reload from scratch waits for every code load in flight
+      int tid = (int)threadIdx.x;
+      asm volatile("" : "+v"(tid));
+      const int i = tid >> 4, jj = tid & 15;
+      float gsum = 0.f, usum = 0.f;
+      for (int w = 0; w < (WIDE ? 16 : a.S); ++w) {
+        gsum += gred[par][w][0][i][jj];
+        usum += gred[par][w][1][i][jj];
+      }
+      if (g1) {  // this lane's own words: row jj of the unit
+        gsum *= scl[0];
+        usum *= scl[1];
+      }
+      float hv = silu_mul(gsum, usum, a.limit);
+      if (tq_bad) hv = __builtin_nanf("");
+      hst[i][(u - us) * 16 + jj] = from_float<bf16s>(hv).bits;
+    }
+  };
   auto unit = [&](int u, Buf& b, int par) {
     const uint32_t rowc = unit_row(u);
     q8v4 B[2][4];
@@ -503,31 +565,55 @@ __global__ __launch_bounds__(1024) void k_moeq_gateup_tiles(MTArgs a, MTRoute p)
         if ((int)g < cur_nr) gred[par][wv][t][g][j] = g1 ? d * inv : d * inv * scl[t];
       }
     }
-    rt_lds_barrier();
-    // SwiGLU: thread (route i, row jj) -> the staged h rows
-    if ((int)threadIdx.x < cur_nr * 16 && u < ue) {
-      // the LDS address is rebuilt here, not kept across the unit loop: held, it is spilled, and a
-      // reload from scratch waits for every code load in flight
-      int tid = (int)threadIdx.x;
-      asm volatile("" : "+v"(tid));
-      const int i = tid >> 4, jj = tid & 15;
-      float gsum = 0.f, usum = 0.f;
-      for (int w = 0; w < a.S; ++w) {
-        gsum += gred[par][w][0][i][jj];
-        usum += gred[par][w][1][i][jj];
-      }
-      if (g1) {  // this lane's own words: row jj of the unit
-        gsum *= scl[0];
-        usum *= scl[1];
-      }
-      float hv = silu_mul(gsum, usum, a.limit);
-      if (tq_bad) hv = __builtin_nanf("");
-      hst[i][(u - us) * 16 + jj] = from_float<bf16s>(hv).bits;
+    finish(u, par, scl);
+  };
+  // WIDE: unit u, both sets
+  auto unit_wide = [&](int u, int par) {
+    const uint32_t rowc = unit_row(u);
+    float scl[2], d[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      q8v4 B[4];
+      q8_decode8(tq, lk, b0.q[t], B);
+      scl[t] = scale_cvt(b0.s[t], a.sdt, (rowc + j) * (uint32_t)a.Gh + grp);
+      q8v4 acc = {0, 0, 0, 0};
+#pragma unroll
+      for (int m = 0; m < 4; ++m) acc = mfma_i8(A[m], B[m], acc);
+      d[t] = (((float)acc[0] + (float)acc[1] * 0.0078125f) + (float)acc[2] * 0.00006103515625f) * inv;
+      if (!g1) d[t] *= scl[t];
     }
+#pragma unroll
+    for (int t = 0; t < 2; ++t) asm volatile("" : "+v"(scl[t]), "+v"(d[t]));  // done with b0 before it is reloaded
+    load_unit(u + 1, b0);
+    __builtin_amdgcn_sched_barrier(0);
+    if (dec1) {
+      float e[2] = {0.f, 0.f};
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        if (t == 1 && split) break;
+        q8v4 B[4];
+        q8_decode8(tq, lk, b1.q[t], B);
+        const float sc = g1 ? 1.f : scale_cvt(b1.s[t], a.sdt, (rowc + j) * (uint32_t)a.Gh + grp1);
+        q8v4 acc = {0, 0, 0, 0};
+#pragma unroll
+        for (int m = 0; m < 4; ++m) acc = mfma_i8(A1[WIDE ? m : 0], B[m], acc);
+        e[t] = (((float)acc[0] + (float)acc[1] * 0.0078125f) + (float)acc[2] * 0.00006103515625f) * inv1 * sc;
+        asm volatile("" : "+v"(e[t]));  // done with b1 before it is reloaded
+      }
+      d[0] += hi ? 0.f : e[0];
+      d[1] += split ? (hi ? e[0] : 0.f) : e[1];
+      load_set1(u + 1, b1);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if ((int)g < cur_nr) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t) gred[par][wv][t][g][j] = d[t];
+    }
+    finish(u, par, scl);
   };
   // u0 and every tile and SEG bound are even, so a segment starts on a pair and only the block's last unit
   // can be a pair's second past the end (loaded again, nothing stored)
-  for (int u = u0; u < u1; u += 2) {
+  for (int u = u0; u < u1; u += WIDE ? 1 : 2) {
     if (u == ue) {      // the next segment
       rt_lds_barrier();  // every h row of this one staged
       flush();
@@ -548,15 +634,23 @@ __global__ __launch_bounds__(1024) void k_moeq_gateup_tiles(MTArgs a, MTRoute p)
                 __builtin_amdgcn_readfirstlane(td->r[2]), __builtin_amdgcn_readfirstlane(td->r[3]));
         wait_vm_q<0>();  // nothing of the switch stays in flight: the units' waits count their own loads
         build_x();
-        build_a();
+        build_a(A);
       } else {
-        issue_a(td->r[j >> 2], td->r[g]);
-        build_a();
+        if constexpr (WIDE) {
+          issue_a(td->r[j >> 2], td->r[g], sl1, inv1);
+          build_a(A1);
+        }
+        issue_a(td->r[j >> 2], td->r[g], sl, inv);
+        build_a(A);
         wait_vm_q<0>();  // nothing of the switch stays in flight: the units' waits count their own loads
       }
     }
-    unit(u, b0, 0);
-    unit(u + 1, b1, 1);
+    if constexpr (WIDE) {
+      unit_wide(u, (u - u0) & 1);
+    } else {
+      unit(u, b0, 0);
+      unit(u + 1, b1, 1);
+    }
   }
   rt_lds_barrier();
   flush();
@@ -569,13 +663,18 @@ __global__ __launch_bounds__(1024) void k_moeq_gateup_tiles(MTArgs a, MTRoute p)
 // tile's routes (rows 2r, 2r + 1; rows past them zero), built in LDS by the
 // slice's first wave when the block enters a segment and read by both; route
 // r's dot is D rows 2r, 2r + 1. The partial sums are kept per slice and row
-// tile and summed over the slices in slice order.
+// tile and summed over the slices in slice order. THREE (hidden sizes beyond
+// 4096): three terms per route, rows 4r .. 4r + 2 as in gate/up, the same
+// MFMAs; h then keeps all but 2^-20 of its slice's max, below its bf16
+// rounding, as the fp32 mat-vecs these shapes used before kept it.
+template <bool THREE>
 __global__ __launch_bounds__(1024) void k_moeq_down_tiles(MTArgs a) {
+  constexpr int NT = THREE ? 3 : 2;  // terms per route
   constexpr int RT = 4;   // row tiles per unit
   constexpr int RW = 2;   // row tiles per wave
   constexpr int SEG = 48;  // units per segment (y staging capacity)
   __shared__ uint4 tqs[TQR_BYTES / 16];
-  __shared__ uint4 ash[8][2 * MT_TILE * 16];         // [slice][row * 16 + slot]
+  __shared__ uint4 ash[8][NT * MT_TILE * 16];        // [slice][(route * NT + term) * 16 + slot]
   __shared__ float s_inv[8][MT_TILE];
   __shared__ float red[2][8][RT][MT_TILE][16];       // [parity][slice][row-tile][route][row]
   __shared__ float yst[MT_TILE][SEG * 16 * RT];      // the segment's y rows
@@ -669,10 +768,11 @@ __global__ __launch_bounds__(1024) void k_moeq_down_tiles(MTArgs a) {
         const float mx = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
         float sc, inv4s;
         q8_scale(rt_wave_reduce(mx, true), sc, inv4s);
-        uint32_t tw[2];
-        q8_digits2(v, sc, tw);
-        aw[q8_aword((uint32_t)(2 * i), lane >> 1, lane & 1)] = tw[0];
-        aw[q8_aword((uint32_t)(2 * i + 1), lane >> 1, lane & 1)] = tw[1];
+        uint32_t tw[NT];
+        if constexpr (THREE) q8_terms<3>(v, sc, tw);
+        else q8_digits2(v, sc, tw);
+#pragma unroll
+        for (int n = 0; n < NT; ++n) aw[q8_aword((uint32_t)(NT * i + n), lane >> 1, lane & 1)] = tw[n];
         if (lane == 0) s_inv[sl][i] = inv4s;
       }
     }
@@ -683,15 +783,16 @@ __global__ __launch_bounds__(1024) void k_moeq_down_tiles(MTArgs a) {
       // reload from scratch waits for every code load in flight
       uint32_t g = lane >> 4;
       asm volatile("" : "+v"(g));
-      const q8v4* as = (const q8v4*)ash[sl] + (j & (2 * MT_TILE - 1)) * 16 + g * 4;
+      const uint32_t arow = THREE ? (j >> 2) * 3u + min(j & 3u, 2u) : j & (2 * MT_TILE - 1);
+      const q8v4* as = (const q8v4*)ash[sl] + arow * 16 + g * 4;
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
         const q8v4 v = as[m];
-        const bool z = (int)j >= 2 * cur_nr;  // rows past the tile's routes
+        const bool z = THREE ? (j & 3u) == 3u : (int)j >= 2 * cur_nr;  // rows of no term, or past the tile's routes
         A[m] = q8v4{z ? 0 : v[0], z ? 0 : v[1], z ? 0 : v[2], z ? 0 : v[3]};
       }
 #pragma unroll
-      for (int h2 = 0; h2 < 2; ++h2) inv[h2] = s_inv[sl][min(2 * (int)g + h2, MT_TILE - 1)];
+      for (int h2 = 0; h2 < 2; ++h2) inv[h2] = s_inv[sl][THREE ? (int)g : min(2 * (int)g + h2, MT_TILE - 1)];
     }
   };
   // the segment's staged y rows to their routes' rows
@@ -738,6 +839,13 @@ __global__ __launch_bounds__(1024) void k_moeq_down_tiles(MTArgs a) {
         q8v4 acc = {0, 0, 0, 0};
 #pragma unroll
         for (int m = 0; m < 4; ++m) acc = mfma_i8(A[m], B[rt][m], acc);
+        if constexpr (THREE) {  // route g: rows 4g .. 4g + 2 = lanes 16 g + j, registers 0 .. 2
+          if ((int)g < cur_nr) {
+            const float d = ((float)acc[0] + (float)acc[1] * 0.0078125f) + (float)acc[2] * 0.00006103515625f;
+            red[par][sl][hf * RW + rt][g][j] = d * inv[0] * scl[rt];
+          }
+          continue;
+        }
         // route r: rows 2r, 2r + 1 = lanes 16 (r / 2) + j, registers 2 (r % 2), 2 (r % 2) + 1
 #pragma unroll
         for (int h2 = 0; h2 < 2; ++h2) {
@@ -873,8 +981,11 @@ static int64_t mt_tiles_ub(int64_t T, int64_t k, int64_t E) {
   return std::min<int64_t>(R, (R + MT_TILE - 1) / MT_TILE + E);
 }
 
-bool moe_tiles_supported(int64_t T, int64_t E, int64_t H, int64_t I, int64_t k, int64_t group_h, int64_t group_i) {
-  return T >= 1 && T <= 256 && k >= 1 && k <= 16 && k <= E && E >= 1 && E <= 1024 && H % 256 == 0 && H <= 4096 &&
+constexpr int64_t MT_MAX_H = 4096, MT_WIDE_MAX_H = 8192;  // one K slice per gate/up wave; two (the WIDE kernel)
+
+bool moe_tiles_supported(int64_t T, int64_t E, int64_t H, int64_t I, int64_t k, int64_t group_h, int64_t group_i,
+                         int64_t max_h = MT_MAX_H) {
+  return T >= 1 && T <= 256 && k >= 1 && k <= 16 && k <= E && E >= 1 && E <= 1024 && H % 256 == 0 && H <= max_h &&
          I % 256 == 0 && I <= 2048 && group_h % 256 == 0 && group_i % 256 == 0 && (int64_t)E * I <= 0x7fffffffLL &&
          (int64_t)E * H <= 0x7fffffffLL && mt_tiles_per_block(mt_tiles_ub(T, k, E), I / 16) <= MT_TPB &&
          mt_tiles_per_block(mt_tiles_ub(T, k, E), H / 64) <= MT_TPB;
@@ -902,8 +1013,14 @@ extern "C" int keep_moe_tiles_supported(int64_t T, int64_t num_experts, int64_t 
   return moe_tiles_supported(T, num_experts, H, I, k, group_size_h, group_size_i) ? 1 : 0;
 }
 
-// The checks both few-token entry points make on the expert side.
-static int mt_check(const void* x, int x_dtype, int64_t T, int64_t H, int64_t I, int64_t k, int64_t num_experts,
+extern "C" int keep_moe_wide_supported(int64_t T, int64_t num_experts, int64_t H, int64_t I, int64_t k,
+                                       int64_t group_size_h, int64_t group_size_i) {
+  if (!::keep::dims_ok({T, num_experts, H, I, k, group_size_h, group_size_i})) return 0;
+  return moe_tiles_supported(T, num_experts, H, I, k, group_size_h, group_size_i, MT_WIDE_MAX_H) ? 1 : 0;
+}
+
+// The checks the few-token entry points make on the expert side.
+static int mt_check(int64_t max_h, const void* x, int x_dtype, int64_t T, int64_t H, int64_t I, int64_t k, int64_t num_experts,
                     const uint16_t* gate_codes, const void* gate_scales, const uint16_t* up_codes,
                     const void* up_scales, const uint16_t* down_codes, const void* down_scales, int scale_dtype,
                     int64_t group_size_h, int64_t group_size_i, const void* prepared, void* h_work, void* workspace,
@@ -912,9 +1029,9 @@ static int mt_check(const void* x, int x_dtype, int64_t T, int64_t H, int64_t I,
   KEEP_REQUIRE(dtype_ok(scale_dtype) && dtype_ok(out_dtype), "bad dtype enum");
   KEEP_REQUIRE(group_size_h > 0 && H % group_size_h == 0 && group_size_i > 0 && I % group_size_i == 0,
                "bad group sizes");
-  KEEP_REQUIRE(moe_tiles_supported(T, num_experts, H, I, k, group_size_h, group_size_i),
+  KEEP_REQUIRE(moe_tiles_supported(T, num_experts, H, I, k, group_size_h, group_size_i, max_h),
                "shape not served by the tiled MoE kernels (T <= 256, k <= 16, E <= 1024, H a multiple of 256 up "
-               "to 4096, I a multiple of 256 up to 2048, scale groups of 256-element multiples)");
+               "to %d, I a multiple of 256 up to 2048, scale groups of 256-element multiples)", (int)max_h);
   KEEP_REQUIRE(x && gate_codes && gate_scales && up_codes && up_scales && down_codes && down_scales && prepared &&
                    h_work && workspace && out,
                "null pointer argument");
@@ -952,11 +1069,13 @@ static MTArgs mt_args(int64_t H, int64_t I, int64_t k, int64_t num_experts, cons
   return a;
 }
 
-// The gate/up launch: unrouted (rp null: x terms and plan in the workspace) or routing its tokens itself
+// The gate/up launch: unrouted (rp null, always so beyond 16 K slices: x terms and plan in the workspace) or routing its tokens itself
 // with `per` (<= 8) logits per router lane.
 template <bool XBF>
 static void mt_launch_gateup(const MTArgs& a, const MTRoute* rp, int per, unsigned g1, hipStream_t s) {
-  if (!rp) {
+  if (a.S > 16) {
+    hipLaunchKernelGGL((k_moeq_gateup_tiles<XBF, 0, true>), dim3(g1), dim3(1024), 0, s, a, MTRoute{});
+  } else if (!rp) {
     hipLaunchKernelGGL((k_moeq_gateup_tiles<XBF, 0>), dim3(g1), dim3(1024), 0, s, a, MTRoute{});
   } else if (per <= 2) {
     hipLaunchKernelGGL((k_moeq_gateup_tiles<XBF, 2>), dim3(g1), dim3(1024), 0, s, a, *rp);
@@ -979,13 +1098,14 @@ static void mt_tail(const MTArgs& a, int x_dtype, int64_t T, int64_t H, int64_t 
   const unsigned g2 = (unsigned)mt_grid(tiles_ub, H / 64);
   if (x_dtype == KEEP_BF16) mt_launch_gateup<true>(a, rp, per, g1, s);
   else mt_launch_gateup<false>(a, rp, per, g1, s);
-  hipLaunchKernelGGL(k_moeq_down_tiles, dim3(g2), dim3(1024), 0, s, a);
+  if (H > MT_MAX_H) hipLaunchKernelGGL((k_moeq_down_tiles<true>), dim3(g2), dim3(1024), 0, s, a);
+  else hipLaunchKernelGGL((k_moeq_down_tiles<false>), dim3(g2), dim3(1024), 0, s, a);
   const int64_t n = T * H;
   hipLaunchKernelGGL(k_moe_combine, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a.y, idx, w, (int)T, (int)k,
                      (int)num_experts, (int)H, a.tq_bad, out, out_dtype);
 }
 
-extern "C" int keep_moe_tiles(const void* x, int x_dtype, int64_t T, int64_t H, int64_t I, const int32_t* idx,
+static int mt_run(int64_t max_h, const void* x, int x_dtype, int64_t T, int64_t H, int64_t I, const int32_t* idx,
                               const float* w, int64_t k, int64_t num_experts, const uint16_t* gate_codes,
                               const void* gate_scales, const uint16_t* up_codes, const void* up_scales,
                               const uint16_t* down_codes, const void* down_scales, int scale_dtype,
@@ -993,7 +1113,7 @@ extern "C" int keep_moe_tiles(const void* x, int x_dtype, int64_t T, int64_t H, 
                               void* h_work, void* workspace, int64_t workspace_bytes, void* out, int out_dtype,
                               void* stream) {
   KEEP_REQUIRE_DIMS(T, H, I, k, num_experts, group_size_h, group_size_i);
-  const int chk = mt_check(x, x_dtype, T, H, I, k, num_experts, gate_codes, gate_scales, up_codes, up_scales,
+  const int chk = mt_check(max_h, x, x_dtype, T, H, I, k, num_experts, gate_codes, gate_scales, up_codes, up_scales,
                            down_codes, down_scales, scale_dtype, group_size_h, group_size_i, prepared, h_work,
                            workspace, workspace_bytes, out, out_dtype);
   if (chk != KEEP_OK) return chk;
@@ -1004,12 +1124,13 @@ extern "C" int keep_moe_tiles(const void* x, int x_dtype, int64_t T, int64_t H, 
   const MTArgs a = mt_args(H, I, k, num_experts, gate_codes, gate_scales, up_codes, up_scales, down_codes,
                            down_scales, scale_dtype, group_size_h, group_size_i, prepared, swiglu_limit, h_work, ws, L);
   const int64_t R = T * k;
-  const dim3 xb((unsigned)(64 * (H / 256)));
+  const int64_t S = H / 256;
+  const dim3 xg((unsigned)T, (unsigned)((S + 15) / 16)), xb((unsigned)(64 * std::min<int64_t>(S, 16)));
   if (x_dtype == KEEP_BF16)
-    hipLaunchKernelGGL((k_q8_xterms<true>), dim3((unsigned)T), xb, 0, s, x, (int)H, (uint4*)(ws + L.xt),
+    hipLaunchKernelGGL((k_q8_xterms<true>), xg, xb, 0, s, x, (int)H, (uint4*)(ws + L.xt),
                        (float*)(ws + L.xinv));
   else
-    hipLaunchKernelGGL((k_q8_xterms<false>), dim3((unsigned)T), xb, 0, s, x, (int)H, (uint4*)(ws + L.xt),
+    hipLaunchKernelGGL((k_q8_xterms<false>), xg, xb, 0, s, x, (int)H, (uint4*)(ws + L.xt),
                        (float*)(ws + L.xinv));
   const int rc = keep_route_plan(idx, R, num_experts, MT_TILE, (int32_t*)(ws + L.order), (int32_t*)(ws + L.inverse),
                                  (int32_t*)(ws + L.counts), (int32_t*)(ws + L.offsets), (int32_t*)(ws + L.te),
@@ -1017,7 +1138,7 @@ extern "C" int keep_moe_tiles(const void* x, int x_dtype, int64_t T, int64_t H, 
                                  stream);
   if (rc != KEEP_OK) return rc;
   mt_tail(a, x_dtype, T, H, I, k, num_experts, idx, w, L, out, out_dtype, s);
-  return launch_status("keep_moe_tiles");
+  return launch_status("few-token layer");
 }
 
 // Router declaration (router.hip).
@@ -1026,7 +1147,7 @@ extern "C" int keep_router_dual_topk(const float* logits, int64_t T, int64_t E, 
                                      float tau, const int32_t* slot_map, int64_t num_slots, int32_t* idx, float* w,
                                      int32_t* want, float* want_score, uint8_t* admit, void* stream);
 
-extern "C" int keep_moe_tiles_layer(const float* logits, const float* bias_served, const float* bias_demand,
+static int mt_run_layer(int64_t max_h, const float* logits, const float* bias_served, const float* bias_demand,
                                     int score_func, int renormalize, float route_scale, float tau,
                                     const int32_t* slot_map, int64_t num_slots, int64_t num_experts, int64_t k,
                                     const void* x, int x_dtype, int64_t T, int64_t H, int64_t I,
@@ -1042,7 +1163,7 @@ extern "C" int keep_moe_tiles_layer(const float* logits, const float* bias_serve
   KEEP_REQUIRE(score_func >= 0 && score_func <= 2, "bad score_func %d", score_func);
   KEEP_REQUIRE(!slot_map || (num_slots >= 1 && num_slots <= 1024), "num_slots must be in 1..1024");
   const int64_t S = slot_map ? num_slots : num_experts;  // pool rows
-  const int chk = mt_check(x, x_dtype, T, H, I, k, S, gate_codes, gate_scales, up_codes, up_scales, down_codes,
+  const int chk = mt_check(max_h, x, x_dtype, T, H, I, k, S, gate_codes, gate_scales, up_codes, up_scales, down_codes,
                            down_scales, scale_dtype, group_size_h, group_size_i, prepared, h_work, workspace,
                            workspace_bytes, out, out_dtype);
   if (chk != KEEP_OK) return chk;
@@ -1053,7 +1174,7 @@ extern "C" int keep_moe_tiles_layer(const float* logits, const float* bias_serve
                                          route_scale, tau, slot_map, num_slots, idx, w, want, want_score, admit,
                                          stream);
     if (rc != KEEP_OK) return rc;
-    return keep_moe_tiles(x, x_dtype, T, H, I, idx, w, k, S, gate_codes, gate_scales, up_codes, up_scales,
+    return mt_run(max_h, x, x_dtype, T, H, I, idx, w, k, S, gate_codes, gate_scales, up_codes, up_scales,
                           down_codes, down_scales, scale_dtype, group_size_h, group_size_i, prepared, swiglu_limit,
                           h_work, workspace, workspace_bytes, out, out_dtype, stream);
   }
@@ -1065,7 +1186,7 @@ extern "C" int keep_moe_tiles_layer(const float* logits, const float* bias_serve
   const int per = (int)((num_experts + 63) / 64);
   // up to 128 routes and 512 experts the gate/up kernel routes and plans in every block (no prologue launch;
   // a router lane holding 16 logits would spill inside it); every block of it routes a token fully
-  if (T * k <= PLAN_SMALL_R && per <= 8 && T <= mt_grid(mt_tiles_ub(T, k, S), I / 16)) {
+  if (H <= 4096 && T * k <= PLAN_SMALL_R && per <= 8 && T <= mt_grid(mt_tiles_ub(T, k, S), I / 16)) {
     MTRoute rp{};
     rp.x = x; rp.logits = logits; rp.bias_s = bias_served; rp.bias_d = bias_demand; rp.func = score_func;
     rp.renorm = renormalize; rp.route_scale = route_scale; rp.tau = tau; rp.slot_map = slot_map;
@@ -1076,7 +1197,7 @@ extern "C" int keep_moe_tiles_layer(const float* logits, const float* bias_serve
     rp.to = (int32_t*)(ws + L.to); rp.tc = (int32_t*)(ws + L.tc); rp.nt = (int32_t*)(ws + L.nt);
     rp.max_tiles = (int)L.max_tiles;
     mt_tail(a, x_dtype, T, H, I, k, S, idx, w, L, out, out_dtype, s, &rp, per);
-    return launch_status("keep_moe_tiles_layer");
+    return launch_status("few-token layer");
   }
   MTPro p{};
   p.x = x; p.H = (int)H; p.xt = (uint4*)(ws + L.xt); p.xinv = (float*)(ws + L.xinv);
@@ -1101,5 +1222,62 @@ extern "C" int keep_moe_tiles_layer(const float* logits, const float* bias_serve
   else MT_PRO(16);
 #undef MT_PRO
   mt_tail(a, x_dtype, T, H, I, k, S, idx, w, L, out, out_dtype, s);
-  return launch_status("keep_moe_tiles_layer");
+  return launch_status("few-token layer");
+}
+
+extern "C" int keep_moe_tiles(const void* x, int x_dtype, int64_t T, int64_t H, int64_t I, const int32_t* idx,
+                              const float* w, int64_t k, int64_t num_experts, const uint16_t* gate_codes,
+                              const void* gate_scales, const uint16_t* up_codes, const void* up_scales,
+                              const uint16_t* down_codes, const void* down_scales, int scale_dtype,
+                              int64_t group_size_h, int64_t group_size_i, const void* prepared, float swiglu_limit,
+                              void* h_work, void* workspace, int64_t workspace_bytes, void* out, int out_dtype,
+                              void* stream) {
+  return mt_run(MT_MAX_H, x, x_dtype, T, H, I, idx, w, k, num_experts, gate_codes, gate_scales, up_codes, up_scales,
+      down_codes, down_scales, scale_dtype, group_size_h, group_size_i, prepared, swiglu_limit,
+      h_work, workspace, workspace_bytes, out, out_dtype, stream);
+}
+
+extern "C" int keep_moe_wide(const void* x, int x_dtype, int64_t T, int64_t H, int64_t I, const int32_t* idx,
+                              const float* w, int64_t k, int64_t num_experts, const uint16_t* gate_codes,
+                              const void* gate_scales, const uint16_t* up_codes, const void* up_scales,
+                              const uint16_t* down_codes, const void* down_scales, int scale_dtype,
+                              int64_t group_size_h, int64_t group_size_i, const void* prepared, float swiglu_limit,
+                              void* h_work, void* workspace, int64_t workspace_bytes, void* out, int out_dtype,
+                              void* stream) {
+  return mt_run(MT_WIDE_MAX_H, x, x_dtype, T, H, I, idx, w, k, num_experts, gate_codes, gate_scales, up_codes,
+      up_scales, down_codes, down_scales, scale_dtype, group_size_h, group_size_i, prepared,
+      swiglu_limit, h_work, workspace, workspace_bytes, out, out_dtype, stream);
+}
+
+extern "C" int keep_moe_tiles_layer(const float* logits, const float* bias_served, const float* bias_demand,
+                                    int score_func, int renormalize, float route_scale, float tau,
+                                    const int32_t* slot_map, int64_t num_slots, int64_t num_experts, int64_t k,
+                                    const void* x, int x_dtype, int64_t T, int64_t H, int64_t I,
+                                    const uint16_t* gate_codes, const void* gate_scales, const uint16_t* up_codes,
+                                    const void* up_scales, const uint16_t* down_codes, const void* down_scales,
+                                    int scale_dtype, int64_t group_size_h, int64_t group_size_i,
+                                    const void* prepared, float swiglu_limit, int32_t* idx, float* w, int32_t* want,
+                                    float* want_score, uint8_t* admit, void* h_work, void* workspace,
+                                    int64_t workspace_bytes, void* out, int out_dtype, void* stream) {
+  return mt_run_layer(MT_MAX_H, logits, bias_served, bias_demand, score_func, renormalize, route_scale, tau, slot_map,
+      num_slots, num_experts, k, x, x_dtype, T, H, I, gate_codes, gate_scales, up_codes, up_scales,
+      down_codes, down_scales, scale_dtype, group_size_h, group_size_i, prepared, swiglu_limit, idx,
+      w, want, want_score, admit, h_work, workspace, workspace_bytes, out, out_dtype, stream);
+}
+
+extern "C" int keep_moe_wide_layer(const float* logits, const float* bias_served, const float* bias_demand,
+                                    int score_func, int renormalize, float route_scale, float tau,
+                                    const int32_t* slot_map, int64_t num_slots, int64_t num_experts, int64_t k,
+                                    const void* x, int x_dtype, int64_t T, int64_t H, int64_t I,
+                                    const uint16_t* gate_codes, const void* gate_scales, const uint16_t* up_codes,
+                                    const void* up_scales, const uint16_t* down_codes, const void* down_scales,
+                                    int scale_dtype, int64_t group_size_h, int64_t group_size_i,
+                                    const void* prepared, float swiglu_limit, int32_t* idx, float* w, int32_t* want,
+                                    float* want_score, uint8_t* admit, void* h_work, void* workspace,
+                                    int64_t workspace_bytes, void* out, int out_dtype, void* stream) {
+  return mt_run_layer(MT_WIDE_MAX_H, logits, bias_served, bias_demand, score_func, renormalize, route_scale, tau,
+      slot_map, num_slots, num_experts, k, x, x_dtype, T, H, I, gate_codes, gate_scales, up_codes,
+      up_scales, down_codes, down_scales, scale_dtype, group_size_h, group_size_i, prepared,
+      swiglu_limit, idx, w, want, want_score, admit, h_work, workspace, workspace_bytes, out,
+      out_dtype, stream);
 }

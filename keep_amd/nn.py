@@ -223,8 +223,7 @@ class QuantizedVQSwitchLinear:
         q = quantize_weight_rtn(w.reshape(num_experts * out_dim, in_dim), group_size=group_size, code_bits=code_bits)
         return cls(input_dims=in_dim, output_dims=out_dim, num_experts=num_experts,
                    codes=q.codes.reshape(num_experts, out_dim, in_dim // CODEWORD_DIM),
-                   scales=q.scales.reshape(num_experts, out_dim, in_dim // q.group_size),
-                   codebook=torch.from_numpy(q.codebook.view(np.int32)).to(device), bias=bias,
+                   scales=q.scales.reshape(num_experts, out_dim, in_dim // q.group_size), bias=bias,
                    group_size=q.group_size, code_bits=q.code_bits, use_gather_vqmm=use_gather_vqmm,
                    route_strategy=route_strategy, gather_codebook_duplication=gather_codebook_duplication,
                    rht_signs=None if rht_signs is None else torch.as_tensor(rht_signs).to(device),
@@ -581,10 +580,11 @@ def moe_decode(x: torch.Tensor, idx: torch.Tensor, weight: torch.Tensor, gate, u
     w32 = weight.to(torch.float32).contiguous()
     prep = ops.prepared_table(cb) if prepared else None
     gh, gi = H // gs.shape[-1], I // ds.shape[-1]
-    if prep is not None and moe_tiles_supported(T, E, H, I, k, gh, gi):
+    entry = _tiles_entry(T, E, H, I, k, gh, gi, cb, (gc, uc, dc), (gs, us, ds)) if prep is not None else None
+    if entry is not None:
         ws = torch.empty(int(_lib.load().keep_moe_tiles_workspace_bytes(T, k, E, H)), dtype=torch.uint8,
                          device=device)
-        _lib.call("keep_moe_tiles", x.data_ptr(), ops._DT[x.dtype], T, H, I, idx32.data_ptr(), w32.data_ptr(), k, E,
+        _lib.call(entry, x.data_ptr(), ops._DT[x.dtype], T, H, I, idx32.data_ptr(), w32.data_ptr(), k, E,
                   gc.data_ptr(), gs.data_ptr(), uc.data_ptr(), us.data_ptr(), dc.data_ptr(), ds.data_ptr(),
                   ops._DT[gs.dtype], gh, gi, prep.data_ptr(), float(limit), h_work.data_ptr(), ws.data_ptr(),
                   ws.numel(), out.data_ptr(), ops._DT[od], ops._stream(device))
@@ -594,6 +594,20 @@ def moe_decode(x: torch.Tensor, idx: torch.Tensor, weight: torch.Tensor, gate, u
               ops._DT[gs.dtype], H // gs.shape[-1], I // ds.shape[-1], cb.data_ptr(), ops._ptr(prep),
               float(limit), h_work.data_ptr(), out.data_ptr(), ops._DT[od], ops._stream(device))
     return out
+
+
+def _tiles_entry(T: int, E: int, H: int, I: int, k: int, gh: int, gi: int, cb: torch.Tensor, codes, scales):
+    """The few-token entry point that serves a shape, or None. Hidden sizes beyond 4096 take it on the default
+    table and on aligned pools only: the matrix-core decode needs odd half-units and loads 16 bytes of codes and
+    aligned words of scales, the packed-table kernels take any table and narrower loads."""
+
+    if moe_tiles_supported(T, E, H, I, k, gh, gi):
+        return "keep_moe_tiles"
+    if (H > 4096 and _lib.load().keep_moe_wide_supported(T, E, H, I, k, gh, gi)
+            and cb is ops._default_codebook(16, cb.device)
+            and not any(t.data_ptr() % 16 for t in codes) and not any(t.data_ptr() % 4 for t in scales)):
+        return "keep_moe_wide"
+    return None
 
 
 def moe_tiles_layer(x: torch.Tensor, logits: torch.Tensor, gate, up, down, *, k: int, bias_served=None,
@@ -609,6 +623,12 @@ def moe_tiles_layer(x: torch.Tensor, logits: torch.Tensor, gate, up, down, *, k:
     ``x [T, H]`` (fp16/bf16), ``logits [T, E]``; ``slot_map`` as
     in ``moe_layer``. Returns ``(out [T, H], RouterOutput)``; float32 by default."""
 
+    return _tiles_layer("keep_moe_tiles_layer", x, logits, gate, up, down, k, bias_served, bias_demand, score_func,
+                        renormalize, route_scale, tau, limit, codebook, out_dtype, slot_map, h_work)
+
+
+def _tiles_layer(entry: str, x, logits, gate, up, down, k, bias_served, bias_demand, score_func, renormalize,
+                 route_scale, tau, limit, codebook, out_dtype, slot_map, h_work=None):
     device = x.device
     if x.dtype not in (torch.float16, torch.bfloat16):
         raise ValueError("moe_tiles_layer needs float16 or bfloat16 activations")
@@ -650,7 +670,7 @@ def moe_tiles_layer(x: torch.Tensor, logits: torch.Tensor, gate, up, down, *, k:
     prep = ops.prepared_table(cb)
     gh, gi = H // gs.shape[-1], I // ds.shape[-1]
     ws = torch.empty(int(_lib.load().keep_moe_tiles_workspace_bytes(T, k, S, H)), dtype=torch.uint8, device=device)
-    _lib.call("keep_moe_tiles_layer", z.data_ptr(), ops._ptr(bs), ops._ptr(bd), _lib.SCORE_FUNCS[score_func],
+    _lib.call(entry, z.data_ptr(), ops._ptr(bs), ops._ptr(bd), _lib.SCORE_FUNCS[score_func],
               int(bool(renormalize)), float(route_scale), float(tau), ops._ptr(sm), ns, E, k, x.data_ptr(),
               ops._DT[x.dtype], T, H, I, gc.data_ptr(), gs.data_ptr(), uc.data_ptr(), us.data_ptr(), dc.data_ptr(),
               ds.data_ptr(), ops._DT[gs.dtype], gh, gi, prep.data_ptr(), float(limit), r.idx.data_ptr(),
@@ -929,24 +949,29 @@ class RoutedVQMoE:
                 moe_layer_supported(g.num_experts, g.input_dims, g.output_dims, self.top_k,
                                     g.input_dims // g.scales.shape[-1], d.input_dims // d.scales.shape[-1]))
 
-    def _tiles_layer_path(self, x: torch.Tensor) -> bool:
-        g, d = self.glu.gate_proj, self.glu.down_proj
+    def _tiles_layer_path(self, x: torch.Tensor, logits: torch.Tensor) -> str | None:
+        """The few-token entry point that takes this call from its logits, if any."""
+        g, u, d = self.glu.gate_proj, self.glu.up_proj, self.glu.down_proj
         T = x.shape[0]
-        return (2 <= T <= self.decode_max_tokens and x.dtype in (torch.float16, torch.bfloat16) and
-                self.glu._all_e8p() and self.glu.hot_tier is None and self.top_k <= 16 and
-                moe_tiles_supported(T, g.num_experts, g.input_dims, g.output_dims, self.top_k,
-                                    g.input_dims // g.scales.shape[-1], d.input_dims // d.scales.shape[-1]))
+        if not (2 <= T <= self.decode_max_tokens and x.dtype in (torch.float16, torch.bfloat16) and
+                self.glu._all_e8p() and self.glu.hot_tier is None and self.top_k <= 16):
+            return None
+        entry = _tiles_entry(T, g.num_experts, g.input_dims, g.output_dims, self.top_k,
+                             g.input_dims // g.scales.shape[-1], d.input_dims // d.scales.shape[-1], g.codebook,
+                             (g.codes, u.codes, d.codes), (g.scales, u.scales, d.scales))
+        if entry == "keep_moe_wide" and self.slot_map is None and logits.shape[-1] != g.num_experts:
+            return None  # fewer logits than pool rows: routed apart
+        return None if entry is None else entry + "_layer"
 
     def __call__(self, x: torch.Tensor, logits: torch.Tensor, *, residual: torch.Tensor | None = None):
         extra = self.shared_experts is not None or residual is not None
         od = torch.float32 if extra else self.out_dtype
-        if self._tiles_layer_path(x):
+        entry = self._tiles_layer_path(x, logits)
+        if entry is not None:
             g, u, d = self.glu.gate_proj, self.glu.up_proj, self.glu.down_proj
-            out, r = moe_tiles_layer(x, logits, (g.codes, g.scales), (u.codes, u.scales), (d.codes, d.scales),
-                                     k=self.top_k, bias_served=self.bias_served, bias_demand=self.bias_demand,
-                                     score_func=self.score_func, renormalize=self.renormalize,
-                                     route_scale=self.route_scale, tau=self.tau, limit=self.limit,
-                                     codebook=g.codebook, out_dtype=od, slot_map=self.slot_map)
+            out, r = _tiles_layer(entry, x, logits, (g.codes, g.scales), (u.codes, u.scales), (d.codes, d.scales),
+                                  self.top_k, self.bias_served, self.bias_demand, self.score_func, self.renormalize,
+                                  self.route_scale, self.tau, self.limit, g.codebook, od, self.slot_map)
         elif self._layer_path(x):
             g, u, d = self.glu.gate_proj, self.glu.up_proj, self.glu.down_proj
             one = self.one_launch and _one_launch_ok(x.device, logits.shape[-1], g.input_dims, g.output_dims,

@@ -71,6 +71,9 @@ int main() {
   PROBE(keep_moe_tiles_supported);
   PROBE(keep_moe_tiles);
   PROBE(keep_moe_tiles_layer);
+  PROBE(keep_moe_wide_supported);
+  PROBE(keep_moe_wide);
+  PROBE(keep_moe_wide_layer);
   PROBE(keep_vq_grouped_gemm_q8_workspace_bytes);
   PROBE(keep_vq_grouped_gemm_q8);
   PROBE(keep_vq_grouped_gemm_e8);

@@ -285,3 +285,55 @@ def test_tiles_layer_near_ties_fall_back_to_exact_keys(dev, small_pool):
     out, r2 = keep_amd.moe_tiles_layer(x, z, *pool, k=k)
     assert torch.equal(r2.idx, r.idx) and torch.equal(r2.weight, r.weight)
     assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("xdt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("T, H, I, E, k, gh", [(1, 4352, 256, 6, 2, 256), (5, 5120, 512, 12, 3, 5120),
+                                              (30, 6400, 256, 5, 4, 256), (40, 8192, 256, 9, 2, 4096),
+                                              (9, 7168, 256, 300, 8, 512)])
+def test_wide_hidden_sizes_vs_oracle(dev, xdt, T, H, I, E, k, gh):
+    """17 to 32 K slices: the second set of one slice (4352), of at most 8 (one
+    projection per wave), of 9 and of 16; per-row and grouped scales; from the
+    logits at T <= 32 and beyond, blocks over one and several tiles. The
+    routing equals the router's; the layer is within the path's bound of the
+    oracle and, on the stored terms, as close to it as the packed-table kernels."""
+    gate = synth.projection_np(E, I, H, group_size=gh, seed=81)
+    up = synth.projection_np(E, I, H, group_size=gh, seed=82)
+    down = synth.projection_np(E, H, I, seed=83)
+    x = torch.from_numpy(np.random.default_rng(84).standard_normal((T, H)).astype(np.float32)).to(dev).to(xdt)
+    z = synth.router_logits(T, E, seed=85, device=dev)
+    tt = lambda p: (_t(p[0], dev), _t(p[1], dev))  # noqa: E731
+    lin = lambda p, K, N: keep_amd.QuantizedVQSwitchLinear(  # noqa: E731
+        input_dims=K, output_dims=N, num_experts=E, codes=tt(p)[0], scales=tt(p)[1], group_size=K // p[1].shape[-1],
+        code_bits=16)
+    moe = keep_amd.RoutedVQMoE(keep_amd.QuantizedVQSwitchGLU(gate_proj=lin(gate, H, I), up_proj=lin(up, H, I),
+                                                             down_proj=lin(down, I, H)), top_k=k)
+    out, r = moe(x, z)
+    ref = keep_amd.router_dual_topk(z, k)
+    for a, b in zip(r, ref):
+        assert torch.equal(a, b)
+    same = keep_amd.moe_decode(x, r.idx, r.weight, tt(gate), tt(up), tt(down))
+    assert torch.equal(out, same)
+    want = ops.moe_layer(x.float().cpu().numpy(), r.idx.cpu().numpy(), r.weight.cpu().numpy(), gate, up, down,
+                         h_round="bfloat16")
+    _check(out, want)
+    packed = keep_amd.moe_decode(x, r.idx, r.weight, tt(gate), tt(up), tt(down), prepared=False)
+    exact = ops.moe_layer(x.float().cpu().numpy(), r.idx.cpu().numpy(), r.weight.cpu().numpy(), gate, up, down)
+    err = [np.linalg.norm(o.float().cpu().numpy() - exact) / np.linalg.norm(exact) for o in (out, packed)]
+    assert err[0] <= 1.02 * err[1], f"further from the unrounded layer: {err}"  # the flips of h's bf16 ties
+
+
+def test_wide_hidden_custom_table_stays_on_packed_kernels(dev):
+    """A table with even half-units has no int8 form: beyond 4096 hidden values
+    the layer still takes it, through the packed-table kernels."""
+    E, H, I, k, T = 4, 4608, 256, 2, 3
+    table = keep_amd.ops.e8p_packed_abs_grid()
+    table = (table & ~np.uint32(0xF)) | np.uint32(0xA)  # nibble 0: value 2 / 2
+    cb = torch.from_numpy(table.view(np.int32)).to(dev)
+    pools = [synth.projection(E, n, K, seed=90 + i, device=dev) for i, (n, K) in enumerate([(I, H), (I, H), (H, I)])]
+    pairs = [(p.codes, p.scales) for p in pools]
+    x = synth.rht_activations(T, 4096, seed=94, device=dev).repeat(1, 2)[:, :H].contiguous()
+    r = keep_amd.router_dual_topk(synth.router_logits(T, E, seed=95, device=dev), k)
+    a = keep_amd.moe_decode(x, r.idx, r.weight, *pairs, codebook=cb)
+    assert torch.isfinite(a).all()
+    assert torch.equal(a, keep_amd.moe_decode(x, r.idx, r.weight, *pairs, codebook=cb, prepared=False))
