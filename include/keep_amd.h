@@ -470,6 +470,25 @@ int keep_vq_grouped_gemm_e8(const void* x, int x_dtype, int64_t x_rows, const in
                             const int32_t* tile_count, int64_t n_tiles, int64_t routes, int64_t num_experts,
                             int64_t N, int64_t K, int64_t group_size, void* out, int out_dtype, void* stream);
 
+/* Routed mat-vecs on the matrix cores for few rows: out[r, :] = W[rhs[r]] .
+ * x[lhs ? lhs[r] : r / x_div, :] for `routes` routes (rhs NULL with
+ * num_experts = 1: one matrix against rows 0 .. routes - 1), in route order; a
+ * route with an expert or row out of range gets NaN. Codes 8-bit E8 (fp16 or
+ * bf16 rows; `tables` the packed table, uint32[256]) or E8P (fp16 rows; `tables`
+ * = keep_e8p_prepare's buffer), K and group_size multiples of 512 / 256, K at most 8192 / 4096
+ * (keep_vq_rows_supported). grouped: the routes of one expert share its code
+ * loads, in tiles of up to 16; up to 128 routes are grouped in the kernel,
+ * beyond that a route plan of tiles of 16 (keep_route_plan) is passed. Routed
+ * results do not depend on the grouping, bit for bit. Replaces
+ * gather_vqmm_verify_rows (src/ramp/ops/vq_switch.py:286-377) and the direct
+ * routes of gather_vqmm. */
+int keep_vq_rows_supported(int x_dtype, int code_bits, int64_t K, int64_t group_size);
+int keep_vq_rows(const void* x, int x_dtype, int64_t x_rows, const void* codes, int code_bits, const void* scales,
+                 int scale_dtype, const void* tables, const int32_t* rhs, const int32_t* lhs, int64_t routes,
+                 int64_t x_div, int grouped, const int32_t* order, const int32_t* tile_expert,
+                 const int32_t* tile_offset, const int32_t* tile_count, int64_t n_tiles, int64_t num_experts,
+                 int64_t N, int64_t K, int64_t group_size, void* out, int out_dtype, void* stream);
+
 /* One matrix against many rows on the matrix cores: out[m, :] = W . x[m, :]
  * for x fp16 or bf16 [rows, K], codes [N, K/8] (code_bits 16: E8P, `tables` =
  * keep_e8p_prepare's buffer; 8: E8, `tables` = the packed 8-bit E8 table),

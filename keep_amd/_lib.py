@@ -61,6 +61,9 @@ _SIGS = {
                                 c_int64, c_int64, c_int64, c_int64, _P, c_int64, _P, c_int, _P],
     "keep_vq_grouped_gemm_e8": [_P, c_int, c_int64, _P, _P, _P, _P, c_int, _P, _P, _P, _P, c_int64, c_int64, c_int64,
                                 c_int64, c_int64, c_int64, _P, c_int, _P],
+    "keep_vq_rows_supported": [c_int, c_int, c_int64, c_int64],
+    "keep_vq_rows": [_P, c_int, c_int64, _P, c_int, _P, c_int, _P, _P, _P, c_int64, c_int64, c_int, _P, _P, _P, _P,
+                     c_int64, c_int64, c_int64, c_int64, c_int64, _P, c_int, _P],
     "keep_vq_gemm": [_P, c_int, c_int64, _P, c_int, _P, c_int, _P, c_int64, c_int64, c_int64, _P, c_int64, _P, c_int,
                      _P],
     "keep_vq_grouped_swiglu_q8": [_P, c_int, c_int64, _P, _P, _P, _P, _P, c_int, _P, _P, _P, _P, c_int64, c_int64,

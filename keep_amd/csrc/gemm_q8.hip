@@ -58,8 +58,8 @@ constexpr int GQ_KB = 128;              // k per K block
 constexpr int GQ_ROW = 2 * GQ_KB + 16;  // LDS bytes per A row: rows 4 banks apart (no conflicts)
 constexpr int GQ_XCDS = 8;
 
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef _Float16 h2v __attribute__((ext_vector_type(2)));
+typedef q8h8 h8;
+typedef q8h2 h2v;
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 // One 32x32x16 MFMA of 16-bit operands (BF: the bits are bf16's, else fp16's).
@@ -70,26 +70,6 @@ __device__ __forceinline__ f32x16 mfma32(h8 a, h8 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(b8, a), __builtin_bit_cast(b8, b), c, 0, 0, 0);
   else
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-}
-
-// Bytes q + 128 (mod 256) of eight integer weights q -> the fp16 values q.
-__device__ __forceinline__ h8 gq_f16_of_bytes(uint2 b) {
-  const uint32_t k = 0x64646464u;
-  const uint32_t d[4] = {__builtin_amdgcn_perm(k, b.x, 0x04010400u), __builtin_amdgcn_perm(k, b.x, 0x04030402u),
-                         __builtin_amdgcn_perm(k, b.y, 0x04010400u), __builtin_amdgcn_perm(k, b.y, 0x04030402u)};
-  h8 r;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const h2v v = __builtin_bit_cast(h2v, d[i]) - h2v{(_Float16)1152.f, (_Float16)1152.f};
-    r[2 * i] = v[0];
-    r[2 * i + 1] = v[1];
-  }
-  return r;
-}
-
-// Natural-order bytes of a packed-nibble-order pair (dims 0, 2, 4, 6 | 1, 3, 5, 7).
-__device__ __forceinline__ uint2 gq_natural(uint2 v) {
-  return make_uint2(__builtin_amdgcn_perm(v.y, v.x, 0x05010400u), __builtin_amdgcn_perm(v.y, v.x, 0x07030602u));
 }
 
 // ------------------------------------------------------------------ row scales
@@ -230,7 +210,7 @@ __global__ __launch_bounds__(GQ_THREADS) void k_gemm_e8(GQArgs a) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) row[i] = v;
     } else {  // row e: sixteen copies of (T'[e], M[e]), T' = T ^ 0x80 per byte, natural dim order
-      const uint2 t = gq_natural(((const uint2*)a.tq)[e]), m = gq_natural(((const uint2*)a.tq)[256 + e]);
+      const uint2 t = q8_natural(((const uint2*)a.tq)[e]), m = q8_natural(((const uint2*)a.tq)[256 + e]);
       const uint4 v = make_uint4(t.x ^ 0x80808080u, t.y ^ 0x80808080u, m.x, m.y);
       uint4* row = tqs + e * 16 + (tid & 1) * 8;
 #pragma unroll
@@ -268,7 +248,7 @@ __global__ __launch_bounds__(GQ_THREADS) void k_gemm_e8(GQArgs a) {
   };
   auto cvt = [&](const uint4& r) -> h8 {
     if constexpr (E8) return __builtin_bit_cast(h8, r);
-    else return gq_f16_of_bytes(make_uint2(r.x ^ r.z, r.y ^ r.w));
+    else return q8_f16_of_bytes(make_uint2(r.x ^ r.z, r.y ^ r.w));
   };
   // HOT: the residual codeword s of this lane's 8 code bytes -> its 8 bytes q + 128
   auto look_r = [&](const uint2& r, int s) -> uint2 {
@@ -458,7 +438,7 @@ __global__ __launch_bounds__(GQ_THREADS) void k_gemm_e8(GQArgs a) {
         Bc[jn] = cvt(look(bb[0].q[jn], 0));
         Lc[jn] = look(bb[0].q[jn], 1);
         if constexpr (HT) {
-          Rc[jn] = gq_f16_of_bytes(look_r(bb[0].r[jn], 0));
+          Rc[jn] = q8_f16_of_bytes(look_r(bb[0].r[jn], 0));
           Lr[jn] = look_r(bb[0].r[jn], 1);
         }
       }
@@ -480,7 +460,7 @@ __global__ __launch_bounds__(GQ_THREADS) void k_gemm_e8(GQArgs a) {
               Bn[jn] = cvt(Lc[jn]);
               if constexpr (HT) {
                 Lrn[jn] = s < 6 ? look_r(b.r[jn], s + 2) : look_r(bn.r[jn], s - 6);
-                Rn[jn] = gq_f16_of_bytes(Lr[jn]);
+                Rn[jn] = q8_f16_of_bytes(Lr[jn]);
               }
             }
 #pragma unroll

@@ -122,6 +122,29 @@ __device__ __forceinline__ q8v4 mfma_i8(q8v4 a, q8v4 b, q8v4 c) {
   return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0);
 }
 
+typedef _Float16 q8h8 __attribute__((ext_vector_type(8)));
+typedef _Float16 q8h2 __attribute__((ext_vector_type(2)));
+
+// Bytes q + 128 (mod 256) of eight integer weights q -> the fp16 values q.
+__device__ __forceinline__ q8h8 q8_f16_of_bytes(uint2 b) {
+  const uint32_t k = 0x64646464u;
+  const uint32_t d[4] = {__builtin_amdgcn_perm(k, b.x, 0x04010400u), __builtin_amdgcn_perm(k, b.x, 0x04030402u),
+                         __builtin_amdgcn_perm(k, b.y, 0x04010400u), __builtin_amdgcn_perm(k, b.y, 0x04030402u)};
+  q8h8 r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const q8h2 v = __builtin_bit_cast(q8h2, d[i]) - q8h2{(_Float16)1152.f, (_Float16)1152.f};
+    r[2 * i] = v[0];
+    r[2 * i + 1] = v[1];
+  }
+  return r;
+}
+
+// Natural-order bytes of a packed-nibble-order pair (dims 0, 2, 4, 6 | 1, 3, 5, 7).
+__device__ __forceinline__ uint2 q8_natural(uint2 v) {
+  return make_uint2(__builtin_amdgcn_perm(v.y, v.x, 0x05010400u), __builtin_amdgcn_perm(v.y, v.x, 0x07030602u));
+}
+
 // Power-of-two s with max_abs * s in [32, 64) (max_abs > 0), and 1 / (4 s);
 // NaN for a non-finite max_abs, so that it reaches the outputs.
 __device__ __forceinline__ void q8_scale(float max_abs, float& s, float& inv4s) {

@@ -38,10 +38,21 @@ NO_RESIDUAL = 0xFFFFFFFF
 # below it the wave-per-rows mat-vec serves every route directly.
 GEMM_ROUTE_THRESHOLD = 128
 GEMM_ROUTE_TILE = 64
-# rows x outputs from which one matrix goes to the MFMA GEMM. Both times grow with K (the mat-vec's also with rows
-# x outputs: 2.0 us per row of 4096 x 4096 in 8 bits, 2.9 in 16; the GEMM's floor there is 25 us in 8 bits, 34 / 42
-# in 16 for fp16 / bf16 rows), so they meet near 13 rows of 4096 outputs and near 100 of 520 at K = 1024.
+# One matrix against M rows: the mat-vec, the matrix-core rows kernel (keep_vq_rows), the MFMA GEMM (keep_vq_gemm).
+# The mat-vec takes ~4 us plus 1 us per 8.1M (8-bit) / 5.3M (E8P) products M N K, the rows kernel 9-14 us until its
+# tiles fill the chip: they meet near 64M / 32M. The GEMM takes 25-40 us until its tiles do and meets the rows kernel
+# near M N = 2M in 8 bits (4096 x 4096: 33 against 41 us at 512 rows, 52 against 44 at 1024), 1.3M for E8P (31 / 40 at
+# 256, 54 / 43 at 512). Where the rows kernel does not serve (bf16 rows of E8P), mat-vec and GEMM meet near 64K.
+ROWS_PRODUCTS = {8: 1 << 26, 16: 1 << 25}
 MATRIX_GEMM_CELLS = 1 << 16
+ROWS_GEMM_CELLS = {8: 1 << 21, 16: 5 << 18}
+# Routed calls by routes per expert: in tiles of 16 against the GEMM's 64. 8-bit, 32 experts 4096 -> 2048: 57 against
+# 65 us at 32 routes per expert, 115 / 138 at 128; E8P, 256 experts: 270 / 311 at 8, 367 / 322 at 16.
+ROWS_PER_EXPERT = {8: 128, 16: 12}
+# Outputs x inputs from which few routes take the rows kernel (a matter of the matrix alone: grouped, flat and
+# single-row calls then agree bit for bit): 4096 -> 2048, 8 rows x top-6 of 256, 24 against 57 us, one row 10.9 / 11.6.
+ROWS_MATRIX = 1 << 21
+PLANNED_ROUTES = 128  # routes keep_vq_rows groups without a route plan
 _VERIFY_DEFAULT_M_ROWS = 4
 VERIFY_MROWS_VALUES = (1, 2, 3, 4, 8)
 
@@ -391,6 +402,45 @@ def matrix_gemm(x: torch.Tensor, codes: torch.Tensor, scales: torch.Tensor, code
     return out
 
 
+def rows_eligible(x: torch.Tensor, codes: torch.Tensor, scales: torch.Tensor, codebook: torch.Tensor, *,
+                  code_bits: int, input_dims: int, group_size: int) -> bool:
+    """Whether ``keep_vq_rows`` serves this call: 8-bit E8 with fp16/bf16 rows, or E8P (default table) with fp16
+    rows; up to 16 K slices of 512 / 256, scale groups of whole slices; aligned pools."""
+
+    ck = 512 if code_bits == 8 else 256
+    if (input_dims % ck or input_dims > 16 * ck or group_size % ck or x.numel() >= 1 << 30
+            or codes.data_ptr() % 16 or scales.data_ptr() % 4 or x.data_ptr() % 16):
+        return False
+    if code_bits == 8:
+        return x.dtype in (torch.float16, torch.bfloat16) and codebook.data_ptr() % 16 == 0
+    return x.dtype == torch.float16 and codebook is _default_codebook(16, codebook.device) and _may_prepare(codebook)
+
+
+def rows_matvec(x: torch.Tensor, codes: torch.Tensor, scales: torch.Tensor, codebook: torch.Tensor,
+                rhs: torch.Tensor | None, *, lhs: torch.Tensor | None = None, x_div: int = 1, grouped: bool = False,
+                input_dims: int, output_dims: int, group_size: int, code_bits: int) -> torch.Tensor:
+    """``keep_vq_rows``: ``out[r] = W[rhs[r]] . x[lhs[r] or r // x_div]`` -> ``[R, N]`` on the matrix cores
+    (``rhs=None``: one matrix against every row of x). ``grouped``: routes of one expert share its codes."""
+
+    device = x.device
+    R = x.shape[0] if rhs is None else rhs.numel()
+    out = torch.empty((R, output_dims), dtype=x.dtype, device=device)
+    if R == 0:
+        return out
+    table = prepared_table(codebook) if code_bits == 16 else codebook
+    plan = (None, None, None, None)
+    n_tiles = 0
+    if grouped and R > PLANNED_ROUTES:  # below, the kernel groups them itself
+        order, _, _, _, te, to, tc, _ = route_plan(rhs, codes.shape[0], 16)
+        plan, n_tiles = (order, te, to, tc), min(te.numel(), R)  # the tiles that hold routes come first
+    _lib.call("keep_vq_rows", x.data_ptr(), _DT[x.dtype], x.shape[0], codes.data_ptr(), code_bits, scales.data_ptr(),
+              _dtype_code(scales, "scales"), table.data_ptr(), _ptr(rhs), _ptr(lhs), R, x_div, int(grouped),
+              _ptr(plan[0]), _ptr(plan[1]), _ptr(plan[2]), _ptr(plan[3]), n_tiles,
+              codes.shape[0], output_dims, input_dims, group_size, out.data_ptr(), _DT[out.dtype],
+              _stream(device))
+    return out
+
+
 def grouped_residual_add(out: torch.Tensor, x: torch.Tensor, codes: torch.Tensor, scales: torch.Tensor,
                          tile_descriptors, *, lhs: torch.Tensor | None, out_index: torch.Tensor | None, routes: int,
                          input_dims: int, output_dims: int, group_size: int,
@@ -631,13 +681,20 @@ def vq_qmm(x, codes, scales, codebook=None, *, in_dim: int, out_dim: int, group_
         raise ValueError(f"scales must have shape ({out_dim}, {in_dim // group_size}), found {tuple(s.shape)}")
     cb = _codebook_tensor(codebook, code_bits, device)
     M = xt.shape[0]
+    cells = M * out_dim
+    few = cells * in_dim >= ROWS_PRODUCTS[code_bits] and rows_eligible(
+        xt, c, s, cb, code_bits=code_bits, input_dims=in_dim, group_size=group_size)
     # E8P on the matrix cores takes the default table only: they decode it from odd half-units, the mat-vec any
-    if (M * out_dim >= MATRIX_GEMM_CELLS and xt.dtype in (torch.float16, torch.bfloat16)
+    if (cells >= (ROWS_GEMM_CELLS[code_bits] if few else MATRIX_GEMM_CELLS)
+            and xt.dtype in (torch.float16, torch.bfloat16)
             and gemm_eligible(code_bits=code_bits, x_dtype=xt.dtype, input_dims=in_dim, group_size=group_size)
             and (code_bits == 8 or (cb is _default_codebook(16, device) and _may_prepare(cb)))
             and _gemm_pointers_ok(c, s, cb, code_bits)):
         return matrix_gemm(xt, c, s, cb, input_dims=in_dim, output_dims=out_dim, group_size=group_size,
                            code_bits=code_bits)
+    if few:
+        return rows_matvec(xt, c.reshape(1, out_dim, -1), s.reshape(1, out_dim, -1), cb, None, input_dims=in_dim,
+                           output_dims=out_dim, group_size=group_size, code_bits=code_bits)
     return routed_matvec(xt, c.reshape(1, out_dim, -1), s.reshape(1, out_dim, -1), cb, None, input_dims=in_dim,
                          output_dims=out_dim, group_size=group_size, code_bits=code_bits, routes=M)
 
@@ -736,11 +793,20 @@ def gather_vqmm(x, codes, scales, codebook, rhs_indices, *, lhs_indices=None, in
            input_dims=int(input_dims), output_dims=int(output_dims), group_size=int(group_size),
            code_bits=int(code_bits), strategy=strategy,
            implementation="mfma_grouped_gemm" if strategy == "sorted_tiled" and eligible else "hip_matvec")
+    few = rows_eligible(xt, c, s, cb, code_bits=code_bits, input_dims=input_dims, group_size=group_size)
     if strategy in ("direct", "per_route_decoded"):
+        if output_dims * input_dims >= ROWS_MATRIX and few:
+            y = rows_matvec(xt, c, s, cb, flat_rhs, lhs=lhs, x_div=x_div, grouped=R > x_div, input_dims=input_dims,
+                            output_dims=output_dims, group_size=group_size, code_bits=code_bits)
+            return y.reshape(out_shape)
         y = routed_matvec(xt, c, s, cb, flat_rhs, lhs=lhs, x_div=x_div, input_dims=input_dims,
                           output_dims=output_dims, group_size=group_size, code_bits=code_bits)
         return y.reshape(out_shape)
     # sorted_tiled
+    if few and R <= ROWS_PER_EXPERT[code_bits] * E:
+        y = rows_matvec(xt, c, s, cb, flat_rhs, lhs=lhs, x_div=x_div, grouped=True, input_dims=input_dims,
+                        output_dims=output_dims, group_size=group_size, code_bits=code_bits)
+        return y.reshape(out_shape)
     full_lhs = lhs if lhs is not None else torch.arange(R, dtype=torch.int32, device=device) // x_div
     order, inverse, _, _, te, to, tc, _ = route_plan(flat_rhs, E, GEMM_ROUTE_TILE)
     sorted_lhs = full_lhs[order.long()].contiguous()
@@ -802,6 +868,11 @@ def gather_vqmm_sorted_routes(x, codes, scales, codebook, sorted_rhs, sorted_lhs
     skip_gather = x_pre_sorted and xt.shape[0] == R
     use_lhs = None if skip_gather else lhs
     eligible = gemm_eligible(code_bits=code_bits, x_dtype=xt.dtype, input_dims=input_dims, group_size=group_size)
+    if (code_bits == 8 and GEMM_ROUTE_THRESHOLD <= R <= ROWS_PER_EXPERT[8] * E
+            and rows_eligible(xt, c, s, cb, code_bits=8, input_dims=input_dims, group_size=group_size)):
+        pos = torch.arange(R, dtype=torch.int32, device=device) if use_lhs is None else use_lhs
+        return rows_matvec(xt, c, s, cb, rhs, lhs=pos, grouped=True, input_dims=input_dims, output_dims=output_dims,
+                           group_size=group_size, code_bits=8)
     if eligible and code_bits == 8 and R >= GEMM_ROUTE_THRESHOLD and _gemm_pointers_ok(c, s, cb, 8):
         # a plan of its own, rows back at their positions: 8-bit calls never had to be sorted, nor their tiles right
         order, _, _, _, te, to, tc, _ = route_plan(rhs, E, GEMM_ROUTE_TILE)
@@ -875,7 +946,7 @@ def gather_vqmm_verify_rows(x, codes, scales, codebook, rhs_indices, *, lhs_indi
             raise ValueError(f"rhs_indices row dimension {rhs.shape[0]} must match x row dimension {xt.shape[0]}")
         top_k = rhs.shape[1]
         flat_rhs = rhs.reshape(-1)
-        flat_lhs = torch.arange(flat_rhs.numel(), dtype=torch.int32, device=device) // top_k
+        flat_lhs = None  # route r is row r // top_k's
         out_shape = (xt.shape[0], top_k, output_dims)
     R = flat_rhs.numel()
     if R == 0:
@@ -889,16 +960,24 @@ def gather_vqmm_verify_rows(x, codes, scales, codebook, rhs_indices, *, lhs_indi
     _trace(token_rows=int(xt.shape[0]), route_count=int(R), has_lhs_indices=lhs_indices is not None,
            input_dims=int(input_dims), output_dims=int(output_dims), group_size=int(group_size),
            code_bits=code_bits, strategy=f"verify_{grouping}", implementation="hip_matvec")
-    if grouping == "flat":
-        y = routed_matvec(xt, c, s, cb, flat_rhs, lhs=flat_lhs, input_dims=input_dims, output_dims=output_dims,
-                          group_size=group_size, code_bits=code_bits)
+    x_div = top_k or 1
+    if output_dims * input_dims >= ROWS_MATRIX and rows_eligible(
+            xt, c, s, cb, code_bits=code_bits, input_dims=input_dims, group_size=group_size):
+        y = rows_matvec(xt, c, s, cb, flat_rhs, lhs=flat_lhs, x_div=x_div, grouped=grouping == "expert",
+                        input_dims=input_dims, output_dims=output_dims, group_size=group_size, code_bits=code_bits)
         return y.reshape(out_shape)
+    if grouping == "flat":
+        y = routed_matvec(xt, c, s, cb, flat_rhs, lhs=flat_lhs, x_div=x_div, input_dims=input_dims,
+                          output_dims=output_dims, group_size=group_size, code_bits=code_bits)
+        return y.reshape(out_shape)
+    if flat_lhs is None:
+        flat_lhs = torch.arange(R, dtype=torch.int32, device=device) // top_k
     order, inverse, _, _, te, to, tc, _ = route_plan(flat_rhs, E, mr)
     sorted_lhs = flat_lhs[order.long()].contiguous()
     routed = torch.empty((R, output_dims), dtype=output_dtype(xt.dtype), device=device)
     _lib.call("keep_vq_matvec_tiles", xt.data_ptr(), _dtype_code(xt, "x"), xt.shape[0], c.data_ptr(), code_bits,
               s.data_ptr(), _dtype_code(s, "scales"), cb.data_ptr(), sorted_lhs.data_ptr(), R, te.data_ptr(),
-              to.data_ptr(), tc.data_ptr(), te.numel(), mr, E, output_dims, input_dims, group_size,
+              to.data_ptr(), tc.data_ptr(), min(te.numel(), R), mr, E, output_dims, input_dims, group_size,
               routed.data_ptr(), _DT[routed.dtype], _stream(device))
     return routed[inverse.long()].reshape(out_shape)
 

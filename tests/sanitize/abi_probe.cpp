@@ -78,6 +78,8 @@ int main() {
   PROBE(keep_vq_grouped_gemm_q8);
   PROBE(keep_vq_grouped_gemm_e8);
   PROBE(keep_vq_gemm);
+  PROBE(keep_vq_rows_supported);
+  PROBE(keep_vq_rows);
   PROBE(keep_vq_grouped_swiglu_q8);
   PROBE(keep_vq_grouped_swiglu_nested_q8);
   PROBE(keep_vq_grouped_gemm_nested_q8);

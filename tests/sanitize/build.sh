@@ -11,7 +11,7 @@ mkdir -p "$OUT"
 HIPCC=${HIPCC:-/opt/rocm/bin/hipcc}
 SAN="-Xarch_host -fsanitize=address -Xarch_host -fsanitize=undefined -Xarch_host -fno-sanitize-recover=all"
 pids=()
-for src in abi.cpp matvec.hip moe.hip moe_i8.hip moe_tiles.hip router.hip plan.hip gemm_q8.hip rht.hip layer.hip block.hip encode.hip; do
+for src in abi.cpp matvec.hip moe.hip moe_i8.hip moe_tiles.hip router.hip plan.hip gemm_q8.hip rows.hip rht.hip layer.hip block.hip encode.hip; do
   $HIPCC -x hip -O1 -g -fPIC -std=c++17 --offload-arch=gfx950 $SAN -Xclang -target-feature -Xclang -packed-fp32-ops \
     -Wno-unused-command-line-argument -c "$ROOT/keep_amd/csrc/$src" -o "$OUT/${src%.*}.lib.o" &
   pids+=($!)
