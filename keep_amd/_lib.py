@@ -160,4 +160,6 @@ def check(rc: int, what: str) -> None:
 
 
 def call(name: str, *args) -> None:
-    check(getattr(load(), name)(*args), name)
+    rc = getattr(_lib or load(), name)(*args)
+    if rc != KEEP_OK:
+        check(rc, name)

@@ -99,14 +99,13 @@ class QuantizedVQLinear:
             x = apply_rht(x, self.rht_signs, validate_signs=False)  # checked once, at construction
         if self.rotation_matrix is not None:
             x = x @ self.rotation_matrix.to(x.dtype)
-        flat = x.reshape(-1, self.input_dims)
         kw = dict(in_dim=self.input_dims, out_dim=self.output_dims, group_size=self.group_size,
                   code_bits=self.code_bits)
-        if flat.shape[0] == 1:
-            y = ops.vq_qmv(flat[0], self.codes, self.scales, self.codebook, **kw).reshape(1, self.output_dims)
+        if x.numel() == self.input_dims:
+            y = ops.vq_qmv(x.reshape(self.input_dims), self.codes, self.scales, self.codebook, **kw)
         else:
-            y = ops.vq_qmm(flat, self.codes, self.scales, self.codebook, **kw)
-        y = y.reshape(tuple(x.shape[:-1]) + (self.output_dims,))
+            y = ops.vq_qmm(x.reshape(-1, self.input_dims), self.codes, self.scales, self.codebook, **kw)
+        y = y.reshape(x.shape[:-1] + (self.output_dims,))
         if self.bias is not None:
             y = y + self.bias  # type promotion as MLX's: a float32 bias gives a float32 result
         return y
@@ -331,10 +330,10 @@ class HotTier:
     def layer_groups(self, hidden: int, intermediate: int):
         """``(group_size_h, group_size_i)`` of the residual scales, or None when
         the fused decode layer cannot take them (groups of 256-multiples)."""
-        gh = hidden // self.residual_arrays["gate"][1].shape[-1]
-        gi = intermediate // self.residual_arrays["down"][1].shape[-1]
-        dts = {sc.dtype for _, sc in self.residual_arrays.values()}
-        if self.residual_arrays["up"][1].shape[-1] != self.residual_arrays["gate"][1].shape[-1] or len(dts) != 1:
+        gs, us, ds = (self.residual_arrays[n][1] for n in ("gate", "up", "down"))
+        gh = hidden // gs.shape[-1]
+        gi = intermediate // ds.shape[-1]
+        if us.shape[-1] != gs.shape[-1] or not (gs.dtype == us.dtype == ds.dtype):
             return None
         if gh % 256 or gi % 256 or hidden % gh or intermediate % gi:
             return None
@@ -402,8 +401,10 @@ class QuantizedVQSwitchGLU:
         return self.activation(up, gate)
 
     def _all_e8p(self) -> bool:
-        return all(p.code_bits == 16 and p.bias is None and p.rht_signs is None and p.rotation_matrix is None
-                   for p in (self.gate_proj, self.up_proj, self.down_proj))
+        for p in (self.gate_proj, self.up_proj, self.down_proj):
+            if p.code_bits != 16 or p.bias is not None or p.rht_signs is not None or p.rotation_matrix is not None:
+                return False
+        return True
 
     def _can_use_shared_sorted_route_prefill(self, x: torch.Tensor, indices: torch.Tensor) -> bool:
         routes = indices.numel()
@@ -596,6 +597,25 @@ def moe_decode(x: torch.Tensor, idx: torch.Tensor, weight: torch.Tensor, gate, u
     return out
 
 
+def _f32(t, device: torch.device, *shape: int):
+    """``t`` as a contiguous float32 tensor of ``shape`` (one row count, one -1) on ``device``; None stays None."""
+
+    if t is None:
+        return None
+    if (t.dtype == torch.float32 and t.device == device and t.ndim == len(shape) and t.is_contiguous()
+            and (shape[0] == -1 or t.shape[0] == shape[0])):
+        return t
+    return t.to(device=device, dtype=torch.float32).reshape(shape).contiguous()
+
+
+def _router_output(T: int, k: int, device: torch.device) -> RouterOutput:
+    """Uninitialised router outputs, the four 32-bit ones in one allocation (4.4 us on the host against 6.5)."""
+
+    idx, weight, want, score = torch.empty((4, T, k), dtype=torch.int32, device=device).unbind(0)
+    return RouterOutput(idx, weight.view(torch.float32), want, score.view(torch.float32),
+                        torch.empty((T, k), dtype=torch.uint8, device=device))
+
+
 def _tiles_entry(T: int, E: int, H: int, I: int, k: int, gh: int, gi: int, cb: torch.Tensor, codes, scales):
     """The few-token entry point that serves a shape, or None. Hidden sizes beyond 4096 take it on the default
     table and on aligned pools only: the matrix-core decode needs odd half-units and loads 16 bytes of codes and
@@ -644,22 +664,17 @@ def _tiles_layer(entry: str, x, logits, gate, up, down, k, bias_served, bias_dem
     if not (gs.dtype == us.dtype == ds.dtype):
         raise ValueError("gate/up/down scales must share a dtype")
     T = x.shape[0]
-    z = logits.to(device=device, dtype=torch.float32).reshape(T, -1).contiguous()
+    z = _f32(logits, device, T, -1)
     E = z.shape[1]
     if slot_map is None and E != S:
         raise ValueError(f"logits must hold {S} experts, found {E}")
     sm, ns = _slot_args(slot_map, S if slot_map is not None else None, E, device)
-    bs = None if bias_served is None else bias_served.to(device=device, dtype=torch.float32).reshape(-1).contiguous()
-    bd = None if bias_demand is None else bias_demand.to(device=device, dtype=torch.float32).reshape(-1).contiguous()
-    if bias_demand is bias_served:
-        bd = bs
+    bs = _f32(bias_served, device, -1)
+    bd = bs if bias_demand is bias_served else _f32(bias_demand, device, -1)
     for name, b in (("bias_served", bs), ("bias_demand", bd)):
         if b is not None and b.numel() != E:
             raise ValueError(f"{name} must have {E} entries, found {b.numel()}")
-    i32 = dict(dtype=torch.int32, device=device)
-    f32 = dict(dtype=torch.float32, device=device)
-    r = RouterOutput(torch.empty((T, k), **i32), torch.empty((T, k), **f32), torch.empty((T, k), **i32),
-                     torch.empty((T, k), **f32), torch.empty((T, k), dtype=torch.uint8, device=device))
+    r = _router_output(T, k, device)
     od = out_dtype or torch.float32
     out = torch.empty((T, H), dtype=od, device=device)
     if h_work is None:
@@ -775,7 +790,7 @@ def moe_layer(x: torch.Tensor, logits: torch.Tensor, gate, up, down, *, k: int, 
         raise ValueError("gate/up codes must be [E, I, H/8] and down codes [E, H, I/8]")
     if not (gs.dtype == us.dtype == ds.dtype):
         raise ValueError("gate/up/down scales must share a dtype")
-    z = logits.to(device=device, dtype=torch.float32).reshape(1, -1).contiguous()
+    z = _f32(logits, device, 1, -1)
     S = E  # pool rows
     if slot_map is not None:
         E = z.shape[1]
@@ -785,17 +800,12 @@ def moe_layer(x: torch.Tensor, logits: torch.Tensor, gate, up, down, *, k: int, 
     gh, gi = H // gs.shape[-1], I // ds.shape[-1]
     if not one_launch and not moe_layer_supported(E, H, I, k, gh, gi):
         raise ValueError("shape not served by the routed decode layer; use router_dual_topk + moe_decode")
-    bs = None if bias_served is None else bias_served.to(device=device, dtype=torch.float32).reshape(-1).contiguous()
-    bd = None if bias_demand is None else bias_demand.to(device=device, dtype=torch.float32).reshape(-1).contiguous()
-    if bias_demand is bias_served:
-        bd = bs
+    bs = _f32(bias_served, device, -1)
+    bd = bs if bias_demand is bias_served else _f32(bias_demand, device, -1)
     for name, b in (("bias_served", bs), ("bias_demand", bd)):
         if b is not None and b.numel() != E:
             raise ValueError(f"{name} must have {E} entries, found {b.numel()}")
-    i32 = dict(dtype=torch.int32, device=device)
-    f32 = dict(dtype=torch.float32, device=device)
-    r = RouterOutput(torch.empty((1, k), **i32), torch.empty((1, k), **f32), torch.empty((1, k), **i32),
-                     torch.empty((1, k), **f32), torch.empty((1, k), dtype=torch.uint8, device=device))
+    r = _router_output(1, k, device)
     od = out_dtype or torch.float32
     out = torch.empty((1, H), dtype=od, device=device)
     cb = ops._codebook_tensor(codebook, 16, device)
@@ -833,8 +843,10 @@ def moe_layer(x: torch.Tensor, logits: torch.Tensor, gate, up, down, *, k: int, 
                   r.want.data_ptr(), r.want_score.data_ptr(), r.admit.data_ptr(), ws.data_ptr(), ws.numel(),
                   out.data_ptr(), ops._DT[od], ops._stream(device))
         return out, r
-    if h_work is None:
-        h_work = torch.empty((k * I,), dtype=torch.bfloat16, device=device)
+    hot_route = None
+    if h_work is None:  # with a tier, each route's residual row (int32) behind h
+        h_work = torch.empty((k * I + 2 * k,), dtype=torch.bfloat16, device=device)
+        hot_route = h_work.data_ptr() + 2 * k * I
     elif h_work.numel() < k * I or h_work.dtype != torch.bfloat16:
         raise ValueError("h_work must hold k*I bfloat16 elements")
     if hot_tier is not None:
@@ -844,7 +856,9 @@ def moe_layer(x: torch.Tensor, logits: torch.Tensor, gate, up, down, *, k: int, 
         if groups is None:
             raise ValueError("residual scale groups must be 256-element multiples (one dtype) for the decode layer")
         (rgc, rgs), (ruc, rus), (rdc, rds) = (hot_tier.residual_arrays[n] for n in ("gate", "up", "down"))
-        hot_route = torch.empty((k,), **i32)
+        if hot_route is None:
+            rows = torch.empty((k,), dtype=torch.int32, device=device)
+            hot_route = rows.data_ptr()
         _lib.call("keep_moe_layer_nested", z.data_ptr(), ops._ptr(bs), ops._ptr(bd), _lib.SCORE_FUNCS[score_func],
                   int(bool(renormalize)), float(route_scale), float(tau), ops._ptr(sm), ns, E, k, x.data_ptr(),
                   ops._DT[x.dtype], H, I, gc.data_ptr(), gs.data_ptr(), uc.data_ptr(), us.data_ptr(), dc.data_ptr(),
@@ -853,7 +867,7 @@ def moe_layer(x: torch.Tensor, logits: torch.Tensor, gate, up, down, *, k: int, 
                   r.want.data_ptr(), r.want_score.data_ptr(), r.admit.data_ptr(), h_work.data_ptr(), out.data_ptr(),
                   ops._DT[od], hot_tier._hot32.data_ptr(), hot_tier.rows, rgc.data_ptr(), rgs.data_ptr(),
                   ruc.data_ptr(), rus.data_ptr(), rdc.data_ptr(), rds.data_ptr(), ops._DT[rgs.dtype], groups[0],
-                  groups[1], hot_tier.image().data_ptr(), hot_route.data_ptr(), ops._stream(device))
+                  groups[1], hot_tier.image().data_ptr(), hot_route, ops._stream(device))
         return out, r
     _lib.call("keep_moe_layer", z.data_ptr(), ops._ptr(bs), ops._ptr(bd), _lib.SCORE_FUNCS[score_func],
               int(bool(renormalize)), float(route_scale), float(tau), ops._ptr(sm), ns, E, k, x.data_ptr(),

@@ -162,6 +162,10 @@ def e8_1bit_half2_table() -> np.ndarray:
 # --------------------------------------------------------------------------- tensor plumbing
 
 _DT = {torch.float32: _lib.KEEP_F32, torch.float16: _lib.KEEP_F16, torch.bfloat16: _lib.KEEP_BF16}
+_CODES = {8: torch.uint8, 16: torch.int16}  # as calls usually hold them: the other forms take the slower checks
+_CODE_BITS = {torch.uint8: 8, torch.int16: 16}
+_PLAIN = (*_DT, *_CODE_BITS, torch.int32)
+_raw_stream = torch._C._cuda_getCurrentRawStream
 
 
 def _dtype_code(t: torch.Tensor, what: str) -> int:
@@ -187,6 +191,9 @@ def _device_of(*ts) -> torch.device:
 
 
 def _to_dev(a, device: torch.device, dtype: torch.dtype | None = None) -> torch.Tensor:
+    if (isinstance(a, torch.Tensor) and a.device == device and a.dtype in _PLAIN and a.is_contiguous()
+            and (dtype is None or a.dtype == dtype)):
+        return a
     if isinstance(a, np.ndarray):
         if a.dtype == np.uint16:
             a = a.view(np.int16)
@@ -205,6 +212,8 @@ def _to_dev(a, device: torch.device, dtype: torch.dtype | None = None) -> torch.
 
 
 def _codes_tensor(codes, code_bits: int, device) -> torch.Tensor:
+    if isinstance(codes, torch.Tensor) and codes.dtype == _CODES.get(code_bits):
+        return _to_dev(codes, device)
     t = codes if isinstance(codes, torch.Tensor) else None
     name = str(t.dtype if t is not None else np.asarray(codes).dtype)
     want = ("uint16", "int16") if code_bits == 16 else ("uint8", "int8")
@@ -217,6 +226,8 @@ def _codes_tensor(codes, code_bits: int, device) -> torch.Tensor:
 def _code_bits_of(codes) -> int:
     """8 for uint8/int8 codes (8-bit E8), 16 for uint16/int16 (E8P)."""
 
+    if isinstance(codes, torch.Tensor) and codes.dtype in _CODE_BITS:
+        return _CODE_BITS[codes.dtype]
     name = str(codes.dtype if isinstance(codes, torch.Tensor) else np.asarray(codes).dtype).rsplit(".", 1)[-1]
     if name in ("uint8", "int8"):
         return 8
@@ -228,6 +239,9 @@ def _code_bits_of(codes) -> int:
 def _codebook_tensor(codebook, code_bits: int, device) -> torch.Tensor:
     if codebook is None:
         return _default_codebook(code_bits, device)
+    if (isinstance(codebook, torch.Tensor) and codebook.dtype == torch.int32 and codebook.device == device
+            and codebook.shape == (256,) and codebook.is_contiguous()):
+        return codebook
     name = str(codebook.dtype).rsplit(".", 1)[-1]
     if name not in ("uint32", "int32"):
         raise ValueError(f"codebook dtype must be uint32, found {codebook.dtype}")
@@ -244,7 +258,10 @@ def _index_tensor(ix, device) -> torch.Tensor:
 
 
 def _stream(device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The current stream's handle, without building a ``torch.cuda.Stream`` (0.1 us against 1.9)."""
+
+    index = device.index
+    return _raw_stream(torch.cuda.current_device() if index is None else index)
 
 
 def _check_impl(implementation: str) -> None:
@@ -637,6 +654,20 @@ def decode_weight_matrix(codes, scales=None, *, code_bits: int = 8, codebook=Non
 # --------------------------------------------------------------------------- vq_qmv / vq_qmm
 
 
+def _matrix_matvec(x, rows: int, codes, scales, codebook, shape, in_dim: int, out_dim: int, group_size: int,
+                   code_bits: int) -> torch.Tensor:
+    """``keep_vq_matvec`` of one matrix ``[N, K/8]`` against ``rows`` rows, as ``shape``."""
+
+    od = output_dtype(x.dtype)
+    out = torch.empty(shape, dtype=od, device=x.device)
+    if rows:
+        _lib.call("keep_vq_matvec", x.data_ptr(), _dtype_code(x, "x"), rows, codes.data_ptr(), code_bits,
+                  scales.data_ptr(), _dtype_code(scales, "scales"), codebook.data_ptr(), None, None, rows, 1, 1,
+                  out_dim, in_dim, group_size, None, None, 0, None, None, 0, out.data_ptr(), _DT[od],
+                  _stream(x.device))
+    return out
+
+
 def vq_qmv(x, codes, scales, codebook=None, *, in_dim: int, out_dim: int, group_size: int = 512,
            code_bits: Literal[8, 16] = 8, implementation: str = "hip",
            codebook_duplication: Literal[1, 4, 8] = 1) -> torch.Tensor:
@@ -656,9 +687,7 @@ def vq_qmv(x, codes, scales, codebook=None, *, in_dim: int, out_dim: int, group_
     if tuple(s.shape) != (out_dim, in_dim // group_size):
         raise ValueError(f"scales must have shape ({out_dim}, {in_dim // group_size}), found {tuple(s.shape)}")
     cb = _codebook_tensor(codebook, code_bits, device)
-    y = routed_matvec(xt.reshape(1, in_dim), c.reshape(1, out_dim, -1), s.reshape(1, out_dim, -1), cb, None,
-                      input_dims=in_dim, output_dims=out_dim, group_size=group_size, code_bits=code_bits, routes=1)
-    return y.reshape(out_dim)
+    return _matrix_matvec(xt, 1, c, s, cb, (out_dim,), in_dim, out_dim, group_size, code_bits)
 
 
 def vq_qmm(x, codes, scales, codebook=None, *, in_dim: int, out_dim: int, group_size: int = 512,
@@ -695,8 +724,7 @@ def vq_qmm(x, codes, scales, codebook=None, *, in_dim: int, out_dim: int, group_
     if few:
         return rows_matvec(xt, c.reshape(1, out_dim, -1), s.reshape(1, out_dim, -1), cb, None, input_dims=in_dim,
                            output_dims=out_dim, group_size=group_size, code_bits=code_bits)
-    return routed_matvec(xt, c.reshape(1, out_dim, -1), s.reshape(1, out_dim, -1), cb, None, input_dims=in_dim,
-                         output_dims=out_dim, group_size=group_size, code_bits=code_bits, routes=M)
+    return _matrix_matvec(xt, M, c, s, cb, (M, out_dim), in_dim, out_dim, group_size, code_bits)
 
 
 # --------------------------------------------------------------------------- routed operators
