@@ -288,3 +288,29 @@ def test_routed_8bit_gemm_vs_oracle(dev, xdt, E, T, k, N, K, G):
     for out in (y, z):
         assert torch.isnan(out[torch.from_numpy(~good)]).all()
         _check(out[torch.from_numpy(good)], want[good], tol=TOL + ulp)
+
+
+@pytest.mark.parametrize("tail", [1, 700])
+@pytest.mark.parametrize("gap", [False, True])
+def test_empty_tiles_of_a_plan_change_nothing(tail, gap):
+    # N = 1544: four column blocks of 512 (the last ragged), so the items do not divide by the XCDs; the arrays end
+    # in `tail` empty tiles, and one may lie between live ones. Every row is computed alike: the bits are the same.
+    E, N, K, R = 9, 1544, 256, 200
+    g = torch.Generator().manual_seed(tail + gap)
+    codes = torch.randint(-32768, 32768, (E, N, K // 8), dtype=torch.int16, generator=g).cuda()
+    scales = torch.rand((E, N, 1), generator=g).half().cuda()
+    x = torch.randn((R, K), generator=g).half().cuda()
+    rhs = torch.randint(0, E, (R,), dtype=torch.int32, generator=g).cuda()
+    order, _, _, _, te, to, tc, _ = kops.route_plan(rhs, E, kops.GEMM_ROUTE_TILE)
+    n = int((tc > 0).sum())
+    cb = kops._default_codebook(16, x.device)
+
+    def gemm(*tiles):
+        return kops.grouped_gemm(x, codes, scales, cb, tuple(t.contiguous() for t in tiles), lhs=order, routes=R,
+                                input_dims=K, output_dims=N, group_size=K, out_index=order)
+
+    want = gemm(te[:n], to[:n], tc[:n])
+    hole = torch.zeros(1, dtype=torch.int32, device=x.device)
+    parts = [[t[:2], hole, t[2:n]] if gap else [t[:n]] for t in (te, to, tc)]
+    got = gemm(*(torch.cat(p + [hole.repeat(tail)]) for p in parts))
+    assert not torch.isnan(want).any() and torch.equal(got, want)
