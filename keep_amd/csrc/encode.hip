@@ -226,8 +226,10 @@ __global__ __launch_bounds__(ENC_THREADS) void k_e8_encode(const float* x, int64
 // vector) itself, off by less than EST = 2^-16 (|t|^2 / 2 + 64): 21 bits of
 // every factor, at most 48 additions of terms summing below 2 (|t|^2 / 2 + 64).
 // The bounds carry EST on top, so they are positive and order as their bits;
-// the low 8 bits make way for the row's place, which only lowers them. Each
-// lane keeps its two least (three operations per bound); the least of both
+// the low 8 bits make way for the row's place. Cleared they only lower a bound;
+// with the place in them a bound may stand up to 255 ulp higher, so the place
+// orders the bounds but is cleared again before one is held against a distance.
+// Each lane keeps its two least (three operations per bound); the least of both
 // halves is measured exactly (enc_row / enc_dist8, the scan's own arithmetic),
 // and a row whose bound is within the error of that distance (one vector in
 // 65 of an RTN weight has any) is queued, for the wave's lanes to measure side
@@ -461,8 +463,9 @@ __global__ __launch_bounds__(ENC_THREADS, 4) void k_encode_bounds(const float* x
         cnt += (uint32_t)__popcll(hit);
       }
     };
-    append(__uint_as_float(upper ? m1[0] : m1[1]) <= thr, row_of(upper ? m1[0] : m1[1], !upper) << 6 | (uint32_t)lane);
-    const unsigned long long again = __ballot(__uint_as_float(min(m2[0], m2[1])) <= thr);
+    const uint32_t other = upper ? m1[0] : m1[1];  // the other half's least
+    append(__uint_as_float(other & keep) <= thr, row_of(other, !upper) << 6 | (uint32_t)lane);
+    const unsigned long long again = __ballot(__uint_as_float(min(m2[0], m2[1]) & keep) <= thr);
     uint32_t sets = ((uint32_t)again != 0u ? 1u : 0u) | ((uint32_t)(again >> 32) != 0u ? 2u : 0u);
     while (cnt || sets) {
       if (cnt >= 64 || !sets) drain();

@@ -183,3 +183,20 @@ def test_encode_bounds_edges_bit_exact(dev, code_bits, n):
     enc = kenc.encode_e8p_rtn if code_bits == 16 else kenc.encode_e8_1bit_rtn
     got = _u(enc(torch.from_numpy(v).to(dev)))
     np.testing.assert_array_equal(got[~odd], oenc.nearest(v[~odd], code_bits))
+
+
+@pytest.mark.parametrize("code_bits", [8, 16])
+def test_encode_near_ties_of_large_vectors(dev, code_bits):
+    """Vectors of nearly equal large components, where many rows lie within the
+    bounds' error of the nearest: each encoded alone (no other vector's second
+    look covers it), the codes are the exhaustive scan's."""
+    rng = np.random.default_rng(47)
+    size = np.repeat([20.0, 33.0, 47.0, 58.0, 63.0], 64)[:, None]
+    v = size + rng.uniform(-0.05, 0.05, (320, 8))
+    v[:8] = 47.40516663  # ties broken in the last digits only
+    v = (v * rng.choice([-1.0, 1.0], (320, 8))).astype(np.float32)
+    v[8] = [47.40516663, -47.42156601, 47.43971252, -47.40866852, -47.39600754, 47.46210098, 47.44778824, -47.42797089]
+    enc = kenc.encode_e8p_rtn if code_bits == 16 else kenc.encode_e8_1bit_rtn
+    t = torch.from_numpy(v).to(dev)
+    got = _u(torch.cat([enc(t[i:i + 1].clone()) for i in range(len(v))]))
+    np.testing.assert_array_equal(got, oenc.nearest(v, code_bits))
