@@ -254,9 +254,8 @@ __global__ __launch_bounds__(1024) void k_moe_layer1(const float* logits, const 
     float v[4];
     if (a.xbf) q8_half4<true>(c, lane & 1, v);
     else q8_half4<false>(c, lane & 1, v);
-    float mx = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
     float s, inv4s;
-    q8_scale(rt_wave_max_abs(mx), s, inv4s);
+    q8_scale(__uint_as_float(rt_wave_u32<true>(rt_abs_bits4(v))), s, inv4s);
     uint32_t tw[3];
     q8_terms<3>(v, s, tw);
     uint32_t* aw = (uint32_t*)ash;

@@ -168,9 +168,8 @@ __global__ __launch_bounds__(1024) void k_moeq_route_gateup(const float* logits,
   auto build = [&](uint4 c, int slice) {
     float v[4];
     q8_half4<XBF>(c, lane & 1, v);
-    float mx = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
     float s, inv4s;
-    q8_scale(rt_wave_reduce(mx, true), s, inv4s);
+    q8_scale(__uint_as_float(__builtin_amdgcn_readfirstlane(rt_wave_u32<true>(rt_abs_bits4(v)))), s, inv4s);
     uint32_t tw[3];
     q8_terms<3>(v, s, tw);
     uint32_t* aw = (uint32_t*)ash;
@@ -483,9 +482,8 @@ __global__ __launch_bounds__(512) void k_moeq_down(const int32_t* idx, const flo
     for (int r = 0; r < KMAX; ++r) {
       float v[4];
       q8_half4<true>(hq[r], lane & 1, v);
-      const float mx = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
       float s;
-      q8_scale(rt_wave_reduce(mx, true), s, inv4s[r]);
+      q8_scale(__uint_as_float(__builtin_amdgcn_readfirstlane(rt_wave_u32<true>(rt_abs_bits4(v)))), s, inv4s[r]);
       uint32_t tw[2];
       q8_digits2(v, s, tw);
       aw[q8_aword((uint32_t)(wv * 2 * KMAX + 2 * r), lane >> 1, lane & 1)] = tw[0];

@@ -72,9 +72,8 @@ __device__ __forceinline__ void mt_xterms(const void* x, int H, uint4* xt, float
   const uint4 c = ldg16_q((const uint4*)x + ((size_t)t * H >> 3) + s * 32 + (lane >> 1));
   float v[4];
   q8_half4<XBF>(c, lane & 1, v);
-  const float mx = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
   float sc, inv4s;
-  q8_scale(rt_wave_reduce(mx, true), sc, inv4s);
+  q8_scale(__uint_as_float(__builtin_amdgcn_readfirstlane(rt_wave_u32<true>(rt_abs_bits4(v)))), sc, inv4s);
   uint32_t tw[3];
   q8_terms<3>(v, sc, tw);
   uint32_t* base = (uint32_t*)(xt + ((size_t)t * S + s) * 3 * 16);
@@ -447,9 +446,8 @@ __global__ __launch_bounds__(1024) void k_moeq_gateup_tiles(MTArgs a, MTRoute p)
       for (int i = 0; i < MT_TILE; ++i) {
         float v[4];
         q8_half4<XBF>(xc[i], lane & 1, v);
-        const float mx = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
         float sc, inv4s;
-        q8_scale(rt_wave_reduce(mx, true), sc, inv4s);
+        q8_scale(__uint_as_float(__builtin_amdgcn_readfirstlane(rt_wave_u32<true>(rt_abs_bits4(v)))), sc, inv4s);
         uint32_t tw[3];
         q8_terms<3>(v, sc, tw);
         uint32_t* base = (uint32_t*)RL.xl[wv][i];
@@ -765,9 +763,8 @@ __global__ __launch_bounds__(1024) void k_moeq_down_tiles(MTArgs a) {
       for (int i = 0; i < MT_TILE; ++i) {
         float v[4];
         q8_half4<true>(hq[i], lane & 1, v);
-        const float mx = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
         float sc, inv4s;
-        q8_scale(rt_wave_reduce(mx, true), sc, inv4s);
+        q8_scale(__uint_as_float(__builtin_amdgcn_readfirstlane(rt_wave_u32<true>(rt_abs_bits4(v)))), sc, inv4s);
         uint32_t tw[NT];
         if constexpr (THREE) q8_terms<3>(v, sc, tw);
         else q8_digits2(v, sc, tw);

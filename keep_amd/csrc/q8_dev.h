@@ -146,7 +146,8 @@ __device__ __forceinline__ uint2 q8_natural(uint2 v) {
 }
 
 // Power-of-two s with max_abs * s in [32, 64) (max_abs > 0), and 1 / (4 s);
-// NaN for a non-finite max_abs, so that it reaches the outputs.
+// NaN for a non-finite max_abs, so that it reaches the outputs (the maximum is
+// taken over the bits, rt_abs_bits4: a NaN among the values is then the maximum).
 __device__ __forceinline__ void q8_scale(float max_abs, float& s, float& inv4s) {
   const int e = max_abs > 0.f ? (int)((__float_as_uint(max_abs) >> 23) & 0xffu) - 126 : 0;  // max_abs < 2^e
   const int es = min(max(127 + 6 - e, 1), 254), ei = min(max(127 - 8 + e, 1), 254);

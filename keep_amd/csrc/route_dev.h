@@ -107,9 +107,13 @@ __device__ __forceinline__ uint32_t rt_wave_u32(uint32_t v) {
   const auto p32 = __builtin_amdgcn_permlane32_swap(v, v, false, false);
   return rt_op_u32<MAX>(p32[0], p32[1]);
 }
-// Max over the wave of non-negative floats (or NaN, which wins), by their bits.
-__device__ __forceinline__ float rt_wave_max_abs(float v) {
-  return __uint_as_float(rt_wave_u32<true>(__float_as_uint(v)));
+// The bits of the largest |v|: a NaN outranks every number, so that a maximum over the wave
+// (rt_wave_u32<true>) keeps it (fmaxf would drop it).
+__device__ __forceinline__ uint32_t rt_abs_bits4(const float (&v)[4]) {
+  uint32_t m = 0u;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) m = max(m, __float_as_uint(v[i]) & 0x7fffffffu);
+  return m;
 }
 
 __device__ __forceinline__ float rt_score_of(float z, int func) {

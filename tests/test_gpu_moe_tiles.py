@@ -337,3 +337,78 @@ def test_wide_hidden_custom_table_stays_on_packed_kernels(dev):
     a = keep_amd.moe_decode(x, r.idx, r.weight, *pairs, codebook=cb)
     assert torch.isfinite(a).all()
     assert torch.equal(a, keep_amd.moe_decode(x, r.idx, r.weight, *pairs, codebook=cb, prepared=False))
+
+
+@pytest.mark.parametrize("xdt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("T, k", [(3, 2), (30, 6), (40, 6)])
+def test_nan_token_reaches_its_output(dev, small_pool, xdt, T, k):
+    """A NaN in one value of a token makes that token's output NaN and no
+    other's: every launch form of the few-token layer (a wave's maximum must
+    not lose the NaN), with the tokens' routes sharing tiles."""
+    H, E = 1024, 20
+    pool = tuple((p.codes[:E], p.scales[:E]) for p in small_pool)
+    x = synth.rht_activations(T, H, seed=100 + T, device=dev).to(xdt)
+    z = synth.router_logits(T, E, seed=101 + T, device=dev)
+    want, r = keep_amd.moe_tiles_layer(x, z, *pool, k=k)
+    bad = x.clone()
+    bad[1, 777] = float("nan")
+    for out in (keep_amd.moe_tiles_layer(bad, z, *pool, k=k)[0], keep_amd.moe_decode(bad, r.idx, r.weight, *pool)):
+        assert torch.isnan(out[1]).all()
+        keep = torch.arange(T, device=dev) != 1
+        assert torch.equal(out[keep], want[keep])
+
+
+def test_nan_in_an_expert_reaches_the_outputs(dev, small_pool):
+    """A NaN scale of one gate row makes one value of h NaN: every token of that expert is NaN, no other."""
+    H, E, T, k = 1024, 20, 12, 3
+    pool = [(p.codes[:E].contiguous(), p.scales[:E].clone()) for p in small_pool]
+    x = synth.rht_activations(T, H, seed=110, device=dev)
+    z = synth.router_logits(T, E, seed=111, device=dev)
+    want, r = keep_amd.moe_tiles_layer(x, z, *pool, k=k)
+    e = int(r.idx[0, 0])
+    pool[0][1][e, 300] = float("nan")
+    hit = (r.idx == e).any(1)
+    assert hit.any() and not hit.all()
+    for out in (keep_amd.moe_tiles_layer(x, z, *pool, k=k)[0], keep_amd.moe_decode(x, r.idx, r.weight, *pool)):
+        assert torch.isnan(out[hit]).all()
+        assert torch.equal(out[~hit], want[~hit])
+
+
+@pytest.mark.parametrize("one_launch", [False, True])
+@pytest.mark.parametrize("xdt", [torch.float16, torch.bfloat16])
+def test_nan_token_one_token_layer(dev, xdt, one_launch):
+    E, H, I, k = 16, 4096, 512, 4
+    pool = [(p.codes, p.scales.clone()) for p in (synth.projection(E, I, H, seed=120, device=dev),
+                                                  synth.projection(E, I, H, seed=121, device=dev),
+                                                  synth.projection(E, H, I, seed=122, device=dev))]
+    x = synth.rht_activations(1, H, seed=123, device=dev).to(xdt)
+    z = synth.router_logits(1, E, seed=124, device=dev)
+    out, r = keep_amd.moe_layer(x, z, *pool, k=k, one_launch=one_launch)
+    assert torch.isfinite(out).all()
+    bad = x.clone()
+    bad[0, 3001] = float("nan")
+    out, _ = keep_amd.moe_layer(bad, z, *pool, k=k, one_launch=one_launch)
+    assert torch.isnan(out).all()
+    pool[1][1][int(r.idx[0, 0]), 100] = float("nan")  # one value of h
+    out, _ = keep_amd.moe_layer(x, z, *pool, k=k, one_launch=one_launch)
+    assert torch.isnan(out).all()
+
+
+@pytest.mark.parametrize("H", [4352, 7168])
+def test_nan_token_wide(dev, H):
+    """The same beyond 4096 hidden values, in a token (either set of slices) and in an expert's h."""
+    E, I, k, T = 6, 512, 2, 9
+    pool = [(p.codes, p.scales.clone()) for p in (synth.projection(E, I, H, seed=125, device=dev),
+                                                  synth.projection(E, I, H, seed=126, device=dev),
+                                                  synth.projection(E, H, I, seed=127, device=dev))]
+    x = torch.randn((T, H), generator=torch.Generator().manual_seed(128)).to(dev).half()
+    r = keep_amd.router_dual_topk(synth.router_logits(T, E, seed=129, device=dev), k)
+    want = keep_amd.moe_decode(x, r.idx, r.weight, *pool)
+    x[1, 17] = x[5, H - 1] = float("nan")
+    e = int(r.idx[0, 0])
+    pool[0][1][e, 500] = float("nan")
+    hit = (r.idx == e).any(1)
+    hit[1] = hit[5] = True
+    assert not hit.all()
+    out = keep_amd.moe_decode(x, r.idx, r.weight, *pool)
+    assert torch.isnan(out[hit]).all() and torch.equal(out[~hit], want[~hit])
