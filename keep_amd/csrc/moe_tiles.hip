@@ -36,6 +36,8 @@
 // terms for the tile it enters. Up to 32 tokens otherwise, one prologue
 // launch routes, plans and builds the terms; beyond, the router runs on its
 // own launch.
+#include <type_traits>
+
 #include "common.h"
 #include "moe_dev.h"
 #include "plan_dev.h"
@@ -64,8 +66,15 @@ struct MTArgs {
 
 // ------------------------------------------------------------------ x terms
 
+constexpr int MT_MAX_H = 4096, MT_WIDE_MAX_H = 8192;  // one K slice per gate/up wave; two (the WIDE kernel)
+
 // Token t, K slice s (one wave): the three int8 terms of x[t] * s_slice over
 // the slice's 256 values in the A-slot layout of q8_aword, and 1 / (4 s_slice).
+// Beyond MT_MAX_H a slice with infinities (and no NaN) takes the infinities'
+// signs for its terms and an infinite factor: a gate or up sum it enters is
+// infinite, of the right sign for one infinity, so that the token's output is
+// NaN through silu(-inf) whatever the SwiGLU clamp, as on the packed-table
+// kernels (a NaN sum would be clamped to the limit).
 template <bool XBF>
 __device__ __forceinline__ void mt_xterms(const void* x, int H, uint4* xt, float* xinv, int t, int s, int lane) {
   const int S = H >> 8;
@@ -73,7 +82,14 @@ __device__ __forceinline__ void mt_xterms(const void* x, int H, uint4* xt, float
   float v[4];
   q8_half4<XBF>(c, lane & 1, v);
   float sc, inv4s;
-  q8_scale(__uint_as_float(__builtin_amdgcn_readfirstlane(rt_wave_u32<true>(rt_abs_bits4(v)))), sc, inv4s);
+  const float mx = __uint_as_float(__builtin_amdgcn_readfirstlane(rt_wave_u32<true>(rt_abs_bits4(v))));
+  q8_scale(mx, sc, inv4s);
+  if (H > MT_MAX_H && mx == __builtin_inff()) {
+    sc = 1.f;
+    inv4s = mx;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = fabsf(v[i]) == mx ? copysignf(1.f, v[i]) : 0.f;
+  }
   uint32_t tw[3];
   q8_terms<3>(v, sc, tw);
   uint32_t* base = (uint32_t*)(xt + ((size_t)t * S + s) * 3 * 16);
@@ -300,7 +316,7 @@ __device__ __forceinline__ int mt_route_of_lanes(int rr, uint32_t i) {
 // the place of two units in flight (the same bytes), and their dots are added
 // before the cross-wave sum. 4 bf16 tokens, top-8 of 128 experts of 7168 x
 // 2048, groups of 512: 85 us per layer against 286 on the packed-table
-// mat-vecs, which decode every route's codes on the VALU.
+// mat-vecs, which decode every route's codes on the VALU. Infinities: mt_xterms.
 template <bool XBF, int RPER, bool WIDE = false>
 __global__ __launch_bounds__(1024) void k_moeq_gateup_tiles(MTArgs a, MTRoute p) {
   constexpr int SEG = 128;  // units per segment (h staging capacity)
@@ -664,7 +680,8 @@ __global__ __launch_bounds__(1024) void k_moeq_gateup_tiles(MTArgs a, MTRoute p)
 // tile and summed over the slices in slice order. THREE (hidden sizes beyond
 // 4096): three terms per route, rows 4r .. 4r + 2 as in gate/up, the same
 // MFMAs; h then keeps all but 2^-20 of its slice's max, below its bf16
-// rounding, as the fp32 mat-vecs these shapes used before kept it.
+// rounding, as the fp32 mat-vecs these shapes used before kept it. (A sum over
+// an infinity of h comes out NaN here; the combine forms it again.)
 template <bool THREE>
 __global__ __launch_bounds__(1024) void k_moeq_down_tiles(MTArgs a) {
   constexpr int NT = THREE ? 3 : 2;  // terms per route
@@ -895,9 +912,43 @@ __global__ __launch_bounds__(1024) void k_moeq_down_tiles(MTArgs a) {
 
 // ------------------------------------------------------------------ combine
 
+// One value of y again, in fp32 on the decoded weights: down row `row` against
+// a route's h. For the sums that came out NaN beyond MT_MAX_H: a slice of h
+// that holds an infinity has no int8 terms, and the sum is an infinity where
+// the packed-table kernels gave one.
+struct MTDown {
+  const uint16_t *dc, *h;
+  const void* ds;
+  const uint2* tm;  // keep_e8p_prepare's T, then M
+  int32_t sdt, I, Gi, gsz_i;
+};
+struct MTNone {};
+__device__ float mt_down_dot(const MTDown& a, int64_t route, int64_t row) {
+  const uint16_t *codes = a.dc + row * (a.I >> 3), *h = a.h + route * a.I;
+  float sum = 0.f;
+  for (int grp = 0; grp < a.Gi; ++grp) {
+    float v = 0.f;
+    for (int c = grp * (a.gsz_i >> 3); c < (grp + 1) * (a.gsz_i >> 3); ++c) {
+      const uint2 t = a.tm[codes[c] >> 8], m = a.tm[256 + (codes[c] & 255)];
+      const uint32_t b[2] = {t.x ^ m.x, t.y ^ m.y};  // dims 2 i, 2 i + 1
+      const uint4 hv = ldg16_q(h + c * 8);
+      for (uint32_t half = 0; half < 2; ++half) {
+        float f[4];
+        q8_half4<true>(hv, half, f);
+        for (int i = 0; i < 4; ++i) v = fmaf(0.25f * (float)((int)(b[half] << (24 - 8 * i)) >> 24), f[i], v);
+      }
+    }
+    const uint32_t si = (uint32_t)(row * a.Gi) + (uint32_t)grp;
+    sum += v * scale_cvt(scale_raw(a.ds, a.sdt, si), a.sdt, si);
+  }
+  return sum;
+}
+
+// down: MTDown where a NaN of y is formed again.
+template <typename Down>
 __global__ __launch_bounds__(256) void k_moe_combine(const float* y, const int32_t* idx, const float* w, int T,
                                                      int k, int E, int H, const uint32_t* tq_bad, void* out,
-                                                     int odt) {
+                                                     int odt, Down down) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= (int64_t)T * H) return;
   const int t = (int)(i / H), n = (int)(i - (int64_t)t * H);
@@ -922,7 +973,12 @@ __global__ __launch_bounds__(256) void k_moe_combine(const float* y, const int32
       if (r0 + r < k) {
         const bool ok = e[r] >= 0 && e[r] < E;
         bad |= wt[r] != 0.f && !ok;
-        if (ok && wt[r] != 0.f) o = fmaf(wt[r], yv[r], o);
+        if (ok && wt[r] != 0.f) {
+          if constexpr (std::is_same<Down, MTDown>::value)
+            if (__builtin_expect(yv[r] != yv[r], 0))
+              yv[r] = mt_down_dot(down, (int64_t)t * k + r0 + r, (int64_t)e[r] * H + n);
+          o = fmaf(wt[r], yv[r], o);
+        }
       }
     }
   }
@@ -977,8 +1033,6 @@ static int64_t mt_tiles_ub(int64_t T, int64_t k, int64_t E) {
   const int64_t R = T * k;
   return std::min<int64_t>(R, (R + MT_TILE - 1) / MT_TILE + E);
 }
-
-constexpr int64_t MT_MAX_H = 4096, MT_WIDE_MAX_H = 8192;  // one K slice per gate/up wave; two (the WIDE kernel)
 
 bool moe_tiles_supported(int64_t T, int64_t E, int64_t H, int64_t I, int64_t k, int64_t group_h, int64_t group_i,
                          int64_t max_h = MT_MAX_H) {
@@ -1098,8 +1152,13 @@ static void mt_tail(const MTArgs& a, int x_dtype, int64_t T, int64_t H, int64_t 
   if (H > MT_MAX_H) hipLaunchKernelGGL((k_moeq_down_tiles<true>), dim3(g2), dim3(1024), 0, s, a);
   else hipLaunchKernelGGL((k_moeq_down_tiles<false>), dim3(g2), dim3(1024), 0, s, a);
   const int64_t n = T * H;
-  hipLaunchKernelGGL(k_moe_combine, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a.y, idx, w, (int)T, (int)k,
-                     (int)num_experts, (int)H, a.tq_bad, out, out_dtype);
+  auto combine = [&](auto down) {
+    hipLaunchKernelGGL((k_moe_combine<decltype(down)>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a.y, idx, w,
+                       (int)T, (int)k, (int)num_experts, (int)H, a.tq_bad, out, out_dtype, down);
+  };
+  if (H > MT_MAX_H)
+    combine(MTDown{a.dc, a.h, a.ds, (const uint2*)((const char*)a.tq - TQR_OFFSET + TQ_OFFSET), a.sdt, a.I, a.Gi, a.gsz_i});
+  else combine(MTNone{});
 }
 
 static int mt_run(int64_t max_h, const void* x, int x_dtype, int64_t T, int64_t H, int64_t I, const int32_t* idx,

@@ -412,3 +412,88 @@ def test_nan_token_wide(dev, H):
     assert not hit.all()
     out = keep_amd.moe_decode(x, r.idx, r.weight, *pool)
     assert torch.isnan(out[hit]).all() and torch.equal(out[~hit], want[~hit])
+
+
+def _plain_layer(x, idx, w, pools, limit=0.0):
+    """The layer on decoded weights in float64 with h rounded to bf16; the clamp as the kernels' (a NaN gate or up
+    projection gives the limit, as fminf / fmaxf do)."""
+    dec = lambda p, K: e8p.decode_e8p(p[0].cpu().numpy().view(np.uint16)).reshape(p[0].shape[:2] + (K,)) * np.repeat(  # noqa: E731,E501
+        p[1].double().cpu().numpy(), K // p[1].shape[-1], -1)
+    gate, up, down = dec(pools[0], x.shape[1]), dec(pools[1], x.shape[1]), dec(pools[2], pools[2][0].shape[-1] * 8)
+    xd, out = x.double().cpu().numpy(), np.zeros((x.shape[0], down.shape[1]))
+    with np.errstate(all="ignore"):
+        for t, (es, ws) in enumerate(zip(idx.cpu().numpy(), w.double().cpu().numpy())):
+            for e, wt in zip(es, ws):
+                g, u = gate[e] @ xd[t], up[e] @ xd[t]
+                if limit > 0:
+                    g, u = np.fmin(g, limit), np.fmin(np.fmax(u, -limit), limit)
+                out[t] += wt * (down[e] @ ops.round_bf16(g / (1 + np.exp(-g)) * u).astype(np.float64))
+    return out
+
+
+def _same_values(got, want, packed, tol=TOL):
+    """NaN and infinities where the plain layer has them, finite values within
+    tol of their row's largest; an infinity of the packed-table kernels stays."""
+    got, packed = got.double().cpu().numpy(), packed.double().cpu().numpy()
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    inf = np.isinf(want) | np.isinf(packed)
+    np.testing.assert_array_equal(np.isinf(got), inf)
+    np.testing.assert_array_equal(got[inf], want[inf])
+    assert (got[np.isinf(packed)] == packed[np.isinf(packed)]).all()
+    fin = np.isfinite(want)
+    scale = np.abs(np.where(fin, want, 0)).max(-1, keepdims=True)
+    assert (np.abs(np.where(fin, got, 0) - np.where(fin, want, 0)) <= tol * scale).all()
+
+
+@pytest.mark.parametrize("limit", [0.0, 7.0])
+@pytest.mark.parametrize("xdt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("H, I, gh", [(4352, 256, 4352), (5120, 512, 256), (8192, 256, 4096)])
+def test_wide_non_finite_tokens(dev, xdt, H, I, gh, limit):
+    """Beyond 4096 hidden values: infinities (one, several of a slice with equal
+    and opposite signs, in either set of slices) and NaN in a token give the
+    plain layer's NaN (not the clamp's finite values), and the other tokens of
+    their tiles stay as they are."""
+    E, k, T = 4, 2, 12
+    pool = [(p.codes, p.scales) for p in (synth.projection(E, I, H, group_size=gh, seed=130, device=dev),
+                                          synth.projection(E, I, H, group_size=gh, seed=131, device=dev),
+                                          synth.projection(E, H, I, seed=132, device=dev))]
+    g = torch.Generator().manual_seed(133)
+    x = torch.randn((T, H), generator=g).to(dev).to(xdt)
+    w = torch.rand((T, k), generator=g).to(dev)
+    idx = torch.stack([torch.randperm(E, generator=g)[:k] for _ in range(T)]).int().to(dev)
+    good = keep_amd.moe_decode(x, idx, w, *pool, limit=limit)
+    inf, nan = float("inf"), float("nan")
+    put = {1: {5: nan}, 2: {300: inf}, 3: {H - 1: -inf}, 4: {10: inf, 20: -inf}, 5: {i: inf for i in range(9)},
+           6: {7: inf, H - 9: inf}, 7: {40: inf, 41: nan}, 9: {H - 200: nan}}
+    for t, vals in put.items():
+        for i, v in vals.items():
+            x[t, i] = v
+    out = keep_amd.moe_decode(x, idx, w, *pool, limit=limit)
+    packed = keep_amd.moe_decode(x, idx, w, *pool, limit=limit, prepared=False)
+    assert torch.equal(torch.isnan(out).all(1), torch.isnan(packed).all(1))
+    _same_values(out, _plain_layer(x, idx, w, pool, limit), packed)
+    rest = [t for t in range(T) if t not in put]
+    assert torch.equal(out[rest], good[rest])
+
+
+def test_wide_non_finite_h(dev):
+    """Values of h beyond bf16 (one, several of a slice and of two) and a NaN
+    one, through scales of single expert rows: infinities keep their signs."""
+    E, H, I, k, T = 8, 4608, 512, 2, 20
+    pool = [(p.codes, p.scales.float()) for p in (synth.projection(E, I, H, seed=140, device=dev),
+                                                  synth.projection(E, I, H, seed=141, device=dev),
+                                                  synth.projection(E, H, I, seed=142, device=dev))]
+    for e, rows in ((1, [70]), (2, [300]), (3, [5, 6]), (4, [100, 400]), (5, list(range(256, 276)))):
+        for n in rows:
+            pool[0][1][e, n] = pool[1][1][e, n] = 1e30
+    pool[1][1][6, 33] = float("nan")
+    g = torch.Generator().manual_seed(143)
+    x = torch.randn((T, H), generator=g).to(dev).half()
+    w = torch.rand((T, k), generator=g).to(dev)
+    idx = torch.stack([torch.randperm(E, generator=g)[:k] for _ in range(T)]).int().to(dev)
+    out = keep_amd.moe_decode(x, idx, w, *pool)
+    packed = keep_amd.moe_decode(x, idx, w, *pool, prepared=False)
+    want = _plain_layer(x, idx, w, pool)
+    assert np.isinf(want).any() and np.isnan(want).any() and np.isfinite(want).all(1).any()
+    assert torch.isinf(packed).any()
+    _same_values(out, want, packed)
