@@ -75,8 +75,10 @@ __device__ __forceinline__ f32x16 mfma32(h8 a, h8 b, f32x16 c) {
 // ------------------------------------------------------------------ row scales
 
 // One wave per row: r = 2^(14 - floor(log2 max |x|)) (1 for a zero row, NaN for a
-// row holding NaN or inf, which then reaches the row's outputs) and 1 / r.
-template <typename XT>
+// row holding NaN or inf, which then reaches the row's outputs) and 1 / r. PASS:
+// the max over the finite values, so that infinities and NaN go through the
+// matrix cores as such (one matrix: as the mat-vec has them, signs and all).
+template <typename XT, bool PASS>
 __global__ __launch_bounds__(256) void k_gq_rowscale(const XT* x, int64_t rows, int K, float2* rs) {
   const int lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -96,8 +98,9 @@ __global__ __launch_bounds__(256) void k_gq_rowscale(const XT* x, int64_t rows, 
     }
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-      bad |= !(fabsf(v[t]) <= 3.4028235e38f);  // NaN or inf
-      mx = fmaxf(mx, fabsf(v[t]));
+      const bool finite = fabsf(v[t]) <= 3.4028235e38f;
+      bad |= !PASS && !finite;
+      mx = fmaxf(mx, PASS && !finite ? 0.f : fabsf(v[t]));
     }
   }
   mx = wave_max(mx);
@@ -616,14 +619,15 @@ __global__ __launch_bounds__(256) void k_route_combine(const float* y, const flo
 // Workspace: the row factors of bf16 / fp32 rows.
 int64_t gq_ws_bytes(int64_t rows) { return (rows * (int64_t)sizeof(float2) + 255) / 256 * 256; }
 
+template <bool PASS = false>
 const float2* gq_rowscale(const void* x, int x_dtype, int64_t rows, int64_t K, void* ws, hipStream_t s) {
   if (x_dtype == KEEP_F16) return nullptr;
   float2* rs = (float2*)ws;
   const dim3 grid((unsigned)((rows + 3) / 4));
   if (x_dtype == KEEP_BF16)
-    hipLaunchKernelGGL((k_gq_rowscale<bf16s>), grid, dim3(256), 0, s, (const bf16s*)x, rows, (int)K, rs);
+    hipLaunchKernelGGL((k_gq_rowscale<bf16s, PASS>), grid, dim3(256), 0, s, (const bf16s*)x, rows, (int)K, rs);
   else
-    hipLaunchKernelGGL((k_gq_rowscale<float>), grid, dim3(256), 0, s, (const float*)x, rows, (int)K, rs);
+    hipLaunchKernelGGL((k_gq_rowscale<float, PASS>), grid, dim3(256), 0, s, (const float*)x, rows, (int)K, rs);
   return rs;
 }
 
@@ -793,7 +797,7 @@ extern "C" int keep_vq_gemm(const void* x, int x_dtype, int64_t rows, const void
   hipStream_t s = (hipStream_t)stream;
   GQArgs a{};
   a.x = x; a.xdt = x_dtype; a.x_rows = rows;
-  a.rs = factors ? gq_rowscale(x, x_dtype, rows, K, workspace, s) : nullptr;
+  a.rs = factors ? gq_rowscale<true>(x, x_dtype, rows, K, workspace, s) : nullptr;
   a.c0 = a.c1 = (const uint16_t*)codes; a.s0 = a.s1 = scales; a.sdt = scale_dtype;
   a.tq = code_bits == 16 ? (const char*)tables + TQ_OFFSET : (const char*)tables;
   a.n_tiles = (rows + GQ_M - 1) / GQ_M; a.routes = rows;

@@ -314,3 +314,44 @@ def test_empty_tiles_of_a_plan_change_nothing(tail, gap):
     parts = [[t[:2], hole, t[2:n]] if gap else [t[:n]] for t in (te, to, tc)]
     got = gemm(*(torch.cat(p + [hole.repeat(tail)]) for p in parts))
     assert not torch.isnan(want).any() and torch.equal(got, want)
+
+
+def _same_values(got, want, tol):
+    """NaN and infinities where the float64 product has them, finite values within tol of their row's largest."""
+    got = got.double().cpu().numpy()
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    inf = np.isinf(want)
+    np.testing.assert_array_equal(np.isinf(got), inf)
+    np.testing.assert_array_equal(got[inf], want[inf])
+    fin = np.where(np.isfinite(want), want, 0)
+    assert (np.abs(np.where(np.isfinite(want), got, 0) - fin) <= tol * np.abs(fin).max(-1, keepdims=True)).all()
+
+
+@pytest.mark.parametrize("code_bits", [8, 16])
+@pytest.mark.parametrize("xdt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M, N, K, G", [(70, 1040, 384, 3), (64, 1024, 512, 1)])
+def test_one_matrix_gemm_non_finite_rows(dev, code_bits, xdt, M, N, K, G):
+    """vq_qmm on the GEMM with infinities and NaN in its rows: the plain
+    product's, and where the mat-vec has an infinity, that infinity."""
+    rng = np.random.default_rng(M)
+    codes = rng.integers(0, 1 << code_bits, (N, K // 8)).astype(np.uint8 if code_bits == 8 else np.uint16)
+    scales = np.exp(rng.normal(0, 0.3, (N, G))).astype(np.float16)
+    x = torch.from_numpy(rng.standard_normal((M, K)).astype(np.float32)).to(dev).to(xdt)
+    inf, nan = float("inf"), float("nan")
+    for r, vals in {1: {5: inf}, 2: {K - 1: -inf}, 3: {7: inf, 90: -inf}, 4: {9: nan}, 5: {2: inf, 3: inf},
+                    M - 1: {0: inf, 1: nan}}.items():
+        for i, v in vals.items():
+            x[r, i] = v
+    x[6] = inf
+    kw = dict(input_dims=K, output_dims=N, group_size=K // G, code_bits=code_bits)
+    c, s, cb = _t(codes, dev), _t(scales, dev), kops._default_codebook(code_bits, dev)
+    assert M * N >= kops.MATRIX_GEMM_CELLS
+    y = kops.vq_qmm(x, c, s, in_dim=K, out_dim=N, group_size=K // G, code_bits=code_bits)
+    dense = (e8p.decode_e8_1bit(codes) if code_bits == 8 else e8p.decode_e8p(codes)).astype(np.float64)
+    dense = dense.reshape(N, K) * np.repeat(scales.astype(np.float64), K // G, -1)
+    with np.errstate(invalid="ignore"):
+        want = np.stack([(dense * r).sum(1) for r in x.double().cpu().numpy()])
+    assert code_bits == 8 or np.isinf(want[[1, 2]]).all()
+    _same_values(y, want, TOL + 2.0 ** -7)
+    old = kops.routed_matvec(x, c.reshape(1, N, -1), s.reshape(1, N, -1), cb, None, routes=M, **kw)
+    assert torch.equal(y[torch.isinf(old)], old[torch.isinf(old)])

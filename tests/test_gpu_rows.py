@@ -122,3 +122,28 @@ def test_rows_through_the_operators(dev):
         torch.cuda.synchronize()
         for n in calls:
             assert torch.equal(held[n], eager[n]), n
+
+
+@pytest.mark.parametrize("bits, xdt", [(8, torch.float16), (8, torch.bfloat16), (16, torch.float16)])
+def test_rows_non_finite_rows(dev, bits, xdt):
+    """Infinities and NaN in a row: the plain product's, for that row's routes alone."""
+    E, N, K, G, T, k = 3, 72, 1024, 2, 9, 2
+    codes, scales, dense = _make(E, N, K, G, bits, seed=bits)
+    rng = np.random.default_rng(7)
+    x = torch.from_numpy(rng.standard_normal((T, K)).astype(np.float32)).to(dev).to(xdt)
+    inf = float("inf")
+    for r, vals in {1: {5: inf}, 2: {K - 1: -inf}, 3: {7: inf, 90: -inf}, 4: {9: float("nan")}, 8: {700: inf}}.items():
+        for i, v in vals.items():
+            x[r, i] = v
+    rhs = rng.integers(0, E, T * k).astype(np.int32)
+    y = kops.rows_matvec(x, _t(codes, dev), _t(scales, dev), kops._default_codebook(bits, dev), _t(rhs, dev), x_div=k,
+                         grouped=True, input_dims=K, output_dims=N, group_size=K // G, code_bits=bits)
+    xd = x.double().cpu().numpy()
+    with np.errstate(invalid="ignore"):
+        want = np.stack([(dense[e] * xd[i // k]).sum(1) for i, e in enumerate(rhs)])
+    got = y.double().cpu().numpy()
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    np.testing.assert_array_equal(np.isinf(got), np.isinf(want))
+    np.testing.assert_array_equal(got[np.isinf(want)], want[np.isinf(want)])
+    good = np.isfinite(want).all(1)
+    _check(got[good], want[good], xdt)
