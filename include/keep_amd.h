@@ -410,9 +410,11 @@ int keep_moe_tiles_layer(const float* logits, const float* bias_served, const fl
                          int out_dtype, void* stream);
 
 /* The same few-token layer for hidden sizes up to 8192 (H a multiple of 256;
- * every other limit, the workspace and the arithmetic as keep_moe_tiles /
+ * every other limit and the workspace as keep_moe_tiles /
  * keep_moe_tiles_layer): from 17 K slices on, each gate/up wave takes one or
- * two projections of a second slice. */
+ * two projections of a second slice, x and h enter as four int8 terms (to 2^-27
+ * of their slice's largest value; two for h in keep_moe_tiles), and an infinity
+ * in x or h gives what keep_moe_decode's fp32 sums give. */
 int keep_moe_wide_supported(int64_t T, int64_t num_experts, int64_t H, int64_t I, int64_t k, int64_t group_size_h,
                             int64_t group_size_i);
 int keep_moe_wide(const void* x, int x_dtype, int64_t T, int64_t H, int64_t I, const int32_t* idx, const float* w,

@@ -11,7 +11,7 @@
 // workspace):
 //  1. k_q8_xterms: every token's int8 activation terms per 256-wide K slice
 //     (three terms under a per-slice power of two, as the one-token layer
-//     builds them) and the slice scales;
+//     builds them; four beyond 4096 hidden values) and the slice scales;
 //  2. keep_route_plan: stable sort of the routes by expert, tile descriptors;
 //  3. k_moeq_gateup_tiles: persistent, one block per CU. A unit is one tile x
 //     16 rows of gate and up; 16 waves each own a K slice. Each code load is
@@ -49,8 +49,8 @@ namespace keep {
 constexpr int MT_TILE = 4;  // routes per tile: one MFMA chain serves them all in either kernel
 
 struct MTArgs {
-  const uint4* xt;     // [T][S][3][16] 16-byte slots of int8 terms
-  const float* xinv;   // [T][S] 1 / (4 s)
+  const uint4* xt;     // [T][S][mt_terms(H)][16] 16-byte slots of int8 terms
+  const float* xinv;   // [T][S] 1 / (4 s), for four terms 1 / (512 s) (mt_dot4)
   const int32_t *order, *te, *to, *tc, *ntiles;
   int32_t k, E, H, I, S;
   const uint16_t *gc, *uc, *dc;
@@ -68,8 +68,12 @@ struct MTArgs {
 
 constexpr int MT_MAX_H = 4096, MT_WIDE_MAX_H = 8192;  // one K slice per gate/up wave; two (the WIDE kernel)
 
-// Token t, K slice s (one wave): the three int8 terms of x[t] * s_slice over
-// the slice's 256 values in the A-slot layout of q8_aword, and 1 / (4 s_slice).
+// Terms per x value: three, or beyond MT_MAX_H four (to 2^-27 of the slice's max,
+// where the packed-table kernels' fp32 sums took x as it is).
+__host__ __device__ constexpr int mt_terms(int64_t H) { return H > MT_MAX_H ? 4 : 3; }
+
+// Token t, K slice s (one wave): the int8 terms of x[t] * s_slice over the
+// slice's 256 values in the A-slot layout of q8_aword, and 1 / (4 s_slice).
 // Beyond MT_MAX_H a slice with infinities (and no NaN) takes the infinities'
 // signs for its terms and an infinite factor: a gate or up sum it enters is
 // infinite, of the right sign for one infinity, so that the token's output is
@@ -90,12 +94,14 @@ __device__ __forceinline__ void mt_xterms(const void* x, int H, uint4* xt, float
 #pragma unroll
     for (int i = 0; i < 4; ++i) v[i] = fabsf(v[i]) == mx ? copysignf(1.f, v[i]) : 0.f;
   }
-  uint32_t tw[3];
-  q8_terms<3>(v, sc, tw);
-  uint32_t* base = (uint32_t*)(xt + ((size_t)t * S + s) * 3 * 16);
+  const int nt = mt_terms(H);
+  uint32_t tw[4];
+  q8_terms<4>(v, sc, tw);
+  uint32_t* base = (uint32_t*)(xt + ((size_t)t * S + s) * nt * 16);
 #pragma unroll
-  for (int n = 0; n < 3; ++n) base[q8_aword((uint32_t)n, lane >> 1, lane & 1)] = tw[n];
-  if (lane == 0) xinv[(size_t)t * S + s] = inv4s;
+  for (int n = 0; n < 4; ++n)
+    if (n < nt) base[q8_aword((uint32_t)n, lane >> 1, lane & 1)] = tw[n];
+  if (lane == 0) xinv[(size_t)t * S + s] = H > MT_MAX_H ? inv4s * 0.0078125f : inv4s;  // four terms: mt_dot4's 128
 }
 
 // Block (t, b), wave w: token t's terms of slice 16 b + w.
@@ -305,6 +311,12 @@ __device__ __forceinline__ int mt_route_of_lanes(int rr, uint32_t i) {
   return __builtin_amdgcn_ds_bpermute((int)(i << 2), rr);
 }
 
+// 128 times a route's dot from the sums of its four terms (each below 2^18: a
+// pair is exact in 32 bits).
+__device__ __forceinline__ float mt_dot4(q8v4 acc) {
+  return fmaf((float)((acc[2] << 7) + acc[3]), 0.00006103515625f, (float)((acc[0] << 7) + acc[1]));
+}
+
 // Gate/up: a unit is 16 rows of gate and of up (two code loads per wave, 32
 // KiB per block). One MFMA chain per projection serves all the tile's
 // routes: A row 4i + t is term t of route i's token (t < 3; row 4i + 3 is
@@ -314,8 +326,8 @@ __device__ __forceinline__ int mt_route_of_lanes(int rr, uint32_t i) {
 // set, slice 16 + wv, or where that set holds at most 8 slices one projection
 // of slice 16 + wv % 8, so that all 16 waves share it. A unit's two sets take
 // the place of two units in flight (the same bytes), and their dots are added
-// before the cross-wave sum. 4 bf16 tokens, top-8 of 128 experts of 7168 x
-// 2048, groups of 512: 85 us per layer against 286 on the packed-table
+// before the cross-wave sum. x enters in four terms, row 4i + 3 the fourth. 4 bf16 tokens, top-8 of 128 experts of 7168 x
+// 2048, groups of 512: 87 us per layer against 286 on the packed-table
 // mat-vecs, which decode every route's codes on the VALU. Infinities: mt_xterms.
 template <bool XBF, int RPER, bool WIDE = false>
 __global__ __launch_bounds__(1024) void k_moeq_gateup_tiles(MTArgs a, MTRoute p) {
@@ -420,7 +432,7 @@ __global__ __launch_bounds__(1024) void k_moeq_gateup_tiles(MTArgs a, MTRoute p)
   uint4 araw[4];
   auto issue_a = [&](int route_a, int route_d, int sl, float& inv) {  // the routes of A row j and of this lane's D rows
     const int tok_a = route_a / a.k, tok_d = route_d / a.k;
-    const uint4* asrc = a.xt + ((size_t)tok_a * a.S + sl) * 48 + min(j & 3u, 2u) * 16 + g * 4;
+    const uint4* asrc = a.xt + ((size_t)tok_a * a.S + sl) * (WIDE ? 64 : 48) + (WIDE ? j & 3u : min(j & 3u, 2u)) * 16 + g * 4;
 #pragma unroll
     for (int m = 0; m < 4; ++m) araw[m] = ldg16_q(asrc + m);
     inv = a.xinv[(size_t)tok_d * a.S + sl];
@@ -485,7 +497,7 @@ __global__ __launch_bounds__(1024) void k_moeq_gateup_tiles(MTArgs a, MTRoute p)
   auto build_a = [&](q8v4 (&A)[4]) {
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
-      const bool z = (j & 3u) == 3u;
+      const bool z = !WIDE && (j & 3u) == 3u;
       A[m] = q8v4{z ? 0 : (int)araw[m].x, z ? 0 : (int)araw[m].y, z ? 0 : (int)araw[m].z, z ? 0 : (int)araw[m].w};
     }
   };
@@ -593,7 +605,7 @@ __global__ __launch_bounds__(1024) void k_moeq_gateup_tiles(MTArgs a, MTRoute p)
       q8v4 acc = {0, 0, 0, 0};
 #pragma unroll
       for (int m = 0; m < 4; ++m) acc = mfma_i8(A[m], B[m], acc);
-      d[t] = (((float)acc[0] + (float)acc[1] * 0.0078125f) + (float)acc[2] * 0.00006103515625f) * inv;
+      d[t] = mt_dot4(acc) * inv;
       if (!g1) d[t] *= scl[t];
     }
 #pragma unroll
@@ -611,7 +623,7 @@ __global__ __launch_bounds__(1024) void k_moeq_gateup_tiles(MTArgs a, MTRoute p)
         q8v4 acc = {0, 0, 0, 0};
 #pragma unroll
         for (int m = 0; m < 4; ++m) acc = mfma_i8(A1[WIDE ? m : 0], B[m], acc);
-        e[t] = (((float)acc[0] + (float)acc[1] * 0.0078125f) + (float)acc[2] * 0.00006103515625f) * inv1 * sc;
+        e[t] = mt_dot4(acc) * inv1 * sc;
         asm volatile("" : "+v"(e[t]));  // done with b1 before it is reloaded
       }
       d[0] += hi ? 0.f : e[0];
@@ -677,17 +689,17 @@ __global__ __launch_bounds__(1024) void k_moeq_gateup_tiles(MTArgs a, MTRoute p)
 // tile's routes (rows 2r, 2r + 1; rows past them zero), built in LDS by the
 // slice's first wave when the block enters a segment and read by both; route
 // r's dot is D rows 2r, 2r + 1. The partial sums are kept per slice and row
-// tile and summed over the slices in slice order. THREE (hidden sizes beyond
-// 4096): three terms per route, rows 4r .. 4r + 2 as in gate/up, the same
-// MFMAs; h then keeps all but 2^-20 of its slice's max, below its bf16
-// rounding, as the fp32 mat-vecs these shapes used before kept it. (A sum over
+// tile and summed over the slices in slice order. FOUR (hidden sizes beyond
+// 4096): four terms per route, rows 4r .. 4r + 3, the same MFMAs; h then keeps
+// all but 2^-27 of its slice's max, as good as the fp32 mat-vecs these shapes
+// used before kept it. (A sum over
 // an infinity of h comes out NaN here; the combine forms it again.)
-template <bool THREE>
+template <bool FOUR>
 __global__ __launch_bounds__(1024) void k_moeq_down_tiles(MTArgs a) {
-  constexpr int NT = THREE ? 3 : 2;  // terms per route
+  constexpr int NT = FOUR ? 4 : 2;  // terms per route
   constexpr int RT = 4;   // row tiles per unit
   constexpr int RW = 2;   // row tiles per wave
-  constexpr int SEG = 48;  // units per segment (y staging capacity)
+  constexpr int SEG = FOUR ? 40 : 48;  // units per segment (y staging capacity: the LDS the A terms leave)
   __shared__ uint4 tqs[TQR_BYTES / 16];
   __shared__ uint4 ash[8][NT * MT_TILE * 16];        // [slice][(route * NT + term) * 16 + slot]
   __shared__ float s_inv[8][MT_TILE];
@@ -783,11 +795,11 @@ __global__ __launch_bounds__(1024) void k_moeq_down_tiles(MTArgs a) {
         float sc, inv4s;
         q8_scale(__uint_as_float(__builtin_amdgcn_readfirstlane(rt_wave_u32<true>(rt_abs_bits4(v)))), sc, inv4s);
         uint32_t tw[NT];
-        if constexpr (THREE) q8_terms<3>(v, sc, tw);
+        if constexpr (FOUR) q8_terms<4>(v, sc, tw);
         else q8_digits2(v, sc, tw);
 #pragma unroll
         for (int n = 0; n < NT; ++n) aw[q8_aword((uint32_t)(NT * i + n), lane >> 1, lane & 1)] = tw[n];
-        if (lane == 0) s_inv[sl][i] = inv4s;
+        if (lane == 0) s_inv[sl][i] = FOUR ? inv4s * 0.0078125f : inv4s;
       }
     }
   };
@@ -797,16 +809,16 @@ __global__ __launch_bounds__(1024) void k_moeq_down_tiles(MTArgs a) {
       // reload from scratch waits for every code load in flight
       uint32_t g = lane >> 4;
       asm volatile("" : "+v"(g));
-      const uint32_t arow = THREE ? (j >> 2) * 3u + min(j & 3u, 2u) : j & (2 * MT_TILE - 1);
+      const uint32_t arow = FOUR ? j : j & (2 * MT_TILE - 1);
       const q8v4* as = (const q8v4*)ash[sl] + arow * 16 + g * 4;
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
         const q8v4 v = as[m];
-        const bool z = THREE ? (j & 3u) == 3u : (int)j >= 2 * cur_nr;  // rows of no term, or past the tile's routes
+        const bool z = !FOUR && (int)j >= 2 * cur_nr;  // rows past the tile's routes
         A[m] = q8v4{z ? 0 : v[0], z ? 0 : v[1], z ? 0 : v[2], z ? 0 : v[3]};
       }
 #pragma unroll
-      for (int h2 = 0; h2 < 2; ++h2) inv[h2] = s_inv[sl][THREE ? (int)g : min(2 * (int)g + h2, MT_TILE - 1)];
+      for (int h2 = 0; h2 < 2; ++h2) inv[h2] = s_inv[sl][FOUR ? (int)g : min(2 * (int)g + h2, MT_TILE - 1)];
     }
   };
   // the segment's staged y rows to their routes' rows
@@ -853,11 +865,8 @@ __global__ __launch_bounds__(1024) void k_moeq_down_tiles(MTArgs a) {
         q8v4 acc = {0, 0, 0, 0};
 #pragma unroll
         for (int m = 0; m < 4; ++m) acc = mfma_i8(A[m], B[rt][m], acc);
-        if constexpr (THREE) {  // route g: rows 4g .. 4g + 2 = lanes 16 g + j, registers 0 .. 2
-          if ((int)g < cur_nr) {
-            const float d = ((float)acc[0] + (float)acc[1] * 0.0078125f) + (float)acc[2] * 0.00006103515625f;
-            red[par][sl][hf * RW + rt][g][j] = d * inv[0] * scl[rt];
-          }
+        if constexpr (FOUR) {  // route g: rows 4g .. 4g + 3 = lanes 16 g + j, registers 0 .. 3
+          if ((int)g < cur_nr) red[par][sl][hf * RW + rt][g][j] = mt_dot4(acc) * inv[0] * scl[rt];
           continue;
         }
         // route r: rows 2r, 2r + 1 = lanes 16 (r / 2) + j, registers 2 (r % 2), 2 (r % 2) + 1
@@ -1002,7 +1011,7 @@ static MTWorkspace mt_layout(int64_t T, int64_t k, int64_t E, int64_t H) {
   const int64_t R = T * k, S = H / 256;
   w.max_tiles = (R + MT_TILE - 1) / MT_TILE + E;
   size_t o = 0;
-  w.xt = o; o = mt_align(o + (size_t)T * S * 3 * 256);
+  w.xt = o; o = mt_align(o + (size_t)T * S * mt_terms(H) * 256);
   w.xinv = o; o = mt_align(o + (size_t)T * S * 4);
   w.order = o; o = mt_align(o + (size_t)R * 4);
   w.inverse = o; o = mt_align(o + (size_t)R * 4);

@@ -497,3 +497,39 @@ def test_wide_non_finite_h(dev):
     assert np.isinf(want).any() and np.isnan(want).any() and np.isfinite(want).all(1).any()
     assert torch.isinf(packed).any()
     _same_values(out, want, packed)
+
+
+@pytest.mark.parametrize("amp", [1.0, 512.0, 30000.0])
+@pytest.mark.parametrize("xdt", [torch.float16, torch.bfloat16])
+def test_wide_keeps_the_bits_of_x_and_h(dev, xdt, amp):
+    """One large value in every slice of 256: the others lose no more than in
+    the packed-table kernels' fp32 sums. h against the float64 layer's rounded
+    to bf16, by the share of values off by a rounding; down against the float64
+    product of the h it was given."""
+    E, H, I, k, T = 4, 7168, 1024, 2, 8
+    pool = [(p.codes, p.scales * 0.02) for p in (synth.projection(E, I, H, group_size=512, seed=150, device=dev),
+                                                 synth.projection(E, I, H, group_size=512, seed=151, device=dev),
+                                                 synth.projection(E, H, I, group_size=512, seed=152, device=dev))]
+    g = torch.Generator().manual_seed(153)
+    x = torch.randn((T, H), generator=g)
+    x.view(T, -1, 256)[:, :, 3] *= amp
+    x = x.clamp(-60000, 60000).to(dev).to(xdt)
+    idx = torch.stack([torch.randperm(E, generator=g)[:k] for _ in range(T)]).int().to(dev)
+    w = torch.rand((T, k), generator=g).to(dev)
+    dec = [torch.from_numpy(e8p.decode_e8p(c.cpu().numpy().view(np.uint16)).astype(np.float64)).to(dev).reshape(
+        c.shape[0], c.shape[1], -1) * s.double().repeat_interleave(512, -1) for c, s in pool]
+    e = idx.reshape(-1).tolist()
+    xr = x.double().repeat_interleave(k, 0)
+    gate, up = (torch.stack([dec[n][j] @ xr[r] for r, j in enumerate(e)]) for n in (0, 1))
+    want_h = (gate / (1 + torch.exp(-gate)) * up).bfloat16()
+    off, err = [], []
+    for prepared in (True, False):
+        h = torch.zeros((T * k, I), dtype=torch.bfloat16, device=dev)
+        out = keep_amd.moe_decode(x, idx, w, *pool, h_work=h.view(-1), prepared=prepared).double()
+        off.append(float((h != want_h).double().mean()))
+        want = torch.stack([dec[2][j] @ h[r].double() for r, j in enumerate(e)]).reshape(T, k, H)
+        want = (want * w.double()[..., None]).sum(1)
+        err.append(float((out - want).norm() / want.norm()))
+    print(f"{xdt} {amp}: h off {off}, down {err}")
+    assert off[0] <= 1.5 * off[1] + 2e-4, "values of h further off than the packed kernels'"
+    assert err[0] <= 1.2 * err[1], "down further off than the packed kernels'"
