@@ -258,8 +258,11 @@ def _index_tensor(ix, device) -> torch.Tensor:
 
 
 def _stream(device) -> int:
-    """The current stream's handle, without building a ``torch.cuda.Stream`` (0.1 us against 1.9)."""
+    """The current stream's handle, without building a ``torch.cuda.Stream`` (0.4 us against 1.9). Every launch asks
+    for it, so a tensor that the GPU does not own is refused here, as ``torch.cuda.current_stream`` refuses it."""
 
+    if device.type != "cuda":
+        raise ValueError(f"Expected a cuda device, but got: {device}")
     index = device.index
     return _raw_stream(torch.cuda.current_device() if index is None else index)
 
