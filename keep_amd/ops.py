@@ -118,26 +118,32 @@ _PREPARED: dict[tuple[int, str], tuple[torch.Tensor, torch.Tensor]] = {}
 def prepared_table(codebook: torch.Tensor) -> torch.Tensor:
     """The prepared E8P table of ``codebook`` for the matrix-core kernels
     (``keep_e8p_prepare``: T and M of the int8 decode, a check word and the
-    64 KiB LDS image, ``keep_e8p_prepared_bytes()`` bytes), cached per codebook tensor."""
+    64 KiB LDS image, ``keep_e8p_prepared_bytes()`` bytes), cached per codebook tensor
+    (one built under graph capture belongs to that graph and is not)."""
 
-    key = (codebook.data_ptr(), str(codebook.device))
-    hit = _PREPARED.get(key)
-    if hit is not None and hit[0] is codebook:
-        return hit[1]
+    hit = _kept_table(codebook)
+    if hit is not None:
+        return hit
     nbytes = _lib.load().keep_e8p_prepared_bytes()
     out = torch.empty(nbytes, dtype=torch.uint8, device=codebook.device)
     _lib.call("keep_e8p_prepare", codebook.data_ptr(), out.data_ptr(), _stream(codebook.device))
-    if not torch.cuda.is_current_stream_capturing():
-        torch.cuda.current_stream(codebook.device).synchronize()  # once: any stream may read it from here on
-    _PREPARED[key] = (codebook, out)
+    if torch.cuda.is_current_stream_capturing():
+        return out  # filled by this graph's replays only: not kept for other calls
+    torch.cuda.current_stream(codebook.device).synchronize()  # once: any stream may read it from here on
+    _PREPARED[(codebook.data_ptr(), str(codebook.device))] = (codebook, out)
     return out
 
 
-def _may_prepare(codebook: torch.Tensor) -> bool:
-    """Whether ``prepared_table`` can serve a call that needs not have it: a table first built under graph
-    capture would be filled by that graph's replays only."""
+def _kept_table(codebook: torch.Tensor) -> torch.Tensor | None:
+    hit = _PREPARED.get((codebook.data_ptr(), str(codebook.device)))
+    return hit[1] if hit is not None and hit[0] is codebook else None
 
-    return (codebook.data_ptr(), str(codebook.device)) in _PREPARED or not torch.cuda.is_current_stream_capturing()
+
+def _may_prepare(codebook: torch.Tensor) -> bool:
+    """Whether ``prepared_table`` can serve a call that needs not have it: under graph capture only a table
+    that is there already (building one would be a launch of every replay)."""
+
+    return not torch.cuda.is_current_stream_capturing() or _kept_table(codebook) is not None
 
 
 def half2_pairs(grid: np.ndarray) -> np.ndarray:

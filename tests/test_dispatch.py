@@ -41,3 +41,20 @@ def test_cpu_activations_are_refused_before_any_launch(launches, call):
         else:
             keep_amd.moe_layer(x, z, *pool, k=2)
     assert launches == []
+
+
+def test_a_table_prepared_under_capture_is_not_kept(launches, monkeypatch):
+    """It holds nothing before that graph's first replay: the next eager call builds its own, once."""
+    cb = torch.from_numpy(ops.e8p_packed_abs_grid().view("int32"))
+    monkeypatch.setattr(ops, "_stream", lambda device: 0)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device: type("S", (), {"synchronize": lambda self: None})())
+    captured = ops.prepared_table(cb)
+    assert launches == ["keep_e8p_prepare"] and not ops._may_prepare(cb)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    assert ops._may_prepare(cb)
+    eager = ops.prepared_table(cb)
+    assert eager is not captured and launches == ["keep_e8p_prepare"] * 2
+    assert ops.prepared_table(cb) is eager
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    assert ops._may_prepare(cb) and ops.prepared_table(cb) is eager
+    assert len(launches) == 2

@@ -533,3 +533,25 @@ def test_wide_keeps_the_bits_of_x_and_h(dev, xdt, amp):
     print(f"{xdt} {amp}: h off {off}, down {err}")
     assert off[0] <= 1.5 * off[1] + 2e-4, "values of h further off than the packed kernels'"
     assert err[0] <= 1.2 * err[1], "down further off than the packed kernels'"
+
+
+def test_table_prepared_in_a_graph_serves_that_graph_alone(dev, small_pool):
+    """A layer on a table first seen under capture: an eager call before the
+    first replay prepares its own, and every replay equals it."""
+    E, T, k = 20, 3, 2
+    pool = tuple((p.codes[:E], p.scales[:E]) for p in small_pool)
+    x = synth.rht_activations(T, 1024, seed=160, device=dev)
+    r = keep_amd.router_dual_topk(synth.router_logits(T, E, seed=161, device=dev), k)
+    want = keep_amd.moe_decode(x, r.idx, r.weight, *pool)  # the default table
+    cb = keep_amd.ops._default_codebook(16, dev).clone()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=torch.cuda.Stream()):
+        held = keep_amd.moe_decode(x, r.idx, r.weight, *pool, codebook=cb)
+    assert torch.equal(keep_amd.moe_decode(x, r.idx, r.weight, *pool, codebook=cb), want)
+    for _ in range(3):
+        held.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(held, want)
+        assert torch.equal(keep_amd.moe_decode(x, r.idx, r.weight, *pool, codebook=cb), want)
