@@ -53,6 +53,8 @@ ROWS_PER_EXPERT = {8: 128, 16: 12}
 # single-row calls then agree bit for bit): 4096 -> 2048, 8 rows x top-6 of 256, 24 against 57 us, one row 10.9 / 11.6.
 ROWS_MATRIX = 1 << 21
 PLANNED_ROUTES = 128  # routes keep_vq_rows groups without a route plan
+# Experts a route plan holds. Routed 8-bit and direct calls beyond stay on the mat-vec, which has no limit.
+PLAN_EXPERTS = 1024
 _VERIFY_DEFAULT_M_ROWS = 4
 VERIFY_MROWS_VALUES = (1, 2, 3, 4, 8)
 
@@ -822,7 +824,7 @@ def gather_vqmm(x, codes, scales, codebook, rhs_indices, *, lhs_indices=None, in
         return torch.zeros(out_shape, dtype=od, device=device)
 
     eligible = gemm_eligible(code_bits=code_bits, x_dtype=xt.dtype, input_dims=input_dims, group_size=group_size) \
-        and (code_bits == 16 or _gemm_pointers_ok(c, s, cb, 8))
+        and (code_bits == 16 or (E <= PLAN_EXPERTS and _gemm_pointers_ok(c, s, cb, 8)))
     strategy = route_strategy
     if strategy == "auto":
         strategy = "sorted_tiled" if eligible and (sorted_indices or R >= GEMM_ROUTE_THRESHOLD) else "direct"
@@ -830,7 +832,8 @@ def gather_vqmm(x, codes, scales, codebook, rhs_indices, *, lhs_indices=None, in
            input_dims=int(input_dims), output_dims=int(output_dims), group_size=int(group_size),
            code_bits=int(code_bits), strategy=strategy,
            implementation="mfma_grouped_gemm" if strategy == "sorted_tiled" and eligible else "hip_matvec")
-    few = rows_eligible(xt, c, s, cb, code_bits=code_bits, input_dims=input_dims, group_size=group_size)
+    few = E <= PLAN_EXPERTS and rows_eligible(xt, c, s, cb, code_bits=code_bits, input_dims=input_dims,
+                                              group_size=group_size)
     if strategy in ("direct", "per_route_decoded"):
         if output_dims * input_dims >= ROWS_MATRIX and few:
             y = rows_matvec(xt, c, s, cb, flat_rhs, lhs=lhs, x_div=x_div, grouped=R > x_div, input_dims=input_dims,
@@ -905,12 +908,13 @@ def gather_vqmm_sorted_routes(x, codes, scales, codebook, sorted_rhs, sorted_lhs
     skip_gather = x_pre_sorted and xt.shape[0] == R
     use_lhs = None if skip_gather else lhs
     eligible = gemm_eligible(code_bits=code_bits, x_dtype=xt.dtype, input_dims=input_dims, group_size=group_size)
-    if (code_bits == 8 and GEMM_ROUTE_THRESHOLD <= R <= ROWS_PER_EXPERT[8] * E
+    planned = code_bits == 8 and R >= GEMM_ROUTE_THRESHOLD and E <= PLAN_EXPERTS
+    if (planned and R <= ROWS_PER_EXPERT[8] * E
             and rows_eligible(xt, c, s, cb, code_bits=8, input_dims=input_dims, group_size=group_size)):
         pos = torch.arange(R, dtype=torch.int32, device=device) if use_lhs is None else use_lhs
         return rows_matvec(xt, c, s, cb, rhs, lhs=pos, grouped=True, input_dims=input_dims, output_dims=output_dims,
                            group_size=group_size, code_bits=8)
-    if eligible and code_bits == 8 and R >= GEMM_ROUTE_THRESHOLD and _gemm_pointers_ok(c, s, cb, 8):
+    if planned and eligible and _gemm_pointers_ok(c, s, cb, 8):
         # a plan of its own, rows back at their positions: 8-bit calls never had to be sorted, nor their tiles right
         order, _, _, _, te, to, tc, _ = route_plan(rhs, E, GEMM_ROUTE_TILE)
         return grouped_gemm_e8(xt, c, s, cb, (te, to, tc), lhs=order if use_lhs is None else use_lhs[order.long()],
@@ -998,7 +1002,7 @@ def gather_vqmm_verify_rows(x, codes, scales, codebook, rhs_indices, *, lhs_indi
            input_dims=int(input_dims), output_dims=int(output_dims), group_size=int(group_size),
            code_bits=code_bits, strategy=f"verify_{grouping}", implementation="hip_matvec")
     x_div = top_k or 1
-    if output_dims * input_dims >= ROWS_MATRIX and rows_eligible(
+    if output_dims * input_dims >= ROWS_MATRIX and E <= PLAN_EXPERTS and rows_eligible(
             xt, c, s, cb, code_bits=code_bits, input_dims=input_dims, group_size=group_size):
         y = rows_matvec(xt, c, s, cb, flat_rhs, lhs=flat_lhs, x_div=x_div, grouped=grouping == "expert",
                         input_dims=input_dims, output_dims=output_dims, group_size=group_size, code_bits=code_bits)

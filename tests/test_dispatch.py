@@ -1,6 +1,8 @@
 """Which entry points the operators reach, on the CPU with the launches
 recorded instead of made: no launch on tensors the GPU does not own."""
 
+from types import SimpleNamespace
+
 import pytest
 import torch
 
@@ -13,7 +15,14 @@ def launches(monkeypatch):
     """The entry points called, none of them run; a GPU's stream and capture state stubbed."""
     calls, real = [], _lib.call
     host = ("keep_e8p_packed_abs_grid", "keep_e8_1bit_packed")  # tables built on the host
-    monkeypatch.setattr(_lib, "call", lambda name, *a: real(name, *a) if name in host else calls.append(name))
+
+    def call(name, *args):
+        if name in host:
+            return real(name, *args)
+        calls.append(name)
+        if name == "keep_route_plan" and args[2] > 1024:
+            raise ValueError("E must be in 1..1024")  # the library's check
+    monkeypatch.setattr(_lib, "call", call)
     monkeypatch.setattr(ops, "_raw_stream", lambda index: 0)
     monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
@@ -22,7 +31,8 @@ def launches(monkeypatch):
 
 
 def _moe(T, H=512, I=256, E=4, k=2):
-    codes = lambda n, K: (torch.zeros((E, n, K // 8), dtype=torch.int16), torch.ones((E, n, 1), dtype=torch.float16))  # noqa: E731
+    def codes(n, K):
+        return torch.zeros((E, n, K // 8), dtype=torch.int16), torch.ones((E, n, 1), dtype=torch.float16)
     return (torch.zeros((T, H), dtype=torch.float16), torch.zeros((T, E)), (codes(I, H), codes(I, H), codes(H, I)),
             torch.zeros((T, k), dtype=torch.int32), torch.ones((T, k)))
 
@@ -47,7 +57,7 @@ def test_a_table_prepared_under_capture_is_not_kept(launches, monkeypatch):
     """It holds nothing before that graph's first replay: the next eager call builds its own, once."""
     cb = torch.from_numpy(ops.e8p_packed_abs_grid().view("int32"))
     monkeypatch.setattr(ops, "_stream", lambda device: 0)
-    monkeypatch.setattr(torch.cuda, "current_stream", lambda device: type("S", (), {"synchronize": lambda self: None})())
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device: SimpleNamespace(synchronize=lambda: None))
     captured = ops.prepared_table(cb)
     assert launches == ["keep_e8p_prepare"] and not ops._may_prepare(cb)
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
@@ -58,3 +68,49 @@ def test_a_table_prepared_under_capture_is_not_kept(launches, monkeypatch):
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
     assert ops._may_prepare(cb) and ops.prepared_table(cb) is eager
     assert len(launches) == 2
+
+
+@pytest.fixture
+def routed(launches, monkeypatch):
+    """The operators on CPU tensors taken for the GPU's; the entry points that one call reached."""
+    monkeypatch.setattr(ops, "_device_of", lambda *ts: torch.device("cpu"))
+    monkeypatch.setattr(ops, "_stream", lambda device: 0)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+
+    def run(fn, *args, **kw):
+        launches.clear()
+        fn(*args, **kw)
+        return list(launches)
+    return run
+
+
+def _switch(E, N, K, bits=8, G=1):
+    codes = torch.empty((E, N, K // 8), dtype=torch.uint8 if bits == 8 else torch.int16)  # never read
+    return codes, torch.empty((E, N, G), dtype=torch.float16), dict(input_dims=K, output_dims=N, group_size=K // G)
+
+
+@pytest.mark.parametrize("T", [2, 65])
+def test_more_experts_than_a_plan_holds(routed, T):
+    """Route plans hold 1024 experts. Calls that never needed one are served beyond, by the mat-vec."""
+    N, K, k = 4096, 512, 2
+    x, rhs = torch.empty((T, K), dtype=torch.float16), torch.zeros((T, k), dtype=torch.int32)
+    flat, lhs = rhs.reshape(-1), torch.arange(T * k, dtype=torch.int32) // k
+    for E in (1024, 1025):
+        c, s, kw = _switch(E, N, K)
+        assert N * K >= ops.ROWS_MATRIX
+        got = {
+            "auto": routed(ops.gather_vqmm, x, c, s, None, rhs, code_bits=8, **kw),
+            "direct": routed(ops.gather_vqmm, x, c, s, None, rhs, code_bits=8, route_strategy="direct", **kw),
+            "sorted": routed(ops.gather_vqmm_sorted_routes, x, c, s, None, flat, lhs, code_bits=8, **kw),
+            "flat": routed(ops.gather_vqmm_verify_rows, x, c, s, None, rhs, grouping="flat", **kw),
+        }
+        for name, calls in got.items():
+            if E > 1024:
+                assert calls == ["keep_vq_matvec"], (name, calls)
+            elif name != "sorted" or T * k >= ops.GEMM_ROUTE_THRESHOLD:
+                assert calls[-1] == "keep_vq_rows", (name, calls)
+    # what a plan refused it refuses
+    for fn, over in ((ops.gather_vqmm, dict(code_bits=8, route_strategy="sorted_tiled")),
+                     (ops.gather_vqmm_verify_rows, dict(grouping="expert"))):
+        with pytest.raises(ValueError, match="1024"):
+            routed(fn, x, c, s, None, rhs, **over, **kw)
