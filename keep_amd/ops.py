@@ -25,6 +25,7 @@ from __future__ import annotations
 
 from contextlib import contextmanager
 from contextvars import ContextVar
+from functools import lru_cache
 from typing import Any, Iterator, Literal
 
 import numpy as np
@@ -430,18 +431,22 @@ def matrix_gemm(x: torch.Tensor, codes: torch.Tensor, scales: torch.Tensor, code
     return out
 
 
+@lru_cache(maxsize=1024)
+def _rows_supported(x_dtype: int, code_bits: int, input_dims: int, group_size: int) -> bool:
+    return bool(_lib.load().keep_vq_rows_supported(x_dtype, code_bits, input_dims, group_size))
+
+
 def rows_eligible(x: torch.Tensor, codes: torch.Tensor, scales: torch.Tensor, codebook: torch.Tensor, *,
                   code_bits: int, input_dims: int, group_size: int) -> bool:
-    """Whether ``keep_vq_rows`` serves this call: 8-bit E8 with fp16/bf16 rows, or E8P (default table) with fp16
-    rows; up to 16 K slices of 512 / 256, scale groups of whole slices; aligned pools."""
+    """Whether ``keep_vq_rows`` serves this call: types and sizes (``keep_vq_rows_supported``), x under 2 GiB,
+    aligned pools; for E8P the default table."""
 
-    ck = 512 if code_bits == 8 else 256
-    if (input_dims % ck or input_dims > 16 * ck or group_size % ck or x.numel() >= 1 << 30
+    if (not _rows_supported(_DT.get(x.dtype, -1), code_bits, input_dims, group_size) or x.numel() >= 1 << 30
             or codes.data_ptr() % 16 or scales.data_ptr() % 4 or x.data_ptr() % 16):
         return False
     if code_bits == 8:
-        return x.dtype in (torch.float16, torch.bfloat16) and codebook.data_ptr() % 16 == 0
-    return x.dtype == torch.float16 and codebook is _default_codebook(16, codebook.device) and _may_prepare(codebook)
+        return codebook.data_ptr() % 16 == 0
+    return codebook is _default_codebook(16, codebook.device) and _may_prepare(codebook)
 
 
 def rows_matvec(x: torch.Tensor, codes: torch.Tensor, scales: torch.Tensor, codebook: torch.Tensor,
@@ -774,11 +779,13 @@ def gather_vqmm(x, codes, scales, codebook, rhs_indices, *, lhs_indices=None, in
     Token layout: ``x [T, K]``, ``rhs_indices [T, k]`` -> ``[T, k, N]``.
     Per-route layout: ``lhs_indices`` and ``rhs_indices`` of R routes -> ``[R, N]``.
 
-    ``route_strategy="auto"``: E8P calls with 16-bit activations and at least
-    ``GEMM_ROUTE_THRESHOLD`` routes (or ``sorted_indices``) take
-    ``sorted_tiled`` -- the device route plan plus the MFMA grouped GEMM --
-    everything else takes ``direct``, the wave-per-rows decode mat-vec.
-    ``per_route_decoded`` is the same mat-vec (one launch for all routes).
+    ``route_strategy="auto"``: calls that the MFMA grouped GEMM serves
+    (``gemm_eligible``) with at least ``GEMM_ROUTE_THRESHOLD`` routes (or
+    ``sorted_indices``) take ``sorted_tiled``, a device route plan and that
+    GEMM; everything else takes ``direct``, the wave-per-rows decode mat-vec
+    (``per_route_decoded`` is the same). In either, the matrix-core rows kernel
+    takes the calls it serves (``rows_eligible``) that have few routes per
+    expert (sorted) or a large matrix (direct); the trace names the kernel.
     """
 
     _check_impl(implementation)
@@ -828,24 +835,21 @@ def gather_vqmm(x, codes, scales, codebook, rhs_indices, *, lhs_indices=None, in
     strategy = route_strategy
     if strategy == "auto":
         strategy = "sorted_tiled" if eligible and (sorted_indices or R >= GEMM_ROUTE_THRESHOLD) else "direct"
+    sort = strategy == "sorted_tiled"
+    few = ((R <= ROWS_PER_EXPERT[code_bits] * E if sort else output_dims * input_dims >= ROWS_MATRIX)
+           and E <= PLAN_EXPERTS
+           and rows_eligible(xt, c, s, cb, code_bits=code_bits, input_dims=input_dims, group_size=group_size))
     _trace(token_rows=int(xt.shape[0]), route_count=int(R), has_lhs_indices=lhs_indices is not None,
            input_dims=int(input_dims), output_dims=int(output_dims), group_size=int(group_size),
            code_bits=int(code_bits), strategy=strategy,
-           implementation="mfma_grouped_gemm" if strategy == "sorted_tiled" and eligible else "hip_matvec")
-    few = E <= PLAN_EXPERTS and rows_eligible(xt, c, s, cb, code_bits=code_bits, input_dims=input_dims,
-                                              group_size=group_size)
-    if strategy in ("direct", "per_route_decoded"):
-        if output_dims * input_dims >= ROWS_MATRIX and few:
-            y = rows_matvec(xt, c, s, cb, flat_rhs, lhs=lhs, x_div=x_div, grouped=R > x_div, input_dims=input_dims,
-                            output_dims=output_dims, group_size=group_size, code_bits=code_bits)
-            return y.reshape(out_shape)
+           implementation="mfma_rows" if few else "mfma_grouped_gemm" if sort and eligible else "hip_matvec")
+    if few:
+        y = rows_matvec(xt, c, s, cb, flat_rhs, lhs=lhs, x_div=x_div, grouped=sort or R > x_div,
+                        input_dims=input_dims, output_dims=output_dims, group_size=group_size, code_bits=code_bits)
+        return y.reshape(out_shape)
+    if not sort:
         y = routed_matvec(xt, c, s, cb, flat_rhs, lhs=lhs, x_div=x_div, input_dims=input_dims,
                           output_dims=output_dims, group_size=group_size, code_bits=code_bits)
-        return y.reshape(out_shape)
-    # sorted_tiled
-    if few and R <= ROWS_PER_EXPERT[code_bits] * E:
-        y = rows_matvec(xt, c, s, cb, flat_rhs, lhs=lhs, x_div=x_div, grouped=True, input_dims=input_dims,
-                        output_dims=output_dims, group_size=group_size, code_bits=code_bits)
         return y.reshape(out_shape)
     full_lhs = lhs if lhs is not None else torch.arange(R, dtype=torch.int32, device=device) // x_div
     order, inverse, _, _, te, to, tc, _ = route_plan(flat_rhs, E, GEMM_ROUTE_TILE)
@@ -871,9 +875,11 @@ def gather_vqmm_sorted_routes(x, codes, scales, codebook, sorted_rhs, sorted_lhs
                               projection: str = "auto", validate_indices: bool = False, tile_descriptors=None,
                               x_pre_sorted: bool = False) -> torch.Tensor:
     """Already-sorted routed matmul -> ``[R, N]`` in sorted order
-    (reference ``vq_switch.py:620-913``). E8P with 16-bit activations runs the
-    MFMA grouped GEMM (``tile_descriptors`` or a device route plan of 64-route
-    tiles); other calls run the mat-vec over the sorted routes."""
+    (reference ``vq_switch.py:620-913``). E8P runs the MFMA grouped GEMM
+    (``tile_descriptors`` or a device route plan of 64-route tiles), and so do
+    8-bit codes with fp16 or bf16 rows from ``GEMM_ROUTE_THRESHOLD`` routes on,
+    on a plan of their own (or, few routes per expert, the rows kernel); other
+    calls run the mat-vec over the sorted routes."""
 
     if projection not in ("auto", "gate_up", "down"):
         raise ValueError("projection must be 'auto', 'gate_up', or 'down'")
@@ -952,10 +958,11 @@ def gather_vqmm_verify_rows(x, codes, scales, codebook, rhs_indices, *, lhs_indi
     The code format follows ``codes``' dtype: uint8 codes index a packed 8-bit
     E8 table (the reference kernel's contract, ``gather_vqmm.py:387-388``;
     default ``codebook`` the E8 table), uint16 codes are E8P.
-    ``grouping="flat"``: one launch, every route on the decode mat-vec.
-    ``grouping="expert"``: routes sorted by expert on the device and folded in
-    tiles of up to ``m_rows`` same-expert routes that share every code load;
-    per route bit-identical with ``"flat"``.
+    ``grouping="flat"``: every route by itself; ``grouping="expert"``: routes of
+    one expert folded in tiles that share every code load, per route
+    bit-identical with ``"flat"``. Large matrices that the rows kernel serves
+    (``rows_eligible``) run on it, in tiles of up to 16 routes; the others on
+    the decode mat-vec, by expert in tiles of up to ``m_rows``.
     """
 
     if grouping not in ("expert", "flat"):
@@ -998,12 +1005,13 @@ def gather_vqmm_verify_rows(x, codes, scales, codebook, rhs_indices, *, lhs_indi
         if m_rows not in VERIFY_MROWS_VALUES:
             raise ValueError(f"m_rows must be one of {VERIFY_MROWS_VALUES}")
         mr = int(m_rows)
+    few = output_dims * input_dims >= ROWS_MATRIX and E <= PLAN_EXPERTS and rows_eligible(
+        xt, c, s, cb, code_bits=code_bits, input_dims=input_dims, group_size=group_size)
     _trace(token_rows=int(xt.shape[0]), route_count=int(R), has_lhs_indices=lhs_indices is not None,
            input_dims=int(input_dims), output_dims=int(output_dims), group_size=int(group_size),
-           code_bits=code_bits, strategy=f"verify_{grouping}", implementation="hip_matvec")
+           code_bits=code_bits, strategy=f"verify_{grouping}", implementation="mfma_rows" if few else "hip_matvec")
     x_div = top_k or 1
-    if output_dims * input_dims >= ROWS_MATRIX and E <= PLAN_EXPERTS and rows_eligible(
-            xt, c, s, cb, code_bits=code_bits, input_dims=input_dims, group_size=group_size):
+    if few:
         y = rows_matvec(xt, c, s, cb, flat_rhs, lhs=flat_lhs, x_div=x_div, grouped=grouping == "expert",
                         input_dims=input_dims, output_dims=output_dims, group_size=group_size, code_bits=code_bits)
         return y.reshape(out_shape)

@@ -76,6 +76,7 @@ def routed(launches, monkeypatch):
     monkeypatch.setattr(ops, "_device_of", lambda *ts: torch.device("cpu"))
     monkeypatch.setattr(ops, "_stream", lambda device: 0)
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device: SimpleNamespace(synchronize=lambda: None))
 
     def run(fn, *args, **kw):
         launches.clear()
@@ -114,3 +115,25 @@ def test_more_experts_than_a_plan_holds(routed, T):
                      (ops.gather_vqmm_verify_rows, dict(grouping="expert"))):
         with pytest.raises(ValueError, match="1024"):
             routed(fn, x, c, s, None, rhs, **over, **kw)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("bits", [8, 16])
+@pytest.mark.parametrize("E, N, K, G, T, k", [(4, 4096, 512, 1, 2, 2), (4, 4096, 512, 1, 65, 2), (4, 512, 512, 1, 65, 2),
+                                              (2, 64, 512, 1, 200, 2), (8, 64, 128, 1, 65, 2), (4, 72, 640, 5, 70, 2),
+                                              (8, 4096, 512, 2, 10, 2), (4, 520, 8704, 17, 40, 4)])
+@pytest.mark.parametrize("strategy", ["auto", "direct", "sorted_tiled", "verify"])
+def test_trace_names_the_kernel_that_runs(routed, monkeypatch, dtype, bits, E, N, K, G, T, k, strategy):
+    c, s, kw = _switch(E, N, K, bits, G)
+    x, rhs = torch.empty((T, K), dtype=dtype), torch.zeros((T, k), dtype=torch.int32)
+    monkeypatch.setattr(ops, "route_plan", lambda rhs, E, tile: tuple(
+        torch.arange(rhs.numel(), dtype=torch.int32) for _ in range(8)))
+    with keep_amd.trace_gather_vqmm_calls() as tr:
+        if strategy == "verify":
+            calls = routed(ops.gather_vqmm_verify_rows, x, c, s, None, rhs, grouping="expert", **kw)
+        else:
+            calls = routed(ops.gather_vqmm, x, c, s, None, rhs, code_bits=bits, route_strategy=strategy, **kw)
+    want = {"keep_vq_rows": "mfma_rows", "keep_vq_grouped_gemm_e8": "mfma_grouped_gemm",
+            "keep_vq_grouped_gemm_q8": "mfma_grouped_gemm", "keep_vq_matvec": "hip_matvec",
+            "keep_vq_matvec_tiles": "hip_matvec"}
+    assert [t["implementation"] for t in tr] == [want[calls[-1]]]
