@@ -134,8 +134,8 @@ class QuantizedVQLinear:
             w = w @ torch.as_tensor(rotation_matrix).to(device=device, dtype=torch.float32)
         q = quantize_weight_rtn(w, group_size=group_size, code_bits=code_bits)
         out_dim, in_dim = w.shape
-        return cls(input_dims=in_dim, output_dims=out_dim, codes=q.codes, scales=q.scales, bias=bias,
-                   group_size=q.group_size, code_bits=q.code_bits, rht_signs=rht_signs,
+        return cls(input_dims=in_dim, output_dims=out_dim, codes=q.codes, scales=q.scales,
+                   codebook=ops._new_codebook(code_bits, device), bias=bias, group_size=q.group_size, code_bits=q.code_bits, rht_signs=rht_signs,
                    rotation_matrix=rotation_matrix)
 
 
@@ -222,7 +222,8 @@ class QuantizedVQSwitchLinear:
         q = quantize_weight_rtn(w.reshape(num_experts * out_dim, in_dim), group_size=group_size, code_bits=code_bits)
         return cls(input_dims=in_dim, output_dims=out_dim, num_experts=num_experts,
                    codes=q.codes.reshape(num_experts, out_dim, in_dim // CODEWORD_DIM),
-                   scales=q.scales.reshape(num_experts, out_dim, in_dim // q.group_size), bias=bias,
+                   scales=q.scales.reshape(num_experts, out_dim, in_dim // q.group_size),
+                   codebook=ops._new_codebook(code_bits, device), bias=bias,
                    group_size=q.group_size, code_bits=q.code_bits, use_gather_vqmm=use_gather_vqmm,
                    route_strategy=route_strategy, gather_codebook_duplication=gather_codebook_duplication,
                    rht_signs=None if rht_signs is None else torch.as_tensor(rht_signs).to(device),
@@ -624,7 +625,7 @@ def _tiles_entry(T: int, E: int, H: int, I: int, k: int, gh: int, gi: int, cb: t
     if moe_tiles_supported(T, E, H, I, k, gh, gi):
         return "keep_moe_tiles"
     if (H > 4096 and _lib.load().keep_moe_wide_supported(T, E, H, I, k, gh, gi)
-            and cb is ops._default_codebook(16, cb.device)
+            and ops.holds_default(cb)
             and not any(t.data_ptr() % 16 for t in codes) and not any(t.data_ptr() % 4 for t in scales)):
         return "keep_moe_wide"
     return None

@@ -23,6 +23,7 @@ tensors on a ROCm device instead of ``mx.array``. Differences, each deliberate:
 
 from __future__ import annotations
 
+import weakref
 from contextlib import contextmanager
 from contextvars import ContextVar
 from functools import lru_cache
@@ -85,6 +86,9 @@ def _trace(**rec) -> None:
 
 _HOST_TABLES: dict[int, np.ndarray] = {}
 _DEVICE_TABLES: dict[tuple[int, str], torch.Tensor] = {}
+_E8P_TABLES: dict[int, tuple[weakref.ref, int]] = {}  # by id: tensors made as the default E8P table, their version then
+_PREPARED: dict[tuple[int, str], tuple[torch.Tensor, int, torch.Tensor]] = {}
+_DEFAULT_PREPARED: dict[torch.device, torch.Tensor] = {}
 
 
 def e8p_packed_abs_grid() -> np.ndarray:
@@ -107,39 +111,68 @@ def e8_1bit_packed() -> np.ndarray:
     return _HOST_TABLES[8].copy()
 
 
+def _new_codebook(code_bits: int, device: torch.device) -> torch.Tensor:
+    """The default table in a tensor of its own."""
+
+    host = e8p_packed_abs_grid() if code_bits == 16 else e8_1bit_packed()
+    with torch.inference_mode(False):  # with a version counter
+        t = torch.from_numpy(host.view(np.int32)).to(device)
+    if code_bits == 16:
+        key = id(t)
+        _E8P_TABLES[key] = (weakref.ref(t, lambda _: _E8P_TABLES.pop(key, None)), t._version)
+    return t
+
+
 def _default_codebook(code_bits: int, device: torch.device) -> torch.Tensor:
     key = (code_bits, str(device))
     if key not in _DEVICE_TABLES:
-        host = e8p_packed_abs_grid() if code_bits == 16 else e8_1bit_packed()
-        _DEVICE_TABLES[key] = torch.from_numpy(host.view(np.int32)).to(device)
+        _DEVICE_TABLES[key] = _new_codebook(code_bits, device)
     return _DEVICE_TABLES[key]
 
 
-_PREPARED: dict[tuple[int, str], tuple[torch.Tensor, torch.Tensor]] = {}
+def holds_default(codebook: torch.Tensor) -> bool:
+    """Whether ``codebook`` is a default E8P table made here (the shared one, a ``from_weights`` layer's) and has
+    not been written to since. Such tables share one prepared table; a written one is served as any other."""
+
+    entry = _E8P_TABLES.get(id(codebook))
+    return entry is not None and entry[0]() is codebook and codebook._version == entry[1]
+
+
+def _version(t: torch.Tensor) -> int:
+    return -1 if t.is_inference() else t._version
 
 
 def prepared_table(codebook: torch.Tensor) -> torch.Tensor:
     """The prepared E8P table of ``codebook`` for the matrix-core kernels
     (``keep_e8p_prepare``: T and M of the int8 decode, a check word and the
-    64 KiB LDS image, ``keep_e8p_prepared_bytes()`` bytes), cached per codebook tensor
-    (one built under graph capture belongs to that graph and is not)."""
+    64 KiB LDS image, ``keep_e8p_prepared_bytes()`` bytes), kept per codebook tensor
+    until that is written to, and once per device for the default table. (One
+    built under graph capture belongs to that graph and is not kept.)"""
 
     hit = _kept_table(codebook)
     if hit is not None:
         return hit
-    nbytes = _lib.load().keep_e8p_prepared_bytes()
-    out = torch.empty(nbytes, dtype=torch.uint8, device=codebook.device)
-    _lib.call("keep_e8p_prepare", codebook.data_ptr(), out.data_ptr(), _stream(codebook.device))
-    if torch.cuda.is_current_stream_capturing():
+    device = codebook.device
+    capturing = torch.cuda.is_current_stream_capturing()
+    default = holds_default(codebook)
+    source = _new_codebook(16, device) if default and not capturing else codebook  # (no copies under capture)
+    out = torch.empty(_lib.load().keep_e8p_prepared_bytes(), dtype=torch.uint8, device=device)
+    _lib.call("keep_e8p_prepare", source.data_ptr(), out.data_ptr(), _stream(device))
+    if capturing:
         return out  # filled by this graph's replays only: not kept for other calls
-    torch.cuda.current_stream(codebook.device).synchronize()  # once: any stream may read it from here on
-    _PREPARED[(codebook.data_ptr(), str(codebook.device))] = (codebook, out)
+    torch.cuda.current_stream(device).synchronize()  # once: any stream may read it from here on
+    if default:
+        _DEFAULT_PREPARED[device] = out
+    else:
+        _PREPARED[(codebook.data_ptr(), str(device))] = (codebook, _version(codebook), out)
     return out
 
 
 def _kept_table(codebook: torch.Tensor) -> torch.Tensor | None:
+    if holds_default(codebook):
+        return _DEFAULT_PREPARED.get(codebook.device)
     hit = _PREPARED.get((codebook.data_ptr(), str(codebook.device)))
-    return hit[1] if hit is not None and hit[0] is codebook else None
+    return hit[2] if hit is not None and hit[0] is codebook and hit[1] == _version(codebook) else None
 
 
 def _may_prepare(codebook: torch.Tensor) -> bool:
@@ -446,7 +479,7 @@ def rows_eligible(x: torch.Tensor, codes: torch.Tensor, scales: torch.Tensor, co
         return False
     if code_bits == 8:
         return codebook.data_ptr() % 16 == 0
-    return codebook is _default_codebook(16, codebook.device) and _may_prepare(codebook)
+    return holds_default(codebook) and _may_prepare(codebook)
 
 
 def rows_matvec(x: torch.Tensor, codes: torch.Tensor, scales: torch.Tensor, codebook: torch.Tensor,
@@ -733,7 +766,7 @@ def vq_qmm(x, codes, scales, codebook=None, *, in_dim: int, out_dim: int, group_
     if (cells >= (ROWS_GEMM_CELLS[code_bits] if few else MATRIX_GEMM_CELLS)
             and xt.dtype in (torch.float16, torch.bfloat16)
             and gemm_eligible(code_bits=code_bits, x_dtype=xt.dtype, input_dims=in_dim, group_size=group_size)
-            and (code_bits == 8 or (cb is _default_codebook(16, device) and _may_prepare(cb)))
+            and (code_bits == 8 or (holds_default(cb) and _may_prepare(cb)))
             and _gemm_pointers_ok(c, s, cb, code_bits)):
         return matrix_gemm(xt, c, s, cb, input_dims=in_dim, output_dims=out_dim, group_size=group_size,
                            code_bits=code_bits)

@@ -27,6 +27,7 @@ def launches(monkeypatch):
     monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
     monkeypatch.setattr(ops, "_PREPARED", {})
+    monkeypatch.setattr(ops, "_DEFAULT_PREPARED", {})
     return calls
 
 
@@ -137,3 +138,30 @@ def test_trace_names_the_kernel_that_runs(routed, monkeypatch, dtype, bits, E, N
             "keep_vq_grouped_gemm_q8": "mfma_grouped_gemm", "keep_vq_matvec": "hip_matvec",
             "keep_vq_matvec_tiles": "hip_matvec"}
     assert [t["implementation"] for t in tr] == [want[calls[-1]]]
+
+
+def test_written_tables_are_not_the_default(routed, launches):
+    """A layer's own copy of the default E8P table takes the matrix cores and the one prepared table of all
+    copies; written to, it is a table like any other: the mat-vec, and prepared again."""
+    cpu = torch.device("cpu")
+    N, K, M = 4096, 512, 128
+    c, s, kw = _switch(1, N, K, bits=16)
+    x = torch.empty((M, K), dtype=torch.float16)
+
+    def qmm(cb):
+        return routed(ops.vq_qmm, x, c[0], s[0], cb, in_dim=K, out_dim=N, group_size=K, code_bits=16)
+
+    a, b = ops._new_codebook(16, cpu), ops._new_codebook(16, cpu)
+    assert qmm(a) == ["keep_e8p_prepare", "keep_vq_rows"] and qmm(b) == ["keep_vq_rows"] and qmm(None) == ["keep_vq_rows"]
+    shared = ops.prepared_table(b)
+    a[3] = a[4]
+    assert qmm(a) == ["keep_vq_matvec"] and qmm(b) == ["keep_vq_rows"]
+    first = ops.prepared_table(a)
+    assert first is not shared and ops.prepared_table(a) is first and ops.prepared_table(b) is shared
+    with torch.inference_mode():
+        a[5] = 0
+    assert ops.prepared_table(a) is not first
+    assert qmm(b.clone()) == ["keep_vq_matvec"]  # a table of the caller's
+    n = len(ops._E8P_TABLES)
+    del b
+    assert len(ops._E8P_TABLES) == n - 1

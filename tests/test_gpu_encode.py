@@ -200,3 +200,23 @@ def test_encode_near_ties_of_large_vectors(dev, code_bits):
     t = torch.from_numpy(v).to(dev)
     got = _u(torch.cat([enc(t[i:i + 1].clone()) for i in range(len(v))]))
     np.testing.assert_array_equal(got, oenc.nearest(v, code_bits))
+
+
+@pytest.mark.parametrize("code_bits", [8, 16])
+def test_from_weights_layers_have_their_own_table(dev, code_bits):
+    """Writing to one layer's codebook changes that layer alone, on one row and
+    on rows enough for the matrix cores."""
+    g = torch.Generator().manual_seed(code_bits)
+    w = torch.randn((1024, 512), generator=g)
+    x = torch.randn((130, 512), generator=g).half().to(dev)
+    a, b = (keep_amd.QuantizedVQLinear.from_weights(w, code_bits=code_bits) for _ in range(2))
+    before = b(x), b(x[0])
+    assert torch.equal(a(x), before[0])
+    a.codebook[:] = a.codebook.flip(0)
+    assert torch.equal(b(x), before[0]) and torch.equal(b(x[0]), before[1])
+    dense = keep_amd.decode_weight_matrix(a.codes, a.scales, code_bits=code_bits, codebook=a.codebook).double()
+    for y, rows in ((a(x), x), (a(x[0]), x[:1])):
+        want = rows.double() @ dense.T
+        assert float((y.double() - want).norm() / want.norm()) < 2e-3 and not torch.allclose(y, before[0][:1], atol=0.1)
+    s = keep_amd.QuantizedVQSwitchLinear.from_weights(w.reshape(2, 512, 512), code_bits=code_bits)
+    assert s.codebook.data_ptr() != b.codebook.data_ptr() and torch.equal(s.codebook, b.codebook)
