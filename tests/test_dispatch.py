@@ -165,3 +165,19 @@ def test_written_tables_are_not_the_default(routed, launches):
     n = len(ops._E8P_TABLES)
     del b
     assert len(ops._E8P_TABLES) == n - 1
+
+
+def test_router_outputs_are_tensors_of_their_own():
+    """Writing to one output leaves another that autograd has saved usable; each has its own storage and alignment."""
+    from keep_amd.nn import _router_output
+
+    r = _router_output(3, 5, torch.device("cpu"))
+    assert [t.dtype for t in r] == [torch.int32, torch.float32, torch.int32, torch.float32, torch.uint8]
+    assert all(t.shape == (3, 5) and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in r)
+    assert len({t.untyped_storage().data_ptr() for t in r}) == 5
+    r.weight.fill_(0.5)
+    y = torch.ones((3, 5), requires_grad=True)
+    z = (y * r.weight).sum()
+    r.idx.zero_()
+    z.backward()
+    assert torch.equal(y.grad, r.weight)
