@@ -1170,7 +1170,7 @@ static void mt_tail(const MTArgs& a, int x_dtype, int64_t T, int64_t H, int64_t 
   else combine(MTNone{});
 }
 
-static int mt_run(int64_t max_h, const void* x, int x_dtype, int64_t T, int64_t H, int64_t I, const int32_t* idx,
+static int mt_run(const char* what, int64_t max_h, const void* x, int x_dtype, int64_t T, int64_t H, int64_t I, const int32_t* idx,
                               const float* w, int64_t k, int64_t num_experts, const uint16_t* gate_codes,
                               const void* gate_scales, const uint16_t* up_codes, const void* up_scales,
                               const uint16_t* down_codes, const void* down_scales, int scale_dtype,
@@ -1203,7 +1203,7 @@ static int mt_run(int64_t max_h, const void* x, int x_dtype, int64_t T, int64_t 
                                  stream);
   if (rc != KEEP_OK) return rc;
   mt_tail(a, x_dtype, T, H, I, k, num_experts, idx, w, L, out, out_dtype, s);
-  return launch_status("few-token layer");
+  return launch_status(what);
 }
 
 // Router declaration (router.hip).
@@ -1212,7 +1212,7 @@ extern "C" int keep_router_dual_topk(const float* logits, int64_t T, int64_t E, 
                                      float tau, const int32_t* slot_map, int64_t num_slots, int32_t* idx, float* w,
                                      int32_t* want, float* want_score, uint8_t* admit, void* stream);
 
-static int mt_run_layer(int64_t max_h, const float* logits, const float* bias_served, const float* bias_demand,
+static int mt_run_layer(const char* what, int64_t max_h, const float* logits, const float* bias_served, const float* bias_demand,
                                     int score_func, int renormalize, float route_scale, float tau,
                                     const int32_t* slot_map, int64_t num_slots, int64_t num_experts, int64_t k,
                                     const void* x, int x_dtype, int64_t T, int64_t H, int64_t I,
@@ -1239,7 +1239,7 @@ static int mt_run_layer(int64_t max_h, const float* logits, const float* bias_se
                                          route_scale, tau, slot_map, num_slots, idx, w, want, want_score, admit,
                                          stream);
     if (rc != KEEP_OK) return rc;
-    return mt_run(max_h, x, x_dtype, T, H, I, idx, w, k, S, gate_codes, gate_scales, up_codes, up_scales,
+    return mt_run(what, max_h, x, x_dtype, T, H, I, idx, w, k, S, gate_codes, gate_scales, up_codes, up_scales,
                           down_codes, down_scales, scale_dtype, group_size_h, group_size_i, prepared, swiglu_limit,
                           h_work, workspace, workspace_bytes, out, out_dtype, stream);
   }
@@ -1262,7 +1262,7 @@ static int mt_run_layer(int64_t max_h, const float* logits, const float* bias_se
     rp.to = (int32_t*)(ws + L.to); rp.tc = (int32_t*)(ws + L.tc); rp.nt = (int32_t*)(ws + L.nt);
     rp.max_tiles = (int)L.max_tiles;
     mt_tail(a, x_dtype, T, H, I, k, S, idx, w, L, out, out_dtype, s, &rp, per);
-    return launch_status("few-token layer");
+    return launch_status(what);
   }
   MTPro p{};
   p.x = x; p.H = (int)H; p.xt = (uint4*)(ws + L.xt); p.xinv = (float*)(ws + L.xinv);
@@ -1287,7 +1287,7 @@ static int mt_run_layer(int64_t max_h, const float* logits, const float* bias_se
   else MT_PRO(16);
 #undef MT_PRO
   mt_tail(a, x_dtype, T, H, I, k, S, idx, w, L, out, out_dtype, s);
-  return launch_status("few-token layer");
+  return launch_status(what);
 }
 
 extern "C" int keep_moe_tiles(const void* x, int x_dtype, int64_t T, int64_t H, int64_t I, const int32_t* idx,
@@ -1297,7 +1297,7 @@ extern "C" int keep_moe_tiles(const void* x, int x_dtype, int64_t T, int64_t H, 
                               int64_t group_size_h, int64_t group_size_i, const void* prepared, float swiglu_limit,
                               void* h_work, void* workspace, int64_t workspace_bytes, void* out, int out_dtype,
                               void* stream) {
-  return mt_run(MT_MAX_H, x, x_dtype, T, H, I, idx, w, k, num_experts, gate_codes, gate_scales, up_codes, up_scales,
+  return mt_run("keep_moe_tiles", MT_MAX_H, x, x_dtype, T, H, I, idx, w, k, num_experts, gate_codes, gate_scales, up_codes, up_scales,
       down_codes, down_scales, scale_dtype, group_size_h, group_size_i, prepared, swiglu_limit,
       h_work, workspace, workspace_bytes, out, out_dtype, stream);
 }
@@ -1309,7 +1309,7 @@ extern "C" int keep_moe_wide(const void* x, int x_dtype, int64_t T, int64_t H, i
                               int64_t group_size_h, int64_t group_size_i, const void* prepared, float swiglu_limit,
                               void* h_work, void* workspace, int64_t workspace_bytes, void* out, int out_dtype,
                               void* stream) {
-  return mt_run(MT_WIDE_MAX_H, x, x_dtype, T, H, I, idx, w, k, num_experts, gate_codes, gate_scales, up_codes,
+  return mt_run("keep_moe_wide", MT_WIDE_MAX_H, x, x_dtype, T, H, I, idx, w, k, num_experts, gate_codes, gate_scales, up_codes,
       up_scales, down_codes, down_scales, scale_dtype, group_size_h, group_size_i, prepared,
       swiglu_limit, h_work, workspace, workspace_bytes, out, out_dtype, stream);
 }
@@ -1324,7 +1324,7 @@ extern "C" int keep_moe_tiles_layer(const float* logits, const float* bias_serve
                                     const void* prepared, float swiglu_limit, int32_t* idx, float* w, int32_t* want,
                                     float* want_score, uint8_t* admit, void* h_work, void* workspace,
                                     int64_t workspace_bytes, void* out, int out_dtype, void* stream) {
-  return mt_run_layer(MT_MAX_H, logits, bias_served, bias_demand, score_func, renormalize, route_scale, tau, slot_map,
+  return mt_run_layer("keep_moe_tiles_layer", MT_MAX_H, logits, bias_served, bias_demand, score_func, renormalize, route_scale, tau, slot_map,
       num_slots, num_experts, k, x, x_dtype, T, H, I, gate_codes, gate_scales, up_codes, up_scales,
       down_codes, down_scales, scale_dtype, group_size_h, group_size_i, prepared, swiglu_limit, idx,
       w, want, want_score, admit, h_work, workspace, workspace_bytes, out, out_dtype, stream);
@@ -1340,7 +1340,7 @@ extern "C" int keep_moe_wide_layer(const float* logits, const float* bias_served
                                     const void* prepared, float swiglu_limit, int32_t* idx, float* w, int32_t* want,
                                     float* want_score, uint8_t* admit, void* h_work, void* workspace,
                                     int64_t workspace_bytes, void* out, int out_dtype, void* stream) {
-  return mt_run_layer(MT_WIDE_MAX_H, logits, bias_served, bias_demand, score_func, renormalize, route_scale, tau,
+  return mt_run_layer("keep_moe_wide_layer", MT_WIDE_MAX_H, logits, bias_served, bias_demand, score_func, renormalize, route_scale, tau,
       slot_map, num_slots, num_experts, k, x, x_dtype, T, H, I, gate_codes, gate_scales, up_codes,
       up_scales, down_codes, down_scales, scale_dtype, group_size_h, group_size_i, prepared,
       swiglu_limit, idx, w, want, want_score, admit, h_work, workspace, workspace_bytes, out,

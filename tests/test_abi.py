@@ -137,3 +137,19 @@ def test_nested_swiglu_argument_validation_before_launch():
             0.0, None, 0, 16, None]
     assert lib.keep_vq_grouped_swiglu_nested_q8(*args) == _lib.KEEP_EINVAL
     assert b"null pointer" in lib.keep_last_error()
+
+
+@pytest.mark.parametrize("name, H", [("keep_moe_tiles_layer", 512), ("keep_moe_wide_layer", 4608)])
+def test_a_failed_launch_names_its_entry_point(name, H):
+    """Without a GPU every launch fails, and the error says which call it was."""
+    import torch
+
+    if torch.cuda.is_available():
+        pytest.skip("the launches would run, on addresses that are none")
+    lib = _lib.load()
+    T, E, I, k = 2, 4, 256, 2
+    p = 1 << 20  # never read: nothing runs
+    rc = getattr(lib, name)(p, None, None, 0, 1, 1.0, 1.0, None, 0, E, k, p, 1, T, H, I, p, p, p, p, p, p, 1, H, I, p,
+                            0.0, p, p, p, p, p, p, p, lib.keep_moe_tiles_workspace_bytes(T, k, E, H), p, 0, None)
+    assert rc != _lib.KEEP_OK and rc != _lib.KEEP_EINVAL
+    assert lib.keep_last_error().decode().startswith(name)
