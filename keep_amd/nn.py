@@ -619,15 +619,24 @@ def _router_output(T: int, k: int, device: torch.device) -> RouterOutput:
                         torch.empty((T, k), dtype=torch.uint8, device=device))
 
 
+# Values of h (T k I) up to which the packed-table kernels serve hidden sizes beyond 4096: two launches, 14-25 us until
+# the VALU decode of every route's codes passes the five launches of keep_moe_wide (24-30 us). Per layer, packed / wide
+# us: 7168 x 2048, one route 15.6 / 28.1, two 22.6 / 28.4, three 31.5 / 28.5; 5120 x 512 top-4, 2 tokens 22.0 / 25.8, 3
+# tokens 29.8 / 26.0; 6144 x 1024 top-2, 2 tokens 18.7 / 26.9, 4 tokens 31.5 / 31.1; 4608 x 768 top-4, one token 25.7 /
+# 25.3. At I = 256 a down row fills half a wave: 4352 x 256, two routes 22.5 / 23.6, four 27.2 / 23.9.
+PACKED_WIDE_H = {True: 4096, False: 512}  # by I >= 512
+
+
 def _tiles_entry(T: int, E: int, H: int, I: int, k: int, gh: int, gi: int, cb: torch.Tensor, codes, scales):
     """The few-token entry point that serves a shape, or None. Hidden sizes beyond 4096 take it on the default
     table and on aligned pools only: the matrix-core decode needs odd half-units and loads 16 bytes of codes and
-    aligned words of scales, the packed-table kernels take any table and narrower loads."""
+    aligned words of scales, the packed-table kernels take any table and narrower loads; and beyond
+    ``PACKED_WIDE_H``."""
 
     if moe_tiles_supported(T, E, H, I, k, gh, gi):
         return "keep_moe_tiles"
-    if (H > 4096 and _lib.load().keep_moe_wide_supported(T, E, H, I, k, gh, gi)
-            and ops.holds_default(cb)
+    if (H > 4096 and T * k * I > PACKED_WIDE_H[I >= 512]
+            and _lib.load().keep_moe_wide_supported(T, E, H, I, k, gh, gi) and ops.holds_default(cb)
             and not any(t.data_ptr() % 16 for t in codes) and not any(t.data_ptr() % 4 for t in scales)):
         return "keep_moe_wide"
     return None

@@ -181,3 +181,11 @@ def test_router_outputs_are_tensors_of_their_own():
     r.idx.zero_()
     z.backward()
     assert torch.equal(y.grad, r.weight)
+
+
+@pytest.mark.parametrize("T, H, I, E, k, wide", [(2, 7168, 2048, 1, 1, False), (3, 7168, 2048, 1, 1, True),
+                                                 (2, 6144, 1024, 4, 2, False), (4, 6144, 1024, 4, 2, True),
+                                                 (1, 8192, 256, 4, 2, False), (2, 8192, 256, 4, 2, True)])
+def test_few_routes_of_wide_layers_stay_on_the_packed_kernels(routed, T, H, I, E, k, wide):
+    x, _, pool, idx, w = _moe(T, H=H, I=I, E=E, k=k)
+    assert routed(keep_amd.moe_decode, x, idx, w, *pool)[-1] == ("keep_moe_wide" if wide else "keep_moe_decode")
