@@ -243,8 +243,8 @@ def test_grouped_gemm_wide_items(dev, form, G):
 @pytest.mark.parametrize("M,N,K,G", [(1024, 64, 128, 1), (129, 513, 640, 5), (2112, 1040, 256, 2), (65, 2056, 384, 1)])
 def test_one_matrix_gemm_vs_oracle(dev, code_bits, xdt, M, N, K, G):
     """vq_qmm on the MFMA GEMM: partial row tiles (65 = one row past a tile),
-    partial column blocks, one K block, both item widths, per-row and grouped
-    scales. fp32 row dots against the fp64 oracle: within the rounding of the
+    partial column blocks, one K block, per-row and grouped scales (items of
+    256 columns; 512 in the test below). fp32 row dots against the fp64 oracle: within the rounding of the
     16-bit output plus the path's bound."""
     rng = np.random.default_rng(M + N)
     codes = rng.integers(0, 1 << code_bits, (N, K // 8)).astype(np.uint8 if code_bits == 8 else np.uint16)
@@ -264,7 +264,7 @@ def test_one_matrix_gemm_vs_oracle(dev, code_bits, xdt, M, N, K, G):
 @pytest.mark.parametrize("E,T,k,N,K,G", [(7, 43, 3, 72, 128, 1), (3, 90, 2, 520, 512, 4), (200, 700, 4, 1032, 256, 2)])
 def test_routed_8bit_gemm_vs_oracle(dev, xdt, E, T, k, N, K, G):
     """8-bit E8 routes on the sorted-route GEMM (tiles of one and two m-tiles,
-    partial column blocks, items of 256 and 512 columns), an out-of-range route
+    partial column blocks, items of 256 columns; 512 in the test below), an out-of-range route
     (NaN), and gather_vqmm_sorted_routes on unsorted routes: each row its own."""
     rng = np.random.default_rng(E + T)
     codes = rng.integers(0, 256, (E, N, K // 8), dtype=np.uint8)
@@ -288,6 +288,69 @@ def test_routed_8bit_gemm_vs_oracle(dev, xdt, E, T, k, N, K, G):
     for out in (y, z):
         assert torch.isnan(out[torch.from_numpy(~good)]).all()
         _check(out[torch.from_numpy(good)], want[good], tol=TOL + ulp)
+
+
+def _dense(codes, scales, code_bits, K):
+    """Decoded weights in float64 on the GPU, from the oracle's grid."""
+    grid = e8p.decode_e8_1bit(np.arange(256, dtype=np.uint8)) if code_bits == 8 else e8p.e8p_full_grid()
+    index = codes.int() if code_bits == 8 else codes.int() & 0xFFFF
+    w = torch.from_numpy(grid.astype(np.float64)).to(codes.device)[index].flatten(-2)
+    return w * scales.double().repeat_interleave(K // scales.shape[-1], -1)
+
+
+def _codes(code_bits, shape, K, dev, g):
+    c = torch.randint(0, 256, (*shape, K // 8 * (code_bits // 8)), dtype=torch.uint8, device=dev, generator=g)
+    return c if code_bits == 8 else c.view(torch.int16)
+
+
+@pytest.mark.parametrize("code_bits", [8, 16])
+@pytest.mark.parametrize("xdt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("G", [1, 2])
+def test_one_matrix_gemm_wide_items(dev, code_bits, xdt, G):
+    """Rows and columns enough that 512-column items take fewer rounds of the
+    chip: 2001 x 4088, a partial tile of rows and a partial last item."""
+    M, N, K = 2001, 4088, 256
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    rounds = [-(-(-(-M // 64) * -(-N // w)) // cus) for w in (256, 512)]
+    assert 8 * rounds[1] <= 5 * rounds[0], "items of 512 columns"
+    g = torch.Generator(device=dev).manual_seed(G + code_bits)
+    codes = _codes(code_bits, (N,), K, dev, g)
+    scales = torch.exp(0.3 * torch.randn((N, G), device=dev, generator=g)).half()
+    x = torch.randn((M, K), device=dev, generator=g).to(xdt)
+    y = kops.matrix_gemm(x, codes, scales, kops._default_codebook(code_bits, dev), input_dims=K, output_dims=N,
+                         group_size=K // G, code_bits=code_bits)
+    ulp = 2.0 ** -9 if xdt == torch.float16 else 2.0 ** -8
+    _check(y, (x.double() @ _dense(codes, scales, code_bits, K).T).cpu().numpy(), tol=TOL + ulp)
+
+
+@pytest.mark.parametrize("xdt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("G", [1, 2])
+def test_routed_8bit_gemm_wide_items(dev, xdt, G):
+    """Four items of 512 columns per CU: 160 experts of 4096 outputs, tiles of one and of two m-tiles, an
+    out-of-range route (NaN)."""
+    E, N, K, T, k = 160, 4096, 256, 2560, 2
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    assert (-(-T * k // 64) + E) * -(-N // 512) >= 4 * cus, "items of 512 columns"
+    g = torch.Generator(device=dev).manual_seed(G)
+    codes = _codes(8, (E, N), K, dev, g)
+    scales = torch.exp(0.3 * torch.randn((E, N, G), device=dev, generator=g)).half()
+    x = torch.randn((T, K), device=dev, generator=g).to(xdt)
+    rhs = torch.randint(0, E, (T, k), device=dev, generator=g, dtype=torch.int32)
+    rhs[7, 1] = E
+    count = torch.bincount(rhs.reshape(-1).long())
+    assert (count > 32).any() and ((count > 0) & (count <= 32)).any()
+    with keep_amd.trace_gather_vqmm_calls() as tr:
+        y = kops.gather_vqmm(x, codes, scales, None, rhs, input_dims=K, output_dims=N, group_size=K // G, code_bits=8)
+    assert tr[0]["implementation"] == "mfma_grouped_gemm"
+    assert torch.isnan(y[7, 1]).all()
+    flat, y = rhs.reshape(-1), y.reshape(T * k, N)
+    want = torch.zeros((T * k, N), dtype=torch.float64, device=dev)
+    for e in range(E):
+        r = torch.nonzero(flat == e)[:, 0]
+        want[r] = x[r // k].double() @ _dense(codes[e], scales[e], 8, K).T
+    good = flat < E
+    ulp = 2.0 ** -9 if xdt == torch.float16 else 2.0 ** -8
+    _check(y[good], want[good].cpu().numpy(), tol=TOL + ulp)
 
 
 @pytest.mark.parametrize("tail", [1, 700])

@@ -102,7 +102,9 @@ def test_rows_through_the_operators(dev):
         "sorted": lambda: kops.gather_vqmm(x, c, s, None, rhs, code_bits=8, route_strategy="sorted_tiled", **kw),
         "qmm": lambda: kops.vq_qmm(x.repeat(8, 1), c[0], s[0], in_dim=K, out_dim=N, group_size=K // G),
     }
-    eager = {n: f() for n, f in calls.items()}
+    with keep_amd.trace_gather_vqmm_calls() as tr:
+        eager = {n: f() for n, f in calls.items()}
+    assert [t["implementation"] for t in tr] == ["mfma_rows"] * 4
     torch.cuda.synchronize()
     for n in ("flat", "direct", "sorted"):
         assert torch.equal(eager["expert"], eager[n]), n
@@ -147,3 +149,68 @@ def test_rows_non_finite_rows(dev, bits, xdt):
     np.testing.assert_array_equal(got[np.isinf(want)], want[np.isinf(want)])
     good = np.isfinite(want).all(1)
     _check(got[good], want[good], xdt)
+
+
+def _units(bits, N, K, tiles, n_tiles):
+    """(units per group of waves, whether a group's run crosses tiles), as the launch shares them out: a group of
+    K / 512 (E8P: / 256) of a block's 16 waves, units of 32 columns, up to 256 blocks."""
+    upt, groups = -(-N // 32), 16 // (K // (512 if bits == 8 else 256))
+    per = -(-tiles * upt // (min(n_tiles * upt, 256) * groups))
+    return per, any((u // upt) != ((min(u + per, tiles * upt) - 1) // upt) for u in range(0, tiles * upt, per))
+
+
+# K slices that leave one, two and sixteen groups per block; ragged last units; odd counts of scales and rows
+LONG = [(8, torch.float16, 90, 520, 8192, 16), (8, torch.bfloat16, 110, 1031, 3584, 7),
+        (16, torch.float16, 90, 520, 4096, 1), (8, torch.bfloat16, 90, 1080, 4096, 8)]
+
+
+@pytest.mark.parametrize("bits,xdt,E,N,K,G", LONG)
+@pytest.mark.parametrize("form", ["planned", "plan", "flat", "matrix"])
+def test_rows_long_runs_vs_oracle(dev, bits, xdt, E, N, K, G, form):
+    """At least five units per group of waves: code buffers refilled, both
+    partial-sum buffers used again, and runs that cross from one expert's tile
+    (or one matrix's rows) to the next, invalid routes among them."""
+    g = torch.Generator(device=dev).manual_seed(K + N)
+    one = form == "matrix"
+    E = 1 if one else E
+    codes = torch.randint(0, 256, (E, N, K // 8 * (bits // 8)), dtype=torch.uint8, device=dev, generator=g)
+    grid = e8p.decode_e8_1bit(np.arange(256, dtype=np.uint8)) if bits == 8 else e8p.e8p_full_grid()
+    grid = torch.from_numpy(grid.astype(np.float32)).to(dev)
+    index = codes if bits == 8 else (codes.view(torch.int16).int() & 0xFFFF)
+    codes = codes if bits == 8 else codes.view(torch.int16)
+    scales = torch.exp(0.3 * torch.randn((E, N, G), device=dev, generator=g)).half()
+    T, k = {"planned": (32, 4), "plan": (70, 4), "flat": (32, 4), "matrix": (2055, 1)}[form]
+    x = torch.randn((T, K), device=dev, generator=g).to(xdt)
+    kw = dict(input_dims=K, output_dims=N, group_size=K // G, code_bits=bits)
+    cb = kops._default_codebook(bits, dev)
+
+    def dense(e):
+        return grid[index[e].int()].reshape(N, K).double() * scales[e].double().repeat_interleave(K // G, 1)
+
+    if one:
+        tiles = n_tiles = -(-T // 16)
+        y = kops.rows_matvec(x, codes, scales, cb, None, **kw)
+        want = x.double() @ dense(0).T
+        good = torch.ones(T, dtype=torch.bool, device=dev)
+    else:
+        rhs = torch.randint(0, E, (T * k,), device=dev, generator=g, dtype=torch.int32)
+        rhs[[5, 61, 90]] = torch.tensor([E, -2, E + 7], dtype=torch.int32, device=dev)
+        flat = rhs.cpu().numpy()
+        good = (rhs >= 0) & (rhs < E)
+        count = np.bincount(np.where((flat < 0) | (flat >= E), E, flat), minlength=E + 1)
+        tiles = n_tiles = T * k
+        if form != "flat":
+            tiles = int((-(-count // 16)).sum())
+        if form == "plan":
+            tiles = n_tiles = min(-(-T * k // 16) + E, T * k)
+        y = kops.rows_matvec(x, codes, scales, cb, rhs, x_div=k, grouped=form != "flat", **kw)
+        want = torch.zeros((T * k, N), dtype=torch.float64, device=dev)
+        for e in np.unique(flat[good.cpu().numpy()]):
+            r = torch.nonzero(rhs == int(e))[:, 0]
+            want[r] = x[r // k].double() @ dense(int(e)).T
+    per, crosses = _units(bits, N, K, tiles, n_tiles)
+    assert per >= 5 and crosses, (per, crosses)
+    y = y.float().cpu().numpy()
+    good = good.cpu().numpy()
+    assert np.isnan(y[~good]).all()
+    _check(y[good], want.cpu().numpy()[good], xdt)
