@@ -6,8 +6,9 @@
 // Arithmetic. As the reference's sorted path (vq_switch.py:712-715,759-771:
 // the gathered rows cast to float16, then an fp16 matmul), the A rows are fp16:
 // fp16 rows as they are; bf16 and fp32 rows times a power of two r per row
-// (k_gq_rowscale: max |x| r in [2^14, 2^15), so no row overflows fp16 and a
-// bf16 row converts exactly), rounded to nearest even. B is the decoded weight
+// (k_gq_rowscale: max |x| r in [2^14, 2^15), so no row overflows fp16 and bf16
+// values convert exactly down to 2^-32 of their row's max; smaller ones to
+// 2^-39 of it), rounded to nearest even. B is the decoded weight
 // x 4, an odd integer |q| <= 15 (E8P) or an even one in [-16, 14] (the nested
 // tier's 8-bit E8), exact in fp16; products are exact in fp32 and the MFMA sums
 // them in fp32. D / (4 r) x the column's scale is the output.
@@ -155,9 +156,11 @@ struct GQArgs {
 // copies of 16 bytes, 64 KiB), so a codeword is one byte permute and one
 // 16-byte lookup with no conversion: 1 VALU instead of the 10 of the byte image
 // this replaced. bf16 rows stay bf16 (the weights are exact in it), without a
-// row factor. LDS-bound: per k-step a wave reads 1 KiB per m-tile and 1 KiB of
-// lookups per n-tile. 2048 bf16 rows against 4096 x 4096, groups of 512: 77 us
-// (896 TFLOP/s; a mat-vec per row took 3,900 us). The result is stored, or added
+// row factor. Per k-step a wave reads 1 KiB per m-tile and 1 KiB of lookups per
+// n-tile from LDS. 2048 bf16 rows against 4096 x 4096, groups of 512: 79 us (868
+// TFLOP/s; a mat-vec per row took 3,900 us), the matrix cores busy 44%, LDS 29%,
+// the VALU 24%; the two waves per SIMD wait 42% of the time (LDS operands, the
+// barrier of each K block). The result is stored, or added
 // to the fp32 output (a.add: the nested tier's residual onto the base
 // projection's). HOT: E8P base codes and, on the tiles of an
 // expert with a residual row (hot[e] in [0, hot_rows)), that row's 8-bit E8
@@ -659,8 +662,10 @@ void gq_launch(GQArgs& a, bool gateup, hipStream_t s, bool e8 = false, bool hot 
   shape(256);
   const int64_t narrow_rounds = (a.total + cus - 1) / cus;
   shape(512);
-  // routed tiles: items of 512 columns once there are four per CU (uneven tiles need several to balance); one
-  // matrix: its items are alike, so whichever form takes fewer rounds of the chip (a wide item takes ~1.6 times a
+  // routed tiles: items of 512 columns once there are four per CU (uneven tiles need several to balance), counted over
+  // the plan's arrays, R / 64 + E tiles with the empty ones, as the host does not know how many hold routes: 2048
+  // tokens of 384 experts top-6, 576 tiles, 1,586 us a layer against 1,761 in items of 256. The line is low for plans
+  // that are mostly empty: 512 tokens top-8 with the tier, 145 of 352 tiles, 704 against 598. One matrix: its items are alike, so whichever form takes fewer rounds of the chip (a wide item takes ~1.6 times a
   // narrow one: its A reads feed twice the MFMAs)
   const bool wide = a.te ? a.total >= 4 * (int64_t)cus : 8 * ((a.total + cus - 1) / cus) <= 5 * narrow_rounds;
   if (!wide) shape(256);

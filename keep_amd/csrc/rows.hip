@@ -25,11 +25,14 @@
 // routes every block groups them itself (plan_small_to): no plan launch, no
 // gather of the routes' rows.
 //
-// Bound: the LDS lookups, 16 bytes per codeword (2.2 us per unit of 32 x 4096
-// in each block); the codes alone would take 9.5 us below. 8 fp16 rows, top-6 of
-// 256 8-bit experts 4096 -> 2048, groups of 512 (48 MB): 24 us, against 128 on
-// the mat-vec in tiles of 4 routes it replaces and 55 on single routes; one
-// matrix 4096 x 4096, 16 rows, 14 against 37.
+// Bound: waiting. 8 fp16 rows, top-6 of 256 8-bit experts 4096 -> 2048, groups of
+// 512 (48 MB): 24 us, against 128 on the mat-vec in tiles of 4 routes it replaces
+// and 55 on single routes; the codes alone would take 9.5. Its waves wait 54% of
+// the time (the first codes and x of each block's six units, the barrier of
+// each) with the VALU busy 37%, LDS 29%, the matrix cores 23%. 333 bf16 rows of
+// the same, 143 us: 48%, 46% and 37%, waves waiting 50%; a third of its units
+// are those of a plan's empty tiles. One matrix 4096 x 4096, 16 rows, 14 us
+// against 37.
 #include <algorithm>
 #include <type_traits>
 
