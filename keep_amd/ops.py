@@ -44,15 +44,24 @@ GEMM_ROUTE_TILE = 64
 # The mat-vec takes ~4 us plus 1 us per 8.1M (8-bit) / 5.3M (E8P) products M N K, the rows kernel 9-14 us until its
 # tiles fill the chip: they meet near 64M / 32M. The GEMM takes 25-40 us until its tiles do and meets the rows kernel
 # near M N = 2M in 8 bits (4096 x 4096: 33 against 41 us at 512 rows, 52 against 44 at 1024), 1.3M for E8P (31 / 40 at
-# 256, 54 / 43 at 512). Where the rows kernel does not serve (bf16 rows of E8P), mat-vec and GEMM meet near 64K.
+# 256, 54 / 43 at 512). Where the rows kernel does not serve, mat-vec and GEMM meet near M N = 64K; bf16 rows of E8P
+# near 80K, with their factors' launch (2048 -> 1024, 64 rows: 28 / 32 us).
 ROWS_PRODUCTS = {8: 1 << 26, 16: 1 << 25}
 MATRIX_GEMM_CELLS = 1 << 16
+BF16_E8P_GEMM_CELLS = 5 << 14
 ROWS_GEMM_CELLS = {8: 1 << 21, 16: 5 << 18}
 # Routed calls by routes per expert: in tiles of 16 against the GEMM's 64. 8-bit, 32 experts 4096 -> 2048: 57 against
 # 65 us at 32 routes per expert, 115 / 138 at 128; E8P, 256 experts: 270 / 311 at 8, 367 / 322 at 16.
 ROWS_PER_EXPERT = {8: 128, 16: 12}
+# From which work on 8-bit routes leave the mat-vec, in outputs (R N; times K / 1600 for longer rows: the mat-vec takes
+# 4 us plus 1 us per 5000 outputs or 8.1M products): the rows kernel without a plan (up to 128 routes), with one, the
+# GEMM. Mat-vec / the other, us in a graph and by calls, 32 experts: 128 routes 512 -> 256 10.5, 18 / 10.9, 16; 256
+# routes 1024 -> 64 7.1, 17 / 17.8, 32, 1024 -> 256 17.7, 18 / 17.3, 33, 512 -> 1024 52, 52 / 17, 33; the GEMM, 1024
+# routes of 4 experts, 1024 -> 64 17.5, 18 / 34, 57, 1024 -> 256 57, 56 / 34, 56.
+ROUTED_WORK = {"rows": 3 << 14, "planned rows": 1 << 17, "gemm": 1 << 18}
 # Outputs x inputs from which few routes take the rows kernel (a matter of the matrix alone: grouped, flat and
 # single-row calls then agree bit for bit): 4096 -> 2048, 8 rows x top-6 of 256, 24 against 57 us, one row 10.9 / 11.6.
+# (Fewer routes pay for that agreement: 4 routes of 2048 -> 1024 8.3 against 4.8 us in a graph.)
 ROWS_MATRIX = 1 << 21
 PLANNED_ROUTES = 128  # routes keep_vq_rows groups without a route plan
 # Experts a route plan holds. Routed 8-bit and direct calls beyond stay on the mat-vec, which has no limit.
@@ -763,10 +772,11 @@ def vq_qmm(x, codes, scales, codebook=None, *, in_dim: int, out_dim: int, group_
     cb = _codebook_tensor(codebook, code_bits, device)
     M = xt.shape[0]
     cells = M * out_dim
-    few = cells * in_dim >= ROWS_PRODUCTS[code_bits] and rows_eligible(
+    few = cells * in_dim > ROWS_PRODUCTS[code_bits] and rows_eligible(
         xt, c, s, cb, code_bits=code_bits, input_dims=in_dim, group_size=group_size)
     # E8P on the matrix cores takes the default table only: they decode it from odd half-units, the mat-vec any
-    if (cells >= (ROWS_GEMM_CELLS[code_bits] if few else MATRIX_GEMM_CELLS)
+    bf16_e8p = code_bits == 16 and xt.dtype == torch.bfloat16
+    if (cells >= (ROWS_GEMM_CELLS[code_bits] if few else BF16_E8P_GEMM_CELLS if bf16_e8p else MATRIX_GEMM_CELLS)
             and xt.dtype in (torch.float16, torch.bfloat16)
             and gemm_eligible(code_bits=code_bits, x_dtype=xt.dtype, input_dims=in_dim, group_size=group_size)
             and (code_bits == 8 or (holds_default(cb) and _may_prepare(cb)))
@@ -806,6 +816,13 @@ def _host_check_indices(name: str, ix: torch.Tensor, upper: int) -> None:
             raise ValueError(f"{name} must be in [0, {upper}), found range [{lo}, {hi}]")
 
 
+def _enough_work(routes: int, output_dims: int, input_dims: int, few: bool) -> bool:
+    """Whether 8-bit routes are work enough for the rows kernel (``few`` routes per expert) or the GEMM."""
+
+    form = "gemm" if not few else "rows" if routes <= PLANNED_ROUTES else "planned rows"
+    return routes * output_dims * max(input_dims, 1600) >= 1600 * ROUTED_WORK[form]
+
+
 def gather_vqmm(x, codes, scales, codebook, rhs_indices, *, lhs_indices=None, input_dims: int, output_dims: int,
                 group_size: int = 512, code_bits: Literal[8, 16] = 8, codebook_duplication: Literal[1, 4, 8] = 1,
                 implementation: str = "hip", sorted_indices: bool = False, route_strategy: str = "auto",
@@ -817,8 +834,8 @@ def gather_vqmm(x, codes, scales, codebook, rhs_indices, *, lhs_indices=None, in
 
     ``route_strategy="auto"``: calls that the MFMA grouped GEMM serves
     (``gemm_eligible``) with at least ``GEMM_ROUTE_THRESHOLD`` routes (or
-    ``sorted_indices``) take ``sorted_tiled``, a device route plan and that
-    GEMM; everything else takes ``direct``, the wave-per-rows decode mat-vec
+    ``sorted_indices``; 8-bit codes: and ``ROUTED_WORK``) take ``sorted_tiled``,
+    a device route plan and that GEMM; everything else takes ``direct``, the wave-per-rows decode mat-vec
     (``per_route_decoded`` is the same). In either, the matrix-core rows kernel
     takes the calls it serves (``rows_eligible``) that have few routes per
     expert (sorted) or a large matrix (direct); the trace names the kernel.
@@ -868,13 +885,16 @@ def gather_vqmm(x, codes, scales, codebook, rhs_indices, *, lhs_indices=None, in
 
     eligible = gemm_eligible(code_bits=code_bits, x_dtype=xt.dtype, input_dims=input_dims, group_size=group_size) \
         and (code_bits == 16 or (E <= PLAN_EXPERTS and _gemm_pointers_ok(c, s, cb, 8)))
+    rows = E <= PLAN_EXPERTS and rows_eligible(xt, c, s, cb, code_bits=code_bits, input_dims=input_dims,
+                                               group_size=group_size)
+    few_sorted = rows and R <= ROWS_PER_EXPERT[code_bits] * E
     strategy = route_strategy
     if strategy == "auto":
-        strategy = "sorted_tiled" if eligible and (sorted_indices or R >= GEMM_ROUTE_THRESHOLD) else "direct"
+        sort = eligible and (sorted_indices or R >= GEMM_ROUTE_THRESHOLD) and (
+            code_bits == 16 or _enough_work(R, output_dims, input_dims, few_sorted))
+        strategy = "sorted_tiled" if sort else "direct"
     sort = strategy == "sorted_tiled"
-    few = ((R <= ROWS_PER_EXPERT[code_bits] * E if sort else output_dims * input_dims >= ROWS_MATRIX)
-           and E <= PLAN_EXPERTS
-           and rows_eligible(xt, c, s, cb, code_bits=code_bits, input_dims=input_dims, group_size=group_size))
+    few = few_sorted if sort else rows and output_dims * input_dims >= ROWS_MATRIX
     _trace(token_rows=int(xt.shape[0]), route_count=int(R), has_lhs_indices=lhs_indices is not None,
            input_dims=int(input_dims), output_dims=int(output_dims), group_size=int(group_size),
            code_bits=int(code_bits), strategy=strategy,
@@ -913,8 +933,8 @@ def gather_vqmm_sorted_routes(x, codes, scales, codebook, sorted_rhs, sorted_lhs
     """Already-sorted routed matmul -> ``[R, N]`` in sorted order
     (reference ``vq_switch.py:620-913``). E8P runs the MFMA grouped GEMM
     (``tile_descriptors`` or a device route plan of 64-route tiles), and so do
-    8-bit codes with fp16 or bf16 rows from ``GEMM_ROUTE_THRESHOLD`` routes on,
-    on a plan of their own (or, few routes per expert, the rows kernel); other
+    8-bit codes with fp16 or bf16 rows from ``GEMM_ROUTE_THRESHOLD`` routes and
+    ``ROUTED_WORK`` on, on a plan of their own (or, few routes per expert, the rows kernel); other
     calls run the mat-vec over the sorted routes."""
 
     if projection not in ("auto", "gate_up", "down"):
@@ -951,8 +971,10 @@ def gather_vqmm_sorted_routes(x, codes, scales, codebook, sorted_rhs, sorted_lhs
     use_lhs = None if skip_gather else lhs
     eligible = gemm_eligible(code_bits=code_bits, x_dtype=xt.dtype, input_dims=input_dims, group_size=group_size)
     planned = code_bits == 8 and R >= GEMM_ROUTE_THRESHOLD and E <= PLAN_EXPERTS
-    if (planned and R <= ROWS_PER_EXPERT[8] * E
-            and rows_eligible(xt, c, s, cb, code_bits=8, input_dims=input_dims, group_size=group_size)):
+    few = planned and R <= ROWS_PER_EXPERT[8] * E and rows_eligible(
+        xt, c, s, cb, code_bits=8, input_dims=input_dims, group_size=group_size)
+    planned = planned and _enough_work(R, output_dims, input_dims, few)
+    if planned and few:
         pos = torch.arange(R, dtype=torch.int32, device=device) if use_lhs is None else use_lhs
         return rows_matvec(xt, c, s, cb, rhs, lhs=pos, grouped=True, input_dims=input_dims, output_dims=output_dims,
                            group_size=group_size, code_bits=8)

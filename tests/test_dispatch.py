@@ -189,3 +189,24 @@ def test_router_outputs_are_tensors_of_their_own():
 def test_few_routes_of_wide_layers_stay_on_the_packed_kernels(routed, T, H, I, E, k, wide):
     x, _, pool, idx, w = _moe(T, H=H, I=I, E=E, k=k)
     assert routed(keep_amd.moe_decode, x, idx, w, *pool)[-1] == ("keep_moe_wide" if wide else "keep_moe_decode")
+
+
+@pytest.mark.parametrize("T, E, N, K, G, last", [
+    (64, 32, 64, 1024, 2, "keep_vq_matvec"), (64, 32, 256, 1024, 2, "keep_vq_matvec"),
+    (64, 32, 512, 1024, 2, "keep_vq_rows"), (64, 32, 256, 4096, 8, "keep_vq_rows"),
+    (32, 32, 64, 2048, 4, "keep_vq_matvec"), (32, 32, 512, 1024, 2, "keep_vq_rows"),
+    (256, 4, 64, 4096, 8, "keep_vq_matvec"), (256, 4, 256, 1024, 2, "keep_vq_grouped_gemm_e8"),
+    (32, 32, 64, 128, 1, "keep_vq_matvec"), (256, 32, 1024, 128, 1, "keep_vq_grouped_gemm_e8")])
+def test_8bit_routes_leave_the_matvec_with_enough_work(routed, monkeypatch, T, E, N, K, G, last):
+    """4 routes a token, through gather_vqmm (also told that they are sorted) and gather_vqmm_sorted_routes."""
+    monkeypatch.setattr(ops, "route_plan", lambda rhs, E, tile: tuple(
+        torch.arange(rhs.numel(), dtype=torch.int32) for _ in range(8)))
+    c, s, kw = _switch(E, N, K, G=G)
+    x, rhs = torch.empty((T, K), dtype=torch.float16), torch.zeros((T, 4), dtype=torch.int32)
+    lhs = torch.arange(T * 4, dtype=torch.int32) // 4
+    assert N * K < ops.ROWS_MATRIX
+    for sort in (False, True):
+        assert routed(ops.gather_vqmm, x, c, s, None, rhs, code_bits=8, sorted_indices=sort, **kw)[-1] == last
+    assert routed(ops.gather_vqmm_sorted_routes, x, c, s, None, rhs.reshape(-1), lhs, code_bits=8, **kw)[-1] == last
+    assert routed(ops.gather_vqmm, x, c, s, None, rhs, code_bits=8, route_strategy="sorted_tiled",
+                  **kw)[-1] != "keep_vq_matvec"
