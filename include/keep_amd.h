@@ -495,8 +495,9 @@ int keep_vq_rows(const void* x, int x_dtype, int64_t x_rows, const void* codes, 
  * for x fp16 or bf16 [rows, K], codes [N, K/8] (code_bits 16: E8P, `tables` =
  * keep_e8p_prepare's buffer; 8: E8, `tables` = the packed 8-bit E8 table),
  * scales [N, K/group_size]. Arithmetic as keep_vq_grouped_gemm_q8 (E8P; bf16
- * rows need its workspace for `rows` rows) or keep_vq_grouped_gemm_e8 (no
- * workspace). Replaces vq_qmm (src/ramp/kernels/vq_qmm.py:93-152) on many rows. */
+ * rows need its workspace for `rows` rows; their factor is that of the finite
+ * values, so an infinity or NaN stays one value of its row) or
+ * keep_vq_grouped_gemm_e8 (no workspace). Replaces vq_qmm (src/ramp/kernels/vq_qmm.py:93-152) on many rows. */
 int keep_vq_gemm(const void* x, int x_dtype, int64_t rows, const void* codes, int code_bits, const void* scales,
                  int scale_dtype, const void* tables, int64_t N, int64_t K, int64_t group_size, void* workspace,
                  int64_t workspace_bytes, void* out, int out_dtype, void* stream);
