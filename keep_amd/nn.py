@@ -610,12 +610,12 @@ def _f32(t, device: torch.device, *shape: int):
 
 
 def _router_output(T: int, k: int, device: torch.device) -> RouterOutput:
-    """Uninitialised router outputs, each a tensor of its own (views of one allocation, 1 us cheaper, would share a
-    version counter: a write to one would spoil another that autograd has saved)."""
+    """Uninitialised router outputs, the four 32-bit ones in one allocation (4.4 us on the host against 6.5).
+    ``unsafe_split`` gives each a version counter of its own, where views would share one: a write to one output
+    would spoil another that autograd has saved."""
 
-    idx = torch.empty((T, k), dtype=torch.int32, device=device)
-    weight = torch.empty((T, k), dtype=torch.float32, device=device)
-    return RouterOutput(idx, weight, torch.empty_like(idx), torch.empty_like(weight),
+    idx, weight, want, score = torch.empty((4 * T, k), dtype=torch.int32, device=device).unsafe_split(T)
+    return RouterOutput(idx, weight.view(torch.float32), want, score.view(torch.float32),
                         torch.empty((T, k), dtype=torch.uint8, device=device))
 
 

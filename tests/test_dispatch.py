@@ -167,14 +167,15 @@ def test_written_tables_are_not_the_default(routed, launches):
     assert len(ops._E8P_TABLES) == n - 1
 
 
-def test_router_outputs_are_tensors_of_their_own():
-    """Writing to one output leaves another that autograd has saved usable; each has its own storage and alignment."""
+def test_router_outputs_have_version_counters_of_their_own():
+    """Writing to one output leaves another that autograd has saved usable."""
     from keep_amd.nn import _router_output
 
     r = _router_output(3, 5, torch.device("cpu"))
     assert [t.dtype for t in r] == [torch.int32, torch.float32, torch.int32, torch.float32, torch.uint8]
-    assert all(t.shape == (3, 5) and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in r)
-    assert len({t.untyped_storage().data_ptr() for t in r}) == 5
+    assert all(t.shape == (3, 5) and t.is_contiguous() and not t._is_view() for t in (r.idx, r.want, r.admit))
+    spans = sorted((t.data_ptr(), t.data_ptr() + t.nbytes) for t in r)
+    assert all(a[1] <= b[0] for a, b in zip(spans, spans[1:]))
     r.weight.fill_(0.5)
     y = torch.ones((3, 5), requires_grad=True)
     z = (y * r.weight).sum()
